@@ -25,6 +25,8 @@
 // through LDS as rows of four values.  Each lane's plain partial sums are
 // folded into compensated (TwoSum) sums every ~64 pairs.  No allocation:
 // the caller passes every buffer and its stream.
+#include "g6_sym.h"
+
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -388,6 +390,114 @@ int launch_adjoint(int n, const T *x, const T *v, const T *m, const T *ga, const
 }
 
 // ---------------------------------------------------------------------------
+// Every unordered pair once (g6_sym.h): the geometry of a pair (separation,
+// r^-1, r.v and what follows from them) serves both of its particles.
+// ---------------------------------------------------------------------------
+
+// The forward: 37.5 VALU instructions per unordered pair (FP32) against 2 x 32.6.
+template <class T>
+struct ForceOp {
+    static constexpr int NV = 7;  // x3 m v3
+    static constexpr int NC = 6;  // acc3 jerk3
+    const T *x, *v, *m;
+    T eps2;
+
+    __device__ __forceinline__ void load(int j, T (&f)[NV]) const
+    {
+        f[3] = m[j];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            f[k] = x[3 * j + k];
+            f[4 + k] = v[3 * j + k];
+        }
+    }
+    // Row r (its values, as a column's) and column c: the row's sums s and,
+    // for BOTH, the column's sums (added to u, or set when FIRST).
+    template <bool BOTH, bool FIRST>
+    __device__ __forceinline__ void pair(const T (&r)[NV], const T *c, bool self, T (&s)[NC],
+                                         T (&u)[NC]) const
+    {
+        const T dx = c[0] - r[0], dy = c[1] - r[1], dz = c[2] - r[2];
+        const T ss = fma_t(dz, dz, fma_t(dy, dy, fma_t(dx, dx, eps2)));
+        T y = rsq<T>(ss);
+        if (!BOTH) y = self ? T(0) : y;
+        const T y2 = y * y, y3 = y * y2;
+        const T wx = c[4] - r[4], wy = c[5] - r[5], wz = c[6] - r[6];
+        const T rv = fma_t(dz, wz, fma_t(dy, wy, dx * wx));
+        const T a = (T(-3) * rv) * y2;
+        const T ex = fma_t(a, dx, wx), ey = fma_t(a, dy, wy), ez = fma_t(a, dz, wz);
+        const T p = c[3] * y3;
+        s[0] = fma_t(p, dx, s[0]); s[1] = fma_t(p, dy, s[1]); s[2] = fma_t(p, dz, s[2]);
+        s[3] = fma_t(p, ex, s[3]); s[4] = fma_t(p, ey, s[4]); s[5] = fma_t(p, ez, s[5]);
+        if (BOTH) {
+            const T g = -r[3] * y3;
+            if (FIRST) {
+                u[0] = g * dx; u[1] = g * dy; u[2] = g * dz;
+                u[3] = g * ex; u[4] = g * ey; u[5] = g * ez;
+            } else {
+                u[0] = fma_t(g, dx, u[0]); u[1] = fma_t(g, dy, u[1]); u[2] = fma_t(g, dz, u[2]);
+                u[3] = fma_t(g, ex, u[3]); u[4] = fma_t(g, ey, u[4]); u[5] = fma_t(g, ez, u[5]);
+            }
+        }
+    }
+};
+
+// Rows per lane, each serving the column values a lane reads from LDS and one
+// rotation of the column's sums (n = 16384, one MI355X): FP32 4 (127 us; 2:
+// 130, 3: 142), FP64 2 (239 us; 1: 255; 4 would leave one wave per SIMD).
+template <class T, class Op>
+struct SymShape;
+template <class T>
+struct SymShape<T, ForceOp<T>> {
+    static constexpr int ipl = sizeof(T) == 4 ? 4 : 2;
+};
+
+// Workgroups a pass aims at: of 400, 700, 1000, 2000 and 4000 the last was
+// the fastest or within 3 % of it at n = 8192..32768 in both precisions
+// (fewer leave the last round of workgroups uneven).
+constexpr int kSymWgs = 4000;
+// Particles from which the pair-once form is the faster one.  A wave's
+// shortest work is one tile (FP32 ~20 us, FP64 ~30), which small n cannot
+// fill the chip with.  Pair by ordered pair against pair-once, us: FP32 forward
+// 21.2 / 27.5 at n = 4000, 31.9 / 29.1 at 5003, 57.8 / 51.0 at 8192, 191 / 127
+// at 16384, 708 / 435 at 32768; FP64 36.3 / 37.0, 51.3 / 38.3, 124 / 86, 381 /
+// 240, 1433 / 891.
+template <class T, class Op>
+constexpr int kSymMin = sizeof(T) == 4 ? 4800 : 4200;
+// The largest workspace asked for (n = 107,000 FP64, 150,000 FP32): beyond,
+// the pair by ordered pair form, which needs none.
+constexpr long long kSymMaxBytes = 2ll << 30;
+
+template <class T, class Op>
+g6s::Plan sym_plan(int n)
+{
+    return g6s::Plan(n, 64 * SymShape<T, Op>::ipl, kSymWgs);
+}
+
+// Bytes of the partial records of a pass over n particles; 0 where the pair
+// by ordered pair kernels are the ones to take.
+template <class T, class Op>
+long long sym_bytes(int n)
+{
+    if (n < kSymMin<T, Op>) return 0;
+    const g6s::Plan p = sym_plan<T, Op>(n);
+    const long long bytes = 8 * (p.row_values(Op::NC) + p.col_values(Op::NC));
+    return bytes <= kSymMaxBytes ? bytes : 0;
+}
+
+template <class T, class Op>
+int launch_sym(int n, const Op &op, T *o0, T *o1, T *o2, void *ws, hipStream_t st)
+{
+    const g6s::Plan p = sym_plan<T, Op>(n);
+    double *rowpart = static_cast<double *>(ws), *colpart = rowpart + p.row_values(Op::NC);
+    hipLaunchKernelGGL((g6s::k_sym<T, Op, SymShape<T, Op>::ipl>), dim3(p.items()),
+                       dim3(g6s::kWG), 0, st, p, op, rowpart, colpart);
+    hipLaunchKernelGGL((g6s::k_sym_sum<T, Op::NC>), dim3((n + 255) / 256, Op::NC), dim3(256), 0,
+                       st, p, rowpart, colpart, o0, o1, o2);
+    return hipGetLastError() == hipSuccess ? 0 : -5;
+}
+
+// ---------------------------------------------------------------------------
 // The fixed-step Hermite scheme around the pair sum (src/amuse_hermite/
 // interface.cc: predictor :266-281, time-symmetric corrector :536-556) as
 // elementwise kernels over the 3n components, and the transposes of both
@@ -563,3 +673,34 @@ G6A_API int g6a_adjoint_f64(int n, const double *x, const double *v, const doubl
     return g6a::launch_adjoint<double>(n, x, v, m, ga, gj, eps2, gx, gv, gm,
                                        static_cast<hipStream_t>(stream));
 }
+
+// Workspace forms: the same sums with every unordered pair evaluated once
+// where that is faster, through `ws` (g6a_workspace_* bytes, owned by the
+// caller; nothing is allocated here).  A null or short workspace takes the
+// forms above.
+namespace g6a {
+template <class T>
+int forces_ws(int n, const T *x, const T *v, const T *m, T eps2, T *acc, T *jerk, void *ws,
+              long long ws_bytes, hipStream_t st)
+{
+    const long long need = sym_bytes<T, ForceOp<T>>(n);
+    if (need == 0 || !ws || ws_bytes < need)
+        return launch_forces<T>(n, x, v, m, eps2, acc, jerk, st);
+    return launch_sym<T>(n, ForceOp<T>{x, v, m, eps2}, acc, jerk, static_cast<T *>(nullptr), ws,
+                         st);
+}
+}  // namespace g6a
+
+#define G6A_WS_API(S, T)                                                                        \
+    G6A_API long long g6a_forces_workspace_##S(int n)                                            \
+    {                                                                                          \
+        return g6a::sym_bytes<T, g6a::ForceOp<T>>(n);                                           \
+    }                                                                                          \
+    G6A_API int g6a_forces_ws_##S(int n, const T *x, const T *v, const T *m, T eps2, T *acc,     \
+                                  T *jerk, void *ws, long long ws_bytes, void *stream)          \
+    {                                                                                          \
+        return g6a::forces_ws<T>(n, x, v, m, eps2, acc, jerk, ws, ws_bytes,                     \
+                                 static_cast<hipStream_t>(stream));                             \
+    }
+G6A_WS_API(f32, float)
+G6A_WS_API(f64, double)

@@ -1,7 +1,7 @@
 """Differentiable direct N-body integration on the GPU.
 
 * :class:`PairForce` — torch.autograd.Function over the hand-written HIP
-  kernels g6a_forces_* (acc, jerk of the softened pair sum, the arithmetic of
+  kernels g6a_forces_ws_* (acc, jerk of the softened pair sum, the arithmetic of
   lib/g6lib/g6lib.c:165-183) and g6a_adjoint_* (their vector-Jacobian
   product: dL/dx, dL/dv, dL/dm from dL/dacc, dL/djerk).  float32 and float64
   tensors on the GPU; no CPU fallback.
@@ -27,6 +27,7 @@
 from __future__ import annotations
 
 import ctypes as C
+import functools
 
 import torch
 from torch.utils.checkpoint import checkpoint
@@ -46,6 +47,12 @@ def _kernels():
             f = getattr(L, "g6a_forces_" + name)
             f.restype = C.c_int
             f.argtypes = [C.c_int, vp, vp, vp, real, vp, vp, vp]
+            f = getattr(L, "g6a_forces_workspace_" + name)
+            f.restype = C.c_longlong
+            f.argtypes = [C.c_int]
+            f = getattr(L, "g6a_forces_ws_" + name)
+            f.restype = C.c_int
+            f.argtypes = [C.c_int, vp, vp, vp, real, vp, vp, vp, C.c_longlong, vp]
             g = getattr(L, "g6a_adjoint_" + name)
             g.restype = C.c_int
             g.argtypes = [C.c_int, vp, vp, vp, vp, vp, real, vp, vp, vp, vp]
@@ -76,22 +83,36 @@ def _suffix(dtype):
     raise TypeError(f"unsupported dtype {dtype}")
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_size(query, dtype, n):
+    return getattr(_kernels(), query + _suffix(dtype))(n)
+
+
+def _workspace(query, dtype, n, device):
+    """Device memory for one launch, from torch's allocator on the current
+    stream (which orders its reuse), and its size; (None, 0) where none is
+    used."""
+    size = _workspace_size(query, dtype, n)
+    ws = torch.empty(size, dtype=torch.uint8, device=device) if size > 0 else None
+    return ws, size
+
+
+def _forces(x, v, m, eps2, acc, jerk, stream):
+    n = x.shape[0]
+    ws, size = _workspace("g6a_forces_workspace_", x.dtype, n, x.device)
+    _call("g6a_forces_ws_", x.dtype, n, x.data_ptr(), v.data_ptr(), m.data_ptr(), float(eps2),
+          acc.data_ptr(), jerk.data_ptr(), _ptr(ws), size, stream)
+
+
 class PairForce(torch.autograd.Function):
     """acc, jerk = PairForce.apply(x, v, m, eps2)  with x, v (n, 3), m (n,)."""
 
     @staticmethod
     def forward(ctx, x, v, m, eps2: float):
         x, v, m = _check(x, "x"), _check(v, "v"), _check(m, "m")
-        n = x.shape[0]
         acc = torch.empty_like(x)
         jerk = torch.empty_like(x)
-        L = _kernels()
-        stream = torch.cuda.current_stream(x.device).cuda_stream
-        rc = getattr(L, "g6a_forces_" + _suffix(x.dtype))(
-            n, x.data_ptr(), v.data_ptr(), m.data_ptr(), float(eps2), acc.data_ptr(),
-            jerk.data_ptr(), stream)
-        if rc != 0:
-            raise RuntimeError(f"g6a_forces failed ({rc})")
+        _forces(x, v, m, eps2, acc, jerk, torch.cuda.current_stream(x.device).cuda_stream)
         ctx.save_for_backward(x, v, m)
         ctx.eps2 = float(eps2)
         return acc, jerk
@@ -145,8 +166,7 @@ class HermiteStep(torch.autograd.Function):
         _call("g6a_step_predict_", x.dtype, n, x.data_ptr(), v.data_ptr(), a.data_ptr(),
               j.data_ptr(), float(dt), xp.data_ptr(), vp.data_ptr(), stream)
         a1, j1 = torch.empty_like(x), torch.empty_like(x)
-        _call("g6a_forces_", x.dtype, n, xp.data_ptr(), vp.data_ptr(), m.data_ptr(), float(eps2),
-              a1.data_ptr(), j1.data_ptr(), stream)
+        _forces(xp, vp, m, eps2, a1, j1, stream)
         x1, v1 = torch.empty_like(x), torch.empty_like(v)
         _call("g6a_step_correct_", x.dtype, n, x.data_ptr(), v.data_ptr(), a.data_ptr(),
               j.data_ptr(), a1.data_ptr(), j1.data_ptr(), float(dt), x1.data_ptr(),

@@ -180,6 +180,19 @@ int g6a_adjoint_f64(int n, const double *x, const double *v, const double *m,
                     const double *ga, const double *gj, double eps2,
                     double *gx, double *gv, double *gm, void *stream);
 
+/* The same sums through a workspace: from a few thousand particles on, every
+ * unordered pair is evaluated once for both of its particles, with partial
+ * sums in `ws` (device memory of the caller, at least the bytes that the
+ * _workspace_ query gives for n; 0: the calls above are the faster ones and
+ * no workspace is used).  A NULL or smaller workspace takes the calls above.
+ * Nothing is allocated; calls that may overlap need workspaces of their own. */
+long long g6a_forces_workspace_f32(int n);
+long long g6a_forces_workspace_f64(int n);
+int g6a_forces_ws_f32(int n, const float *x, const float *v, const float *m, float eps2,
+                      float *acc, float *jerk, void *ws, long long ws_bytes, void *stream);
+int g6a_forces_ws_f64(int n, const double *x, const double *v, const double *m, double eps2,
+                      double *acc, double *jerk, void *ws, long long ws_bytes, void *stream);
+
 /* Fixed-step Hermite scheme around the pair sum (src/amuse_hermite/
  * interface.cc:266-281 predictor, :536-556 corrector) on the same [n][3]
  * device arrays, and the transposes of both linear maps for the backward

@@ -204,3 +204,51 @@ def test_fp32_gradient_vs_fp64():
     for g32, g64 in zip(grads[torch.float32], grads[torch.float64]):
         rel = torch.linalg.vector_norm(g32 - g64) / torch.linalg.vector_norm(g64)
         assert rel < 1e-3, rel.item()
+
+
+# Edges of the pair-once form's blocks (256 rows FP32, 128 FP64): whole blocks
+# with an even and an odd number of them, a last block of one particle and of
+# all but one, a last tile of one column.
+PAIR_ONCE_N = [4864, 4865, 5119, 5120, 5121, 5185, 5311]
+
+
+@pytest.mark.parametrize("n", PAIR_ONCE_N)
+def test_forward_pair_once_edges(n):
+    """Every unordered pair once, with partial sums in a workspace: the rows
+    at the edges of blocks and tiles against the oracle, Newton's third law
+    over all particles, repeat runs bit for bit, and a null workspace gives
+    the pair by ordered pair kernel's bits."""
+    from amuse_amd import diff
+    from conftest import par_oracle
+    x, v, m = tensors(n, 7)
+    ids = np.arange(n, dtype=np.int32)
+    edge = np.concatenate([np.arange(0, n, 64), np.arange(63, n, 64), [n - 2, n - 1]])
+    sel = np.unique(edge)
+    # bounds as in test_forward_kernels_vs_oracle: the same per-pair arithmetic,
+    # plain sums of 64 terms, compensated beyond
+    for dtype, tols in ((torch.float64, (1e-15, 4e-15)), (torch.float32, (2e-6, 1e-5))):
+        name = "f64" if dtype == torch.float64 else "f32"
+        L = diff._kernels()
+        assert getattr(L, "g6a_forces_workspace_" + name)(n) > 0
+        xx, vv, mm = x.to(dtype), v.to(dtype), m.to(dtype)
+        a, j = diff.pair_force(xx, vv, mm, 1e-4)
+        a2, j2 = diff.pair_force(xx, vv, mm, 1e-4)
+        assert torch.equal(a, a2) and torch.equal(j, j2)
+        xn, vn, mn = (t.double().cpu().numpy() for t in (xx, vv, mm))
+        ea, ej, _, sa, sj, _ = par_oracle(oracle.force_ld, ids[sel], xn[sel], vn[sel], 1e-4, ids,
+                                          mn, xn, vn)
+        for val, ex, s, tol, what in ((a, ea, sa, tols[0], "acc"), (j, ej, sj, tols[1], "jerk")):
+            q = val.double().cpu().numpy()
+            d = np.abs(q[sel] - ex).max(1)
+            print(n, dtype, what, "max |d|/sum|term|", (d / s).max(), flush=True)
+            assert (d <= tol * s).all(), (n, dtype, what, (d / s).max())
+            r = np.linalg.norm((mn[:, None] * q).sum(0)) / (mn * np.linalg.norm(q, axis=1)).sum()
+            assert r <= (1e-14 if dtype == torch.float64 else 1e-6), (n, dtype, what, r)
+        out = [torch.empty_like(xx) for _ in range(4)]
+        st = torch.cuda.current_stream().cuda_stream
+        p = [t.data_ptr() for t in (xx, vv, mm)]
+        assert getattr(L, "g6a_forces_" + name)(n, *p, 1e-4, out[0].data_ptr(),
+                                                out[1].data_ptr(), st) == 0
+        assert getattr(L, "g6a_forces_ws_" + name)(n, *p, 1e-4, out[2].data_ptr(),
+                                                   out[3].data_ptr(), None, 0, st) == 0
+        assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
