@@ -442,36 +442,119 @@ struct ForceOp {
     }
 };
 
-// Rows per lane, each serving the column values a lane reads from LDS and one
-// rotation of the column's sums (n = 16384, one MI355X): FP32 4 (127 us; 2:
-// 130, 3: 142), FP64 2 (239 us; 1: 255; 4 would leave one wave per SIMD).
-template <class T, class Op>
-struct SymShape;
+// The adjoint: 98 VALU instructions per unordered pair (FP32) against 2 x 79.
+// Seen from p the combined adjoint of the pair is minus that seen from k and
+// Gr, Gv are even in (r, v), so the pair's contributions to gx and gv of its
+// two particles are equal and opposite.
 template <class T>
-struct SymShape<T, ForceOp<T>> {
-    static constexpr int ipl = sizeof(T) == 4 ? 4 : 2;
+struct AdjointOp {
+    static constexpr int NV = 13;  // x3 m v3 gA3 gJ3
+    static constexpr int NC = 7;   // gx3 gv3 gm
+    const T *x, *v, *m, *ga, *gj;
+    T eps2;
+
+    __device__ __forceinline__ void load(int j, T (&f)[NV]) const
+    {
+        f[3] = m[j];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            f[k] = x[3 * j + k];
+            f[4 + k] = v[3 * j + k];
+            f[7 + k] = ga[3 * j + k];
+            f[10 + k] = gj[3 * j + k];
+        }
+    }
+    template <bool BOTH, bool FIRST>
+    __device__ __forceinline__ void pair(const T (&r)[NV], const T *c, bool self, T (&s)[NC],
+                                         T (&u)[NC]) const
+    {
+        const T d0 = c[0] - r[0], d1 = c[1] - r[1], d2 = c[2] - r[2];
+        const T w0 = c[4] - r[4], w1 = c[5] - r[5], w2 = c[6] - r[6];
+        const T ss = fma_t(d2, d2, fma_t(d1, d1, fma_t(d0, d0, eps2)));
+        T y = rsq<T>(ss);
+        if (!BOTH) y = self ? T(0) : y;
+        const T y2 = y * y, y3 = y * y2;
+        const T y5m3 = (T(-3) * y3) * y2;
+        const T rv = fma_t(d2, w2, fma_t(d1, w1, d0 * w0));
+        const T cj = y5m3 * rv;
+        // r.gA + v.gJ and r.gJ with the column's adjoint inputs (p) and the row's (k)
+        const T sp = fma_t(w2, c[12], fma_t(w1, c[11], fma_t(w0, c[10],
+                     fma_t(d2, c[9], fma_t(d1, c[8], d0 * c[7])))));
+        const T gp = fma_t(d2, c[12], fma_t(d1, c[11], d0 * c[10]));
+        const T sk = fma_t(w2, r[12], fma_t(w1, r[11], fma_t(w0, r[10],
+                     fma_t(d2, r[9], fma_t(d1, r[8], d0 * r[7])))));
+        const T gk = fma_t(d2, r[12], fma_t(d1, r[11], d0 * r[10]));
+        const T mk = r[3], mp = c[3];
+        // the combined adjoint m_k g_p - m_p g_k and its dots
+        const T A0 = fma_t(mk, c[7], -mp * r[7]), A1 = fma_t(mk, c[8], -mp * r[8]),
+                A2 = fma_t(mk, c[9], -mp * r[9]);
+        const T J0 = fma_t(mk, c[10], -mp * r[10]), J1 = fma_t(mk, c[11], -mp * r[11]),
+                J2 = fma_t(mk, c[12], -mp * r[12]);
+        const T sc = fma_t(mk, sp, -mp * sk), gc = fma_t(mk, gp, -mp * gk);
+        // -3 y^5 (r.gA + v.gJ) + 15 y^7 (r.v)(r.gJ)
+        const T cr = fma_t(y5m3, sc, (T(-5) * y2 * cj) * gc);
+        const T cv = y5m3 * gc;
+        const T q0 = fma_t(cr, d0, fma_t(cv, w0, fma_t(cj, J0, y3 * A0)));
+        const T q1 = fma_t(cr, d1, fma_t(cv, w1, fma_t(cj, J1, y3 * A1)));
+        const T q2 = fma_t(cr, d2, fma_t(cv, w2, fma_t(cj, J2, y3 * A2)));
+        const T h0 = fma_t(cv, d0, y3 * J0), h1 = fma_t(cv, d1, y3 * J1),
+                h2 = fma_t(cv, d2, y3 * J2);
+        s[0] += q0; s[1] += q1; s[2] += q2;
+        s[3] += h0; s[4] += h1; s[5] += h2;
+        // dm_k = -(sp y3 + cj r.gJ_p); from p the signs of r and v flip
+        s[6] = fma_t(-cj, gp, fma_t(-sp, y3, s[6]));
+        if (BOTH) {
+            if (FIRST) {
+                u[0] = -q0; u[1] = -q1; u[2] = -q2;
+                u[3] = -h0; u[4] = -h1; u[5] = -h2;
+                u[6] = fma_t(cj, gk, sk * y3);
+            } else {
+                u[0] -= q0; u[1] -= q1; u[2] -= q2;
+                u[3] -= h0; u[4] -= h1; u[5] -= h2;
+                u[6] = fma_t(cj, gk, fma_t(sk, y3, u[6]));
+            }
+        }
+    }
 };
+
+// Rows per lane (each reading of a column from LDS and each rotation of its
+// sums serves so many pairs): more make less overhead, but a wave's shortest
+// work, a tile of 64 columns, longer and the tiles fewer.  us with 1 / 2 / 4 a
+// lane: FP32 forward n = 4500 25.1 / 27.8 / 27, 6500 39.8 / 37.2 / 42, 16384 - /
+// 130 / 127, 32768 - / 472 / 435; FP64 forward 4000 28.4 / 36.0, 6500 56.1 /
+// 53.3, 32768 1060 / 900; FP32 adjoint 4000 34.0 / 46.0, 5003 49.4 / 47.0,
+// 16384 298 / 277; FP64 adjoint 4500 57.7 / 68.2, 5003 73.7 / 69.0, 32768 2156
+// / 2050.  4 a lane in FP64 or the adjoint would leave one wave per SIMD.
+constexpr int kSymNarrow = 4800, kSymWide = 10000;
+template <class T, class Op>
+inline int sym_ipl(int n)
+{
+    if (n < kSymNarrow) return 1;
+    return sizeof(T) == 4 && Op::NC == 6 && n >= kSymWide ? 4 : 2;
+}
 
 // Workgroups a pass aims at: of 400, 700, 1000, 2000 and 4000 the last was
 // the fastest or within 3 % of it at n = 8192..32768 in both precisions
 // (fewer leave the last round of workgroups uneven).
 constexpr int kSymWgs = 4000;
-// Particles from which the pair-once form is the faster one.  A wave's
-// shortest work is one tile (FP32 ~20 us, FP64 ~30), which small n cannot
-// fill the chip with.  Pair by ordered pair against pair-once, us: FP32 forward
-// 21.2 / 27.5 at n = 4000, 31.9 / 29.1 at 5003, 57.8 / 51.0 at 8192, 191 / 127
-// at 16384, 708 / 435 at 32768; FP64 36.3 / 37.0, 51.3 / 38.3, 124 / 86, 381 /
-// 240, 1433 / 891.
+// Particles from which the pair-once form is the faster one.  Pair by
+// ordered pair against pair-once, us: FP32 forward 21.3 / 22.0 at n = 4000,
+// 28.5 / 25.1 at 4500, 58.0 / 49.7 at 8192, 191 / 127 at 16384, 708 / 435 at
+// 32768; FP64 forward 24.0 / 27.3 at 3000, 34.6 / 28.1 at 3500, 51.1 / 37.7 at
+// 5003, 381 / 240 at 16384; FP32 adjoint 35.3 / 33.7 at 3500, 59.9 / 47.0 at
+// 5003, 454 / 277 at 16384, 1744 / 1037 at 32768; FP64 adjoint 26.1 / 27.6 at
+// 2000, 38.7 / 29.0 at 2500, 106 / 69.0 at 5003, 821 / 543 at 16384.
 template <class T, class Op>
-constexpr int kSymMin = sizeof(T) == 4 ? 4800 : 4200;
-// The largest workspace asked for (n = 107,000 FP64, 150,000 FP32): beyond,
-// the pair by ordered pair form, which needs none.
+constexpr int kSymMin = Op::NC == 6 ? (sizeof(T) == 4 ? 4300 : 3300)
+                                    : (sizeof(T) == 4 ? 3600 : 2300);
+// The largest workspace asked for (from about n = 100,000): beyond, the pair
+// by ordered pair form, which needs none.
 constexpr long long kSymMaxBytes = 2ll << 30;
 
 template <class T, class Op>
 g6s::Plan sym_plan(int n)
 {
-    return g6s::Plan(n, 64 * SymShape<T, Op>::ipl, kSymWgs);
+    return g6s::Plan(n, 64 * sym_ipl<T, Op>(n), kSymWgs);
 }
 
 // Bytes of the partial records of a pass over n particles; 0 where the pair
@@ -490,8 +573,15 @@ int launch_sym(int n, const Op &op, T *o0, T *o1, T *o2, void *ws, hipStream_t s
 {
     const g6s::Plan p = sym_plan<T, Op>(n);
     double *rowpart = static_cast<double *>(ws), *colpart = rowpart + p.row_values(Op::NC);
-    hipLaunchKernelGGL((g6s::k_sym<T, Op, SymShape<T, Op>::ipl>), dim3(p.items()),
-                       dim3(g6s::kWG), 0, st, p, op, rowpart, colpart);
+    const dim3 grid(p.items()), wg(g6s::kWG);
+    switch (p.rows / 64) {
+    case 1: hipLaunchKernelGGL((g6s::k_sym<T, Op, 1>), grid, wg, 0, st, p, op, rowpart, colpart); break;
+    case 2: hipLaunchKernelGGL((g6s::k_sym<T, Op, 2>), grid, wg, 0, st, p, op, rowpart, colpart); break;
+    default:
+        // (sym_ipl gives 4 for the FP32 forward alone)
+        if constexpr (sizeof(T) == 4 && Op::NC == 6)
+            hipLaunchKernelGGL((g6s::k_sym<T, Op, 4>), grid, wg, 0, st, p, op, rowpart, colpart);
+    }
     hipLaunchKernelGGL((g6s::k_sym_sum<T, Op::NC>), dim3((n + 255) / 256, Op::NC), dim3(256), 0,
                        st, p, rowpart, colpart, o0, o1, o2);
     return hipGetLastError() == hipSuccess ? 0 : -5;
@@ -689,6 +779,16 @@ int forces_ws(int n, const T *x, const T *v, const T *m, T eps2, T *acc, T *jerk
     return launch_sym<T>(n, ForceOp<T>{x, v, m, eps2}, acc, jerk, static_cast<T *>(nullptr), ws,
                          st);
 }
+
+template <class T>
+int adjoint_ws(int n, const T *x, const T *v, const T *m, const T *ga, const T *gj, T eps2, T *gx,
+               T *gv, T *gm, void *ws, long long ws_bytes, hipStream_t st)
+{
+    const long long need = sym_bytes<T, AdjointOp<T>>(n);
+    if (need == 0 || !ws || ws_bytes < need)
+        return launch_adjoint<T>(n, x, v, m, ga, gj, eps2, gx, gv, gm, st);
+    return launch_sym<T>(n, AdjointOp<T>{x, v, m, ga, gj, eps2}, gx, gv, gm, ws, st);
+}
 }  // namespace g6a
 
 #define G6A_WS_API(S, T)                                                                        \
@@ -701,6 +801,17 @@ int forces_ws(int n, const T *x, const T *v, const T *m, T eps2, T *acc, T *jerk
     {                                                                                          \
         return g6a::forces_ws<T>(n, x, v, m, eps2, acc, jerk, ws, ws_bytes,                     \
                                  static_cast<hipStream_t>(stream));                             \
+    }                                                                                          \
+    G6A_API long long g6a_adjoint_workspace_##S(int n)                                           \
+    {                                                                                          \
+        return g6a::sym_bytes<T, g6a::AdjointOp<T>>(n);                                         \
+    }                                                                                          \
+    G6A_API int g6a_adjoint_ws_##S(int n, const T *x, const T *v, const T *m, const T *ga,       \
+                                   const T *gj, T eps2, T *gx, T *gv, T *gm, void *ws,          \
+                                   long long ws_bytes, void *stream)                            \
+    {                                                                                          \
+        return g6a::adjoint_ws<T>(n, x, v, m, ga, gj, eps2, gx, gv, gm, ws, ws_bytes,           \
+                                  static_cast<hipStream_t>(stream));                            \
     }
 G6A_WS_API(f32, float)
 G6A_WS_API(f64, double)

@@ -2,7 +2,7 @@
 
 * :class:`PairForce` — torch.autograd.Function over the hand-written HIP
   kernels g6a_forces_ws_* (acc, jerk of the softened pair sum, the arithmetic of
-  lib/g6lib/g6lib.c:165-183) and g6a_adjoint_* (their vector-Jacobian
+  lib/g6lib/g6lib.c:165-183) and g6a_adjoint_ws_* (their vector-Jacobian
   product: dL/dx, dL/dv, dL/dm from dL/dacc, dL/djerk).  float32 and float64
   tensors on the GPU; no CPU fallback.
 * :class:`HermiteStep` — one fixed 4th-order Hermite step, the scheme of
@@ -47,15 +47,16 @@ def _kernels():
             f = getattr(L, "g6a_forces_" + name)
             f.restype = C.c_int
             f.argtypes = [C.c_int, vp, vp, vp, real, vp, vp, vp]
-            f = getattr(L, "g6a_forces_workspace_" + name)
-            f.restype = C.c_longlong
-            f.argtypes = [C.c_int]
+            for what in ("forces", "adjoint"):
+                f = getattr(L, f"g6a_{what}_workspace_{name}")
+                f.restype = C.c_longlong
+                f.argtypes = [C.c_int]
             f = getattr(L, "g6a_forces_ws_" + name)
             f.restype = C.c_int
             f.argtypes = [C.c_int, vp, vp, vp, real, vp, vp, vp, C.c_longlong, vp]
-            g = getattr(L, "g6a_adjoint_" + name)
+            g = getattr(L, "g6a_adjoint_ws_" + name)
             g.restype = C.c_int
-            g.argtypes = [C.c_int, vp, vp, vp, vp, vp, real, vp, vp, vp, vp]
+            g.argtypes = [C.c_int, vp, vp, vp, vp, vp, real, vp, vp, vp, vp, C.c_longlong, vp]
             for fn, args in (("g6a_step_predict_", [C.c_int, vp, vp, vp, vp, d, vp, vp, vp]),
                              ("g6a_step_correct_", [C.c_int, vp, vp, vp, vp, vp, vp, d, vp, vp,
                                                     vp]),
@@ -104,6 +105,14 @@ def _forces(x, v, m, eps2, acc, jerk, stream):
           acc.data_ptr(), jerk.data_ptr(), _ptr(ws), size, stream)
 
 
+def _adjoint(x, v, m, ga, gj, eps2, gx, gv, gm, stream):
+    n = x.shape[0]
+    ws, size = _workspace("g6a_adjoint_workspace_", x.dtype, n, x.device)
+    _call("g6a_adjoint_ws_", x.dtype, n, x.data_ptr(), v.data_ptr(), m.data_ptr(), ga.data_ptr(),
+          gj.data_ptr(), float(eps2), gx.data_ptr(), gv.data_ptr(), gm.data_ptr(), _ptr(ws), size,
+          stream)
+
+
 class PairForce(torch.autograd.Function):
     """acc, jerk = PairForce.apply(x, v, m, eps2)  with x, v (n, 3), m (n,)."""
 
@@ -122,17 +131,11 @@ class PairForce(torch.autograd.Function):
         x, v, m = ctx.saved_tensors
         ga = torch.zeros_like(x) if ga is None else ga.contiguous()
         gj = torch.zeros_like(x) if gj is None else gj.contiguous()
-        n = x.shape[0]
         gx = torch.empty_like(x)
         gv = torch.empty_like(v)
         gm = torch.empty_like(m)
-        L = _kernels()
-        stream = torch.cuda.current_stream(x.device).cuda_stream
-        rc = getattr(L, "g6a_adjoint_" + _suffix(x.dtype))(
-            n, x.data_ptr(), v.data_ptr(), m.data_ptr(), ga.data_ptr(), gj.data_ptr(), ctx.eps2,
-            gx.data_ptr(), gv.data_ptr(), gm.data_ptr(), stream)
-        if rc != 0:
-            raise RuntimeError(f"g6a_adjoint failed ({rc})")
+        _adjoint(x, v, m, ga, gj, ctx.eps2, gx, gv, gm,
+                 torch.cuda.current_stream(x.device).cuda_stream)
         return gx, gv, gm, None
 
 
@@ -190,9 +193,7 @@ class HermiteStep(torch.autograd.Function):
               _ptr(gj1), ctx.dt, gx.data_ptr(), gv.data_ptr(), ga.data_ptr(), gj.data_ptr(),
               ga1t.data_ptr(), gj1t.data_ptr(), stream)
         gxp, gvp, gm = torch.empty_like(xp), torch.empty_like(vp), torch.empty_like(m)
-        _call("g6a_adjoint_", xp.dtype, n, xp.data_ptr(), vp.data_ptr(), m.data_ptr(),
-              ga1t.data_ptr(), gj1t.data_ptr(), ctx.eps2, gxp.data_ptr(), gvp.data_ptr(),
-              gm.data_ptr(), stream)
+        _adjoint(xp, vp, m, ga1t, gj1t, ctx.eps2, gxp, gvp, gm, stream)
         _call("g6a_step_predict_t_", xp.dtype, n, gxp.data_ptr(), gvp.data_ptr(), ctx.dt,
               gx.data_ptr(), gv.data_ptr(), ga.data_ptr(), gj.data_ptr(), stream)
         return gx, gv, ga, gj, gm, None, None

@@ -192,6 +192,14 @@ int g6a_forces_ws_f32(int n, const float *x, const float *v, const float *m, flo
                       float *acc, float *jerk, void *ws, long long ws_bytes, void *stream);
 int g6a_forces_ws_f64(int n, const double *x, const double *v, const double *m, double eps2,
                       double *acc, double *jerk, void *ws, long long ws_bytes, void *stream);
+long long g6a_adjoint_workspace_f32(int n);
+long long g6a_adjoint_workspace_f64(int n);
+int g6a_adjoint_ws_f32(int n, const float *x, const float *v, const float *m, const float *ga,
+                       const float *gj, float eps2, float *gx, float *gv, float *gm, void *ws,
+                       long long ws_bytes, void *stream);
+int g6a_adjoint_ws_f64(int n, const double *x, const double *v, const double *m,
+                       const double *ga, const double *gj, double eps2, double *gx, double *gv,
+                       double *gm, void *ws, long long ws_bytes, void *stream);
 
 /* Fixed-step Hermite scheme around the pair sum (src/amuse_hermite/
  * interface.cc:266-281 predictor, :536-556 corrector) on the same [n][3]

@@ -206,10 +206,12 @@ def test_fp32_gradient_vs_fp64():
         assert rel < 1e-3, rel.item()
 
 
-# Edges of the pair-once form's blocks (256 rows FP32, 128 FP64): whole blocks
-# with an even and an odd number of them, a last block of one particle and of
-# all but one, a last tile of one column.
-PAIR_ONCE_N = [4864, 4865, 5119, 5120, 5121, 5185, 5311]
+# Edges of the pair-once form's blocks (64 rows below 4800 particles, then
+# 128, FP32 forward 256 from 10000): whole blocks with an even and an odd
+# number of them, a last block of one particle and of all but one, a last
+# tile of one column, and the sizes at which the shape changes.
+PAIR_ONCE_N = [4352, 4353, 4415, 4799, 4800, 4864, 4865, 5119, 5120, 5121, 5185, 9999, 10000,
+               10240, 10241, 10495]
 
 
 @pytest.mark.parametrize("n", PAIR_ONCE_N)
@@ -252,3 +254,45 @@ def test_forward_pair_once_edges(n):
         assert getattr(L, "g6a_forces_ws_" + name)(n, *p, 1e-4, out[2].data_ptr(),
                                                    out[3].data_ptr(), None, 0, st) == 0
         assert torch.equal(out[0], out[2]) and torch.equal(out[1], out[3])
+
+
+@pytest.mark.parametrize("n", [3600, 3648, 3649, 3711, 4799, 4800, 4864, 4865, 4927, 4992, 5121])
+def test_adjoint_pair_once_edges(n):
+    """The adjoint with every unordered pair once, FP64 and FP32, against the
+    pair by ordered pair kernel in FP64 (which the autograd reference pins):
+    every particle within the rounding of the sums, gx and gv summing to
+    zero, and a null workspace giving that kernel's bits."""
+    from amuse_amd import diff
+    x, v, m = tensors(n, 8)
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    ga, gj = (torch.randn(x.shape, dtype=x.dtype, device="cuda", generator=gen) for _ in range(2))
+    L = diff._kernels()
+    st = torch.cuda.current_stream().cuda_stream
+    old = L.g6a_adjoint_f64
+    old.argtypes = L.g6a_adjoint_ws_f64.argtypes[:10] + [L.g6a_adjoint_ws_f64.argtypes[-1]]
+
+    def ptrs(*t):
+        return [q.data_ptr() for q in t]
+
+    for dtype, tol in ((torch.float64, 1e-14), (torch.float32, 1e-5)):
+        ins = [t.to(dtype) for t in (x, v, m, ga, gj)]
+        wide = [t.double() for t in ins]
+        ref = [torch.empty_like(wide[0]), torch.empty_like(wide[0]), torch.empty_like(wide[2])]
+        assert old(n, *ptrs(*wide), 1e-4, *ptrs(*ref), st) == 0
+        out = [torch.empty_like(ins[0]), torch.empty_like(ins[0]), torch.empty_like(ins[2])]
+        diff._adjoint(*ins, 1e-4, *out, st)
+        for name, o, r in zip(("gx", "gv", "gm"), out, ref):
+            # sums of n terms that cancel to ~n^1/2 of their size: against the
+            # largest component over all particles
+            err = (o.double() - r).abs().max() / r.abs().max()
+            print(n, dtype, name, "max error / max", err.item(), flush=True)
+            assert err <= tol, (n, dtype, name, err.item())
+        for o, r in zip(out[:2], ref[:2]):
+            s = o.double().sum(0).abs().max() / r.abs().sum()
+            assert s <= (1e-15 if dtype == torch.float64 else 1e-7), (n, dtype, s.item())
+        if dtype == torch.float64:
+            assert L.g6a_adjoint_workspace_f64(n) > 0
+            same = [torch.empty_like(o) for o in out]
+            assert L.g6a_adjoint_ws_f64(n, *ptrs(*ins), 1e-4, *ptrs(*same), None, 0, st) == 0
+            for o, r in zip(same, ref):
+                assert torch.equal(o, r)
