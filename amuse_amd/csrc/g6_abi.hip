@@ -82,6 +82,9 @@ struct Unit {
     int sp_rows_cap = 0;
     void *sp_base = nullptr;
     g6k::SpatialBuf sp_buf;
+    // Full passes with every unordered pair once: the partial records
+    double *pass_ws = nullptr;
+    size_t pass_ws_bytes = 0;
     JRecord *h_stage = nullptr;
     JRecord *d_hstage = nullptr;  // the device's address of h_stage
     size_t h_stage_cap = 0;
@@ -636,6 +639,9 @@ int do_open(int cluster)
         if (U.sp_rows) (void)hipFree(U.sp_rows);
         if (U.sp_buf.base) (void)hipFree(U.sp_buf.base);
         if (U.sp_buf.tmp) (void)hipFree(U.sp_buf.tmp);
+        if (U.pass_ws) (void)hipFree(U.pass_ws);
+        U.pass_ws = nullptr;
+        U.pass_ws_bytes = 0;
         U.sp_base = nullptr;
         U.sp_rows = nullptr;
         U.sp_cap = U.sp_rows_cap = 0;
@@ -1101,6 +1107,55 @@ int ensure_spatial(int nj)
     return 0;
 }
 
+// Full passes at least this long evaluate every unordered pair once
+// (g6k::launch_pass).  us of a whole pass, pair by ordered pair against
+// pair-once: FP64 160 / 143 at N = 8192, 461 / 360 at 16384, 1557 / 1207 at 32768,
+// 5700 / 4250 at 65536, 22000 / 15900 at 131072; mixed 105 / 115 at 8192, 198 / 180
+// at 12000, 287 / 268 at 16384, 950 / 803 at 32768, 3310 / 2630 at 65536, 12330 /
+// 9090 at 131072.
+constexpr int kPassMinF64 = 8192, kPassMinMixed = 12000;
+
+// Whether a full pass over nj slots holding distinct ids takes the pair-once
+// kernels: under the automatic choice of shapes (a shape that was set or
+// tuned is taken as asked), with room for their records (`ready`).
+int ensure_pass(int nj, bool &ready)
+{
+    ready = false;
+    if (nj < (U.prec == g6k::kF64 ? kPassMinF64 : kPassMinMixed) || U.tile_njs > 0) return 0;
+    for (const auto &t : U.tune)
+        if (nj >= t.ni_lo && nj <= t.ni_hi) return 0;
+    const size_t need = g6k::pass_bytes(nj, U.prec);
+    if (need > U.pass_ws_bytes) {
+        HIPCHK(hipStreamSynchronize(U.stream), "pass sync");
+        if (U.pass_ws) (void)hipFree(U.pass_ws);
+        U.pass_ws = nullptr;
+        U.pass_ws_bytes = 0;
+        if (hipMalloc(reinterpret_cast<void **>(&U.pass_ws), need) != hipSuccess) {
+            // no room for the records: the other kernels need less
+            (void)hipGetLastError();
+            U.pass_ws = nullptr;
+            return 0;
+        }
+        U.pass_ws_bytes = need;
+    }
+    ready = true;
+    return 0;
+}
+
+int run_force_pass(int nj, double eps2, bool want_nn)
+{
+    Unit::Ev ev;
+    timed_begin(ev, 0, double(nj) * double(nj));
+    HIPCHK(g6k::launch_pass(U.js, U.ib, nj, eps2, U.prec, want_nn, U.pass_ws, U.stream),
+           "pass kernels");
+    timed_end(ev);
+    U.out_direct = false;
+    U.launched = true;
+    U.launched_nn = want_nn;
+    U.last_ni = nj;
+    return 0;
+}
+
 // Full pass (i = every slot) of the mixed path in spatial order: the slots
 // sorted along a Morton curve (g6k::spatial_order), the i-block taken from
 // the sorted copy, the force kernel for spatially ordered slots, the fold,
@@ -1180,6 +1235,12 @@ G6_API int g6x_calc_self(int nj, int i0, int ni, double eps2, int want_nn)
         bool done = false;
         rc = run_force_spatial(nj, eps2, want_nn != 0, done);
         if (rc || done) return rc;
+    }
+    if (distinct && i0 == 0 && ni == nj) {
+        bool ready = false;
+        rc = ensure_pass(nj, ready);
+        if (rc) return rc;
+        if (ready) return run_force_pass(nj, eps2, want_nn != 0);
     }
     HIPCHK(g6k::launch_iblock_self(U.js, U.ib, i0, ni, U.prec, U.stream), "iblock self");
     return run_force(ni, nj, eps2, want_nn != 0, distinct ? i0 : -1);

@@ -237,6 +237,13 @@ hipError_t launch_force(const JStore &s, const IBlock &b, int ni, int nj,
                         const float *tbox = nullptr);
 bool spatial_cfg_supported(const ForceCfg &c);
 
+// Full pass over slots [0, n), all holding distinct ids, every unordered pair
+// once (g6_pass.hip): acc, jerk, pot (and nn) of the slots into b's result
+// rows, through a workspace of pass_bytes.
+size_t pass_bytes(int n, int prec);
+hipError_t launch_pass(const JStore &s, const IBlock &b, int n, double eps2, int prec,
+                       bool want_nn, double *ws, hipStream_t st);
+
 // Spatial order of a full pass (g6_spatial.hip): the mixed predicted slots
 // [0, nj) of `s` (all holding distinct ids) sorted along a Morton curve of
 // their positions into `o` (mixed predicted arrays, id and pid), perm[k] =

@@ -632,3 +632,60 @@ def test_mixed_precision_error_bounds(g6):
         assert np.median(cond) < 2e-7, (name, np.median(cond))
     print("mixed error (max cond, median cond, median rel):", stats)
     assert (nn == onn).mean() > 0.99
+
+
+# Edges of the pair-once full pass: blocks of 512 slots (768 from 50000 FP64,
+# 20000 mixed), tiles of 64: whole blocks, odd and even in number, a last block
+# of one slot and of all but one, and the smallest and first wide sizes.
+@pytest.mark.parametrize("prec,n", [(0, 8192), (0, 8193), (0, 8703), (0, 9216), (0, 9279),
+                                    (0, 50000), (0, 50689), (1, 12000), (1, 12288), (1, 12289),
+                                    (1, 12800), (1, 19999), (1, 20000), (1, 20736), (1, 20737)])
+def test_pair_once_full_pass_edges(g6, prec, n):
+    """Full passes with every unordered pair once (the automatic choice for
+    distinct ids): the slots at the edges of blocks and tiles against the
+    oracle, every nearest neighbour equal to the pair by ordered pair kernel's
+    (same r^2 bits, first slot of a tie), repeat runs bit for bit, Newton's
+    third law over all slots, and the same sums without nearest neighbours."""
+    st = plummer_state(n, n, dt_nonzero=False)
+    ids, m, x, v = st["ids"], st["m"], st["x"], st["v"]
+    # a lattice of exact ties in the middle of the system
+    k = 300
+    g = np.stack(np.meshgrid(np.arange(5), np.arange(6), np.arange(10), indexing="ij"), -1)
+    at = np.random.Generator(np.random.PCG64(n)).choice(n, k, replace=False)
+    x = x.copy()
+    x[at] = 20.0 + g.reshape(-1, 3) / 8.0
+    g6.set_precision(prec)
+    try:
+        g6.reset()
+        upload(g6, x, v, st["a2"], st["j6"], st["k18"], m, st["tj"], ids)
+        g6.set_ti(st["ti"])
+        print_case(f"pair-once pass prec={prec} n={n}")
+        g6.calc_self(n, 0, n, 1e-4, nn=True)
+        a, j, p, nn = g6.fetch(n)
+        g6.calc_self(n, 0, n, 1e-4, nn=True)
+        for q, r in zip((a, j, p, nn), g6.fetch(n)):
+            assert np.array_equal(q, r)
+        g6.calc_self(n, 0, n, 1e-4, nn=False)
+        for q, r in zip((a, j, p), g6.fetch(n, nn=False)):
+            assert np.array_equal(q, r)
+        g6.set_tiles(1, 2, 8)
+        g6.calc_self(n, 0, n, 1e-4, nn=True)
+        nn_ref = g6.fetch(n)[3]
+        g6.set_tiles(0, 0)
+        assert np.array_equal(nn, nn_ref), np.nonzero(nn != nn_ref)[0][:10]
+        s = np.unique(np.concatenate([np.arange(0, n, 512), np.arange(511, n, 512), [63, 64, n - 1],
+                                      at[:8]]))
+        ea, ej, ep, sa, sj, sp = oracle.force_ld(ids[s], x[s], v[s], 1e-4, ids, m, x, v)
+        bounds = ((1e-15, 4e-15, 1e-15) if prec == 0 else (2e-6, 2e-6, 2e-6))
+        for val, ex, sm, tol, name in ((a, ea, sa, bounds[0], "acc"), (j, ej, sj, bounds[1], "jerk"),
+                                       (p, ep, sp, bounds[2], "pot")):
+            d = np.abs(val[s] - ex).reshape(len(s), -1)
+            d = np.sqrt((d * d).sum(1))
+            print(n, prec, name, "max |d|/sum|term|", (d / sm).max(), flush=True)
+            assert (d <= tol * sm).all(), (name, (d / sm).max())
+        for q, name in ((a, "acc"), (j, "jerk")):
+            r = np.linalg.norm((m[:, None] * q).sum(0)) / (m * np.linalg.norm(q, axis=1)).sum()
+            assert r <= (1e-14 if prec == 0 else 1e-7), (name, r)
+    finally:
+        g6.set_tiles(0, 0)
+        g6.set_precision(0)
