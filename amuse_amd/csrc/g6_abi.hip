@@ -1069,7 +1069,11 @@ G6_API int g6x_set_npipes(int npipes)
 }
 G6_API const char *g6x_last_error(void) { return U.err.c_str(); }
 
-// Full passes at least this long take the spatial order (mixed path).
+// Full passes at least this long take the spatial order (mixed path, shapes
+// that were set or tuned; the automatic choice takes the pair-once kernels,
+// in slot order: N = 262144 36.2 against 44.9 ms.  Pair-once in spatial order
+// was no faster, 39.9 ms: the far pairs' fewer instructions issued at a lower
+// rate, and the order itself takes 1.4 ms).
 constexpr int kSpatialMin = 1 << 17;
 
 int ensure_spatial(int nj)
@@ -1230,17 +1234,16 @@ G6_API int g6x_calc_self(int nj, int i0, int ni, double eps2, int want_nn)
     U.latched = false;
     U.in_direct = false;  // the i-block is in the device rows
     const bool distinct = U.id_repeats == 0 && U.n_filled == nj && U.nj_hw == nj;
-    if (U.spatial && distinct && U.prec == g6k::kMixed && i0 == 0 && ni == nj &&
-        nj >= kSpatialMin) {
-        bool done = false;
-        rc = run_force_spatial(nj, eps2, want_nn != 0, done);
-        if (rc || done) return rc;
-    }
     if (distinct && i0 == 0 && ni == nj) {
         bool ready = false;
         rc = ensure_pass(nj, ready);
         if (rc) return rc;
         if (ready) return run_force_pass(nj, eps2, want_nn != 0);
+        if (U.spatial && U.prec == g6k::kMixed && nj >= kSpatialMin) {
+            bool done = false;
+            rc = run_force_spatial(nj, eps2, want_nn != 0, done);
+            if (rc || done) return rc;
+        }
     }
     HIPCHK(g6k::launch_iblock_self(U.js, U.ib, i0, ni, U.prec, U.stream), "iblock self");
     return run_force(ni, nj, eps2, want_nn != 0, distinct ? i0 : -1);

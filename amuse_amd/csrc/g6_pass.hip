@@ -31,7 +31,7 @@ namespace g6k {
 namespace {
 
 constexpr int kCol = g6s::kCol;
-constexpr int kRowFields = 16, kColFields = 8;
+constexpr int kColFields = 8;
 // One launch: rows of every block against the blocks d0 <= d < d1 places on.
 struct PassArgs {
     const double *jx, *jy, *jz, *jm, *jvx, *jvy, *jvz;                     // FP64
@@ -39,7 +39,7 @@ struct PassArgs {
     double eps2;
     int n, nb, d0, d1;
     int per, parts;     // tiles per workgroup, workgroups per row block
-    double *rowrec;     // [workgroup][kRowFields][R]: hi and lo of the sums, r^2, its tile
+    double *rowrec;     // [workgroup][Op::kRow][R]: the sums (FP64: hi and lo), r^2, its tile
     double *colrec;     // [d - max(d0, 1)][kColFields][n]: the sums, r^2
 };
 
@@ -122,6 +122,7 @@ struct PassF64 {
     static constexpr int W = 4;  // LDS words of a column: (x y), (z m), (vx vy), (vz -)
     // tiles a lane's plain sums run over before they are folded (256 pairs)
     static constexpr int kFold = 4;
+    static constexpr int kSum = 2, kRow = 16;  // values of a row's sum, of its record
     // the columns' sums continue on from lane to lane (plain sums of 64 IPL
     // terms): a rotation moves 64-bit values and does not fuse with an add
     static constexpr bool kChain = true;
@@ -190,6 +191,7 @@ struct PassMx {
     using V = float4;
     static constexpr int W = 3;  // (hx hy hz m), (lx ly lz vx), (vy vz - -)
     static constexpr int kFold = 1;
+    static constexpr int kSum = 1, kRow = 9;
     static constexpr bool kChain = false;
 
     struct Row {
@@ -340,7 +342,7 @@ __global__ void __launch_bounds__(kWG, (sizeof(typename Op::T) == 8 ? 2 : IPL ==
     }
     // the rows' record; FP64: hi and lo of the sums so far (in cache between
     // folds: in registers they would cost the kernel a row per lane)
-    double *const rec = p.rowrec + size_t(blockIdx.x) * kRowFields * R;  // wave-uniform
+    double *const rec = p.rowrec + size_t(blockIdx.x) * Op::kRow * R;  // wave-uniform
     const unsigned at = wave * kCol * IPL + lane;
     bool any = false;
     auto fold = [&]() {
@@ -426,13 +428,10 @@ __global__ void __launch_bounds__(kWG, (sizeof(typename Op::T) == 8 ? 2 : IPL ==
     for (int i = 0; i < IPL; i++) {
         if constexpr (sizeof(T) == 4) {
 #pragma unroll
-            for (int k = 0; k < 7; k++) {
-                (rec + 2 * k * R)[at + kCol * i] = tot[i][k].value();
-                (rec + (2 * k + 1) * R)[at + kCol * i] = 0.0;
-            }
+            for (int k = 0; k < 7; k++) (rec + k * R)[at + kCol * i] = tot[i][k].value();
         }
-        (rec + 14 * R)[at + kCol * i] = double(best[i]);
-        (rec + 15 * R)[at + kCol * i] = double(btile[i]);
+        (rec + (Op::kRow - 2) * R)[at + kCol * i] = double(best[i]);
+        (rec + (Op::kRow - 1) * R)[at + kCol * i] = double(btile[i]);
     }
 }
 
@@ -440,6 +439,7 @@ __global__ void __launch_bounds__(kWG, (sizeof(typename Op::T) == 8 ? 2 : IPL ==
 // of 256 particles each (run[2 f], run[2 f + 1]: hi and lo), 7 the smallest
 // r^2 (run[14]) and its range (run[15]: twice its first slot, plus 1 for a
 // row block's).  first: nothing is running yet.  HBM-bound.
+template <class Op>
 __global__ void __launch_bounds__(256) k_pass_sum(PassArgs p, int R, double *__restrict__ run,
                                                   int first)
 {
@@ -448,8 +448,8 @@ __global__ void __launch_bounds__(256) k_pass_sum(PassArgs p, int R, double *__r
     const size_t n = size_t(p.n);
     const int b = i / R, e0 = max(p.d0, 1);
     const double *col = p.colrec + size_t(f) * n + i;
-    const size_t cs = kColFields * n, rs = size_t(kRowFields) * R;
-    const double *row = p.rowrec + size_t(b) * p.parts * rs + size_t(2 * f) * R + (i - b * R);
+    const size_t cs = kColFields * n, rs = size_t(Op::kRow) * R;
+    const double *row = p.rowrec + size_t(b) * p.parts * rs + size_t(Op::kSum * f) * R + (i - b * R);
     // the block opposite (nb even) has no record from the second half's side
     int e1 = p.d1;
     if (e1 > e0 && 2 * (e1 - 1) == p.nb && b < p.nb / 2) e1--;
@@ -461,7 +461,7 @@ __global__ void __launch_bounds__(256) k_pass_sum(PassArgs p, int R, double *__r
 #pragma unroll 4
         for (int k = 0; k < p.parts; k++) {
             two_sum_add_d(h, l, row[k * rs]);
-            l += row[k * rs + R];
+            if (Op::kSum == 2) l += row[k * rs + R];
         }
         run[size_t(2 * f) * n + i] = h;
         run[size_t(2 * f + 1) * n + i] = l;
@@ -539,7 +539,7 @@ struct PassPlan {
 
     int slots;           // workgroups the chip holds at a time
 
-    PassPlan(int n, int ipl, int slots_) : slots(slots_)
+    PassPlan(int n, int ipl, int slots_, int fields) : slots(slots_)
     {
         R = kWG * ipl;
         nb = (n + R - 1) / R;
@@ -552,7 +552,7 @@ struct PassPlan {
         // (a launch over fewer distances may have more workgroups than one of
         // `step`, but not more than these)
         const long long parts = std::min(step * q, std::max(1, kPassWgs / nb));
-        rec = (long long)kColFields * step * n + (long long)kRowFields * R * nb * parts;
+        rec = (long long)kColFields * step * n + (long long)fields * R * nb * parts;
     }
     static constexpr long long kPassRecs = 1ll << 29;
     // Workgroups per row block of a launch over `nd` distances: the split
@@ -572,7 +572,7 @@ struct PassPlan {
         }
         return best;
     }
-    static constexpr int kPassWgs = 4096;
+    static constexpr int kPassWgs = 8192;
 };
 
 // rows per lane
@@ -588,7 +588,8 @@ template <class Op, int IPL>
 hipError_t pass_run(PassArgs a, const JStore &s, const IBlock &b, bool want_nn, double *ws,
                     hipStream_t st)
 {
-    const PassPlan pl(a.n, IPL, pass_slots(IPL, sizeof(typename Op::T) == 8 ? kF64 : kMixed));
+    const PassPlan pl(a.n, IPL, pass_slots(IPL, sizeof(typename Op::T) == 8 ? kF64 : kMixed),
+                      Op::kRow);
     double *run = ws;
     a.colrec = ws + pl.run;
     a.rowrec = a.colrec + (long long)kColFields * pl.step * a.n;
@@ -600,7 +601,7 @@ hipError_t pass_run(PassArgs a, const JStore &s, const IBlock &b, bool want_nn, 
         a.parts = pl.parts_of(a.d1 - a.d0);
         a.per = (u + a.parts - 1) / a.parts;
         hipLaunchKernelGGL((k_pass<Op, IPL>), dim3(pl.nb * a.parts), dim3(kWG), 0, st, a);
-        hipLaunchKernelGGL(k_pass_sum, dim3((a.n + 255) / 256, want_nn ? 8 : 7), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_pass_sum<Op>, dim3((a.n + 255) / 256, want_nn ? 8 : 7), dim3(256), 0, st,
                            a, pl.R, run, int(d == 0));
     }
     hipLaunchKernelGGL(k_pass_end<Op>, dim3((a.n + 4 * kEnd - 1) / (4 * kEnd)), dim3(256), 0, st, a, pl.R, run,
@@ -613,7 +614,8 @@ hipError_t pass_run(PassArgs a, const JStore &s, const IBlock &b, bool want_nn, 
 size_t pass_bytes(int n, int prec)
 {
     const int ipl = pass_ipl(n, prec);
-    const PassPlan pl(n, ipl, pass_slots(ipl, prec));
+    const PassPlan pl(n, ipl, pass_slots(ipl, prec),
+                      prec == kF64 ? PassF64::kRow : PassMx::kRow);
     return sizeof(double) * size_t(pl.run + pl.rec);
 }
 

@@ -87,10 +87,13 @@ int g6x_calc_self_noalloc(int nj, int i0, int ni, double eps2, double acc[][3],
 int g6x_sync(void);
 /* Full passes in spatial order (default 1): a g6x_calc_self over every slot
  * (i0 = 0, ni = nj >= 131072) in the mixed path, with every slot holding a
- * distinct id, sorts the slots along a Morton curve of their positions and
- * takes pairs of far-apart i-blocks and j-tiles with one FP32 subtraction
- * per component relative to the i-block's centre (same error bound as the
- * double-single difference).  0: slot order always. */
+ * distinct id and a tile shape that was set or tuned (njs = 1), sorts the
+ * slots along a Morton curve of their positions and takes pairs of far-apart
+ * i-blocks and j-tiles with one FP32 subtraction per component relative to
+ * the i-block's centre (same error bound as the double-single difference).
+ * 0: slot order always.  The automatic choice of shapes takes full passes in
+ * slot order, every unordered pair once (partial sums in a workspace of the
+ * library, at most about 1.6 GB). */
 int g6x_set_spatial(int on);
 
 /* Kernel timing with HIP events recorded on the unit's own stream around
