@@ -16,7 +16,9 @@
 //             size class); j-tiles of the cluster staged in LDS; mixed
 //             (double-single dx, FP32 r^-3, compensated sums) or FP64; the
 //             inverse quartic collision time max(v^4/s^2, m_ij^2 r^2/s^4) is
-//             reduced per cluster with an atomic maximum
+//             reduced per cluster with an atomic maximum; clusters of more
+//             than 128 particles are taken pair by unordered pair
+//             (g6_cluster_pairs.h) while there is work for the whole chip
 //   correct   the time-symmetric corrector (FP64)
 //   update    t += dt, next step from the collision time, retire clusters
 //             that reached t_end
@@ -28,6 +30,7 @@
 // The four kernels of a step contain no memset and no host synchronisation,
 // so a sequence of steps is captured once into a hipGraph and replayed.
 #include "g6_kernels.h"
+#include "g6_cluster_pairs.h"
 #include "g6_gridbar.h"
 #include "../../include/g6x.h"
 
@@ -80,6 +83,15 @@ struct Dev {
     int wl_cap = 0;
     unsigned int *bar = nullptr;  // grid barrier of kc_run (g6bar::kWords, zero at each launch)
     int fill_target = 512;  // items a rebuilt list aims at (see build_items)
+    // Pair-once clusters (g6_cluster_pairs.h): those of the classes in
+    // pair_class whose records start at ws[ws_at[c]] (ws_at < 0: too large for
+    // it), while the list's boost is 1.  boost: of the current host-built list.
+    double *ws = nullptr;
+    long long *ws_at = nullptr;
+    int pair_per = 1;  // units per wave
+    int pair_class = 0;  // bit k: size class k
+    int boost = 1;
+    int pair_fill = 1024;  // units from which a rebuilt list keeps them
 };
 
 // size class of a cluster of n particles: <=16, <=32, ..., <=2048, more
@@ -90,9 +102,18 @@ __host__ __device__ inline int size_class_d(int n)
     return k;
 }
 
-__device__ __forceinline__ unsigned long long dbits(double x)
+// Whether cluster c of n particles is taken pair-once in a list of this boost.
+__device__ __forceinline__ bool pair_once(const Dev &d, int c, int n, int boost)
 {
-    return static_cast<unsigned long long>(__double_as_longlong(x));
+    return boost == 1 && ((d.pair_class >> size_class_d(n)) & 1) && d.ws_at[c] >= 0;
+}
+
+// Work items of a pair-once cluster: four waves each, and never fewer than
+// its particles need at a particle per thread.
+__host__ __device__ inline int pair_items(int n, int per)
+{
+    const int w = (g6cp::Plan(n, per).waves() + 3) / 4, r = (n + kWG - 1) / kWG;
+    return w > r ? w : r;
 }
 
 // ---------------------------------------------------------------------------
@@ -157,6 +178,19 @@ __device__ __forceinline__ void two_sum_d(double &hi, double &lo, double x)
 union TileU {
     TileF f;
     TileD dd;
+};
+// With the waves' parts of the pair-once items.
+template <bool MIXED>
+union PairLds;
+template <>
+union PairLds<true> {
+    TileU tile;
+    g6cp::WaveLds<float, g6cp::Mixed::W> wave[kWG / 64];
+};
+template <>
+union PairLds<false> {
+    TileU tile;
+    g6cp::WaveLds<double, g6cp::Plain::W> wave[kWG / 64];
 };
 
 // max of two floats known to be >= +0 or NaN, on their bits: one integer
@@ -350,6 +384,59 @@ __device__ __forceinline__ void force_item(const Dev &d, TileU &tile, int c, int
     }
 }
 
+// The operations of the pair-once form, and a cluster's records.
+template <bool MIXED>
+struct PairOp;
+template <>
+struct PairOp<true> {
+    using Op = g6cp::Mixed;
+    static __device__ __forceinline__ Op make(const Dev &d)
+    {
+        return {d.hx[0], d.hx[1], d.hx[2], d.lx[0], d.lx[1], d.lx[2], d.fm,
+                d.fv[0], d.fv[1], d.fv[2], float(d.eps2)};
+    }
+};
+template <>
+struct PairOp<false> {
+    using Op = g6cp::Plain;
+    static __device__ __forceinline__ Op make(const Dev &d)
+    {
+        return {d.px[0], d.px[1], d.px[2], d.m, d.pv[0], d.pv[1], d.pv[2], d.eps2};
+    }
+};
+// (the rows' records follow the columns', which are FP32 in the mixed path)
+template <bool MIXED>
+struct PairRecords {
+    using T = typename PairOp<MIXED>::Op::T;
+    T *col;
+    double *row;
+    __device__ __forceinline__ PairRecords(const Dev &d, int c, const g6cp::Plan &p)
+    {
+        double *w = d.ws + d.ws_at[c];
+        col = reinterpret_cast<T *>(w);
+        row = w + p.col_values();
+    }
+};
+
+// The four waves of item k of pair-once cluster c, each by itself.
+// VALU-bound: about 65 instructions per unordered pair against 50 per ordered
+// one of force_item, and units of 64 steps where force_item at a lane per row
+// leaves a serial chain of all the cluster's particles (2048 of them: 170 us).
+// 16 rounds and the first forces of 512 clusters of 16..2048, mixed: 10.8 ->
+// 5.8 ms; of 100 in FP64: 6.3 -> 2.1 ms.
+template <bool MIXED, int NC>
+__device__ __forceinline__ void pair_item(const Dev &d, PairLds<MIXED> &lds, int c, int k)
+{
+    const g6cp::Plan p(d.cnt[c], d.pair_per);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wi = 4 * k + wave;
+    if (wi >= p.waves()) return;
+    const PairRecords<MIXED> rec(d, c, p);
+    float cq = g6cp::wave_item<typename PairOp<MIXED>::Op, NC>(
+        PairOp<MIXED>::make(d), p, d.off[c], wi, lds.wave[wave], rec.col, rec.row);
+    for (int o = 1; o < 64; o <<= 1) cq = umax_f(cq, __shfl_xor(cq, o));
+    if ((threadIdx.x & 63) == 0) atomicMax(&d.cmax[c], __float_as_uint(cq));
+}
+
 // One force pass over the host-built item list: workgroups pull items off
 // the queue (reset by kc_predict) until it is empty.
 template <bool MIXED>
@@ -370,23 +457,83 @@ __global__ void __launch_bounds__(kWG) kc_force(Dev d)
     }
 }
 
-// ---------------------------------------------------------------------------
-// time-symmetric corrector (FP64), src/amuse_hermite/interface.cc:536-556
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void correct_particle(const Dev &d, int p, double dt)
+// Force item (cluster, where, lanes per row; 0: pair-once).
+template <bool MIXED, int NC>
+__device__ __forceinline__ void any_item(const Dev &d, PairLds<MIXED> &lds, int c, int at, int njs)
 {
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        const double oa = d.a[k][p], oj = d.j[k][p], ov = d.v[k][p], ox = d.x[k][p];
-        const double na = d.na[k][p], nj = d.nj[k][p];
-        const double v1 = ov + (oa + na) * dt / 2 + (oj - nj) * dt * dt / 12;
-        d.x[k][p] = ox + (ov + v1) * dt / 2 + (oa - na) * dt * dt / 12;
-        d.v[k][p] = v1;
-        d.a[k][p] = na;
-        d.j[k][p] = nj;
+    if (njs == 0)
+        pair_item<MIXED, NC>(d, lds, c, at);
+    else
+        force_item<MIXED>(d, lds.tile, c, at, njs);
+    __syncthreads();  // the waves of a pair-once item end at different times
+}
+
+// The same for lists with pair-once items (in a kernel of its own: it takes
+// twice the registers).  NC = 6: without the potential of pair-once clusters,
+// which a step does not use.
+template <bool MIXED, int NC>
+__global__ void __launch_bounds__(kWG, MIXED ? 4 : 2) kc_force_pairs(Dev d)
+{
+    __shared__ PairLds<MIXED> lds;
+    __shared__ int s_item;
+    const int t = threadIdx.x;
+    for (;;) {
+        if (t == 0) s_item = atomicAdd(d.queue, 1);
+        __syncthreads();
+        const int it = s_item;
+        __syncthreads();
+        if (it >= d.nitems) break;
+        const int c = d.item_c[it];
+        if (!d.active[c]) continue;
+        any_item<MIXED, NC>(d, lds, c, d.item_i0[it], d.item_njs[it]);
     }
 }
 
+// The sums of a listed particle of a pair-once cluster into the result rows.
+template <bool MIXED>
+__global__ void __launch_bounds__(256) kc_pair_sum(Dev d)
+{
+    const int q = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
+    if (q >= d.nlist) return;
+    const int pt = d.plist[q];
+    const int c = d.pc[pt], n = d.cnt[c];
+    if (!d.active[c] || !pair_once(d, c, n, d.boost)) return;
+    const g6cp::Plan p(n, d.pair_per);
+    const PairRecords<MIXED> rec(d, c, p);
+    const double z = g6cp::record_sum(p, rec.col, rec.row, pt - d.off[c], k);
+    (k < 3 ? d.na[k] : k < 6 ? d.nj[k - 3] : d.npot)[pt] = z;
+}
+
+// ---------------------------------------------------------------------------
+// time-symmetric corrector (FP64), src/amuse_hermite/interface.cc:536-556
+// ---------------------------------------------------------------------------
+// One axis of a particle of cluster c, its new force from the result rows or,
+// for a pair-once cluster, from its records.
+template <bool MIXED, bool PAIRS>
+__device__ __forceinline__ void correct_axis(const Dev &d, int p, int c, double dt, int boost, int k)
+{
+    const int n = d.cnt[c];
+    double na, nj;
+    if (PAIRS && pair_once(d, c, n, boost)) {
+        const g6cp::Plan pl(n, d.pair_per);
+        const PairRecords<MIXED> rec(d, c, pl);
+        na = g6cp::record_sum(pl, rec.col, rec.row, p - d.off[c], k);
+        nj = g6cp::record_sum(pl, rec.col, rec.row, p - d.off[c], 3 + k);
+    } else {
+        na = d.na[k][p];
+        nj = d.nj[k][p];
+    }
+    const double oa = d.a[k][p], oj = d.j[k][p], ov = d.v[k][p], ox = d.x[k][p];
+    const double v1 = ov + (oa + na) * dt / 2 + (oj - nj) * dt * dt / 12;
+    d.x[k][p] = ox + (ov + v1) * dt / 2 + (oa - na) * dt * dt / 12;
+    d.v[k][p] = v1;
+    d.a[k][p] = na;
+    d.j[k][p] = nj;
+}
+
+// blockIdx.y: the axis (three times the loads in flight of a thread per
+// particle, which the records' sums need).
+template <bool MIXED, bool PAIRS>
 __global__ void __launch_bounds__(256) kc_correct(Dev d)
 {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -394,7 +541,7 @@ __global__ void __launch_bounds__(256) kc_correct(Dev d)
     const int p = d.plist[q];
     const int c = d.pc[p];
     if (!d.active[c]) return;
-    correct_particle(d, p, d.dt[c]);
+    correct_axis<MIXED, PAIRS>(d, p, c, d.dt[c], d.boost, blockIdx.y);
 }
 
 // first forces of each cluster become its current acc and jerk
@@ -567,6 +714,7 @@ __device__ __forceinline__ int wg_sum(int v, int *red)
 
 // Workgroup 0: the work list of the clusters active now.  fill = 0: every
 // cluster at its tuned lanes per i (boost 1), as at the start of a run.
+template <bool PAIRS>
 __device__ void build_work_list(const Dev &d, int fill, int *red)
 {
     const int t = threadIdx.x;
@@ -576,6 +724,15 @@ __device__ void build_work_list(const Dev &d, int fill, int *red)
     for (int k = c0; k < c1; k++) act += d.active[d.corder[k]] ? 1 : 0;
     const int covered = wg_sum(act, red);
     int boost = 1;
+    // (as build_items: pair-once clusters with enough work for the chip stay)
+    if (PAIRS && fill) {
+        int units = 0;
+        for (int k = c0; k < c1; k++) {
+            const int c = d.corder[k], n = d.cnt[c];
+            if (d.active[c] && pair_once(d, c, n, 1)) units += int(g6cp::Plan(n, d.pair_per).work());
+        }
+        if (wg_sum(units, red) >= d.pair_fill) fill = 0;
+    }
     if (fill) {
         const int target = max(1, d.fill_target);
         for (; boost < 64; boost *= 2) {
@@ -599,7 +756,7 @@ __device__ void build_work_list(const Dev &d, int fill, int *red)
         const int c = d.corder[k];
         if (!d.active[c]) continue;
         const int n = d.cnt[c], rows = kWG / lanes_of(d, n, boost);
-        mine += (n + rows - 1) / rows;
+        mine += PAIRS && pair_once(d, c, n, boost) ? pair_items(n, d.pair_per) : (n + rows - 1) / rows;
     }
     int incl = mine;
     const int lane = t & 63;
@@ -619,6 +776,15 @@ __device__ void build_work_list(const Dev &d, int fill, int *red)
         const int c = d.corder[k];
         if (!d.active[c]) continue;
         const int n = d.cnt[c], njs = lanes_of(d, n, boost), rows = kWG / njs;
+        if (PAIRS && pair_once(d, c, n, boost)) {
+            const int items = pair_items(n, d.pair_per);
+            for (int i = 0; i < items && at < d.wl_cap; i++, at++) {
+                d.wl_c[at] = c;
+                d.wl_i0[at] = i;
+                d.wl_njs[at] = 0;
+            }
+            continue;
+        }
         for (int i0 = 0; i0 < n && at < d.wl_cap; i0 += rows, at++) {
             d.wl_c[at] = c;
             d.wl_i0[at] = i0;
@@ -634,19 +800,23 @@ __device__ void build_work_list(const Dev &d, int fill, int *red)
     __syncthreads();
 }
 
-// Rows of work item `it`: the particles of (cluster, i0 .. i0 + kWG/njs - 1).
+// Rows of work item `it`: the particles of (cluster, i0 .. i0 + kWG/njs - 1),
+// or the k-th kWG particles of a pair-once cluster.
+template <bool PAIRS>
 __device__ __forceinline__ int item_particle(const Dev &d, int it, int t, int &c)
 {
     c = d.wl_c[it];
-    const int i = d.wl_i0[it] + t;
-    if (t >= kWG / d.wl_njs[it] || i >= d.cnt[c]) return -1;
+    const int njs = d.wl_njs[it];
+    const int i = d.wl_i0[it] * (PAIRS && !njs ? kWG : 1) + t;
+    if (t >= (PAIRS && !njs ? kWG : kWG / njs) || i >= d.cnt[c]) return -1;
     return d.off[c] + i;
 }
 
-template <bool MIXED>
-__global__ void __launch_bounds__(kWG) kc_run(Dev d, long long max_rounds, long long *rounds_out)
+// (item(c, i0, njs): the force of a work item.)
+template <bool MIXED, bool PAIRS, class Item>
+__device__ __forceinline__ void run_rounds(const Dev &d, long long max_rounds,
+                                           long long *rounds_out, Item &&item)
 {
-    __shared__ TileU tile;
     __shared__ int s_item;
     __shared__ int red[kWG / 64];
     const int t = threadIdx.x;
@@ -663,17 +833,17 @@ __global__ void __launch_bounds__(kWG) kc_run(Dev d, long long max_rounds, long 
         // changes only in the update phase, three barriers below)
         const int nact = load_shared_int(d.nactive);
         if (!built || nact * 2 <= covered) {
-            if (blockIdx.x == 0) build_work_list(d, built, red);
+            if (blockIdx.x == 0) build_work_list<PAIRS>(d, built, red);
             if (!grid_barrier(d.bar, gen++)) break;
             built = 1;
             covered = load_shared_int(&d.ctl[1]);
         }
-        const int nwork = load_shared_int(&d.ctl[0]);
+        const int nwork = load_shared_int(&d.ctl[0]), boost = load_shared_int(&d.ctl[2]);
         // predict (and reset the force queue)
         if (blockIdx.x == 0 && t == 0) *d.queue = 0;
         for (int it = blockIdx.x; it < nwork; it += gridDim.x) {
             int c;
-            const int p = item_particle(d, it, t, c);
+            const int p = item_particle<PAIRS>(d, it, t, c);
             if (p >= 0 && d.active[c]) predict_particle(d, p, d.dt[c]);
         }
         if (!grid_barrier(d.bar, gen++)) break;
@@ -686,14 +856,23 @@ __global__ void __launch_bounds__(kWG) kc_run(Dev d, long long max_rounds, long 
             if (it >= nwork) break;
             const int c = d.wl_c[it];
             if (!d.active[c]) continue;
-            force_item<MIXED>(d, tile, c, d.wl_i0[it], d.wl_njs[it]);
+            item(c, d.wl_i0[it], d.wl_njs[it]);
         }
         if (!grid_barrier(d.bar, gen++)) break;
         // correct
         for (int it = blockIdx.x; it < nwork; it += gridDim.x) {
             int c;
-            const int p = item_particle(d, it, t, c);
-            if (p >= 0 && d.active[c]) correct_particle(d, p, d.dt[c]);
+            const int p = item_particle<PAIRS>(d, it, t, c);
+            if (p >= 0 && d.active[c]) {
+                const double dt = d.dt[c];
+                if constexpr (PAIRS) {
+#pragma unroll 1
+                    for (int k = 0; k < 3; k++) correct_axis<MIXED, PAIRS>(d, p, c, dt, boost, k);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 3; k++) correct_axis<MIXED, PAIRS>(d, p, c, dt, boost, k);
+                }
+            }
         }
         if (!grid_barrier(d.bar, gen++)) break;
         // update: time, next step, retire
@@ -704,6 +883,26 @@ __global__ void __launch_bounds__(kWG) kc_run(Dev d, long long max_rounds, long 
         if (load_shared_int(d.nactive) <= 0 || r >= max_rounds) break;
     }
     if (blockIdx.x == 0 && t == 0) *rounds_out = r;
+}
+
+template <bool MIXED>
+__global__ void __launch_bounds__(kWG, MIXED ? 5 : 4) kc_run(Dev d, long long max_rounds, long long *rounds_out)
+{
+    __shared__ TileU tile;
+    run_rounds<MIXED, false>(d, max_rounds, rounds_out, [&](int c, int i0, int njs) {
+        force_item<MIXED>(d, tile, c, i0, njs);
+    });
+}
+
+// For ensembles with pair-once clusters (bounds: no spills to scratch).
+template <bool MIXED>
+__global__ void __launch_bounds__(kWG, MIXED ? 3 : 1)
+kc_run_pairs(Dev d, long long max_rounds, long long *rounds_out)
+{
+    __shared__ PairLds<MIXED> lds;
+    run_rounds<MIXED, true>(d, max_rounds, rounds_out, [&](int c, int i0, int njs) {
+        any_item<MIXED, 6>(d, lds, c, i0, njs);
+    });
 }
 
 __global__ void kc_zero_words(unsigned int *w, int n)
@@ -721,6 +920,7 @@ struct Ensemble {
     void *base = nullptr;
     int precision = 1;
     std::vector<int> cnt, off;
+    std::vector<long long> ws_at;  // as Dev::ws_at
     int ib_rows = 0;
     int persistent_wgs = 0;
     hipGraphExec_t graph = nullptr;
@@ -728,12 +928,66 @@ struct Ensemble {
     int graph_prec = -1;
     int items_clusters = 0;  // clusters covered by the current work items
     int *wl_base = nullptr;  // the persistent run's work list and cluster order
+    void *pair_base = nullptr;  // the pair-once clusters' record offsets, then the records
     double force_ms = 0.0;
     long long launches = 0;
     std::string err;
 };
 
 int size_class(int n) { return size_class_d(n); }
+
+// The automatic shape of a size class: lanes per i (and kTJ j per tile).
+int auto_njs(int k) { return k <= 1 ? 16 : (k <= 3 ? 4 : 1); }
+
+// Classes taken pair-once: from kPairClass on, while their shape is the
+// automatic one (a shape that was set or tuned is taken as asked).  Up to 128
+// particles a cluster is one block with one busy wave.  Records grow as n^2
+// (8192 particles: 130 MB), and a larger cluster has rows enough for the
+// other kernels.
+constexpr int kPairClass = 4;      // clusters of more than 128
+constexpr int kPairMaxN = 8192;
+void pair_rule(Ensemble *E)
+{
+    E->d.pair_class = 0;
+    if (!E->pair_base) return;
+    for (int k = kPairClass; k < kClasses; k++)
+        if (E->d.njs_class[k] == auto_njs(k) && E->d.tj_class[k] == kTJ) E->d.pair_class |= 1 << k;
+}
+
+// The records of the clusters that can be taken pair-once and the units of a
+// wave: as many as leave four waves for each of the chip's SIMDs, at most 4.
+// With a cluster above kPairMaxN, or without room for the records every cluster keeps the other kernels.
+bool pair_setup(Ensemble *E, int cus)
+{
+    Dev &d = E->d;
+    long long units = 0;
+    for (int n : E->cnt) {
+        if (n > kPairMaxN) return true;
+        if (size_class(n) >= kPairClass) units += g6cp::Plan(n, 1).work();
+    }
+    if (units == 0) return true;
+    d.pair_per = int(std::min(4ll, std::max(1ll, units / (16 * cus))));
+    d.pair_fill = 4 * cus;
+    E->ws_at.assign(d.nc, -1);
+    long long at = 0;
+    for (int c = 0; c < d.nc; c++) {
+        const int n = E->cnt[c];
+        if (size_class(n) < kPairClass) continue;
+        E->ws_at[c] = at;
+        at += (g6cp::Plan(n, d.pair_per).values() + 31) / 32 * 32;
+    }
+    const size_t head = (size_t(d.nc) * sizeof(long long) + 255) / 256 * 256;
+    if (hipMalloc(&E->pair_base, head + size_t(at) * sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        E->pair_base = nullptr;
+        E->ws_at.clear();
+        return true;
+    }
+    d.ws_at = static_cast<long long *>(E->pair_base);
+    d.ws = reinterpret_cast<double *>(static_cast<char *>(E->pair_base) + head);
+    return hipMemcpy(d.ws_at, E->ws_at.data(), size_t(d.nc) * sizeof(long long),
+                     hipMemcpyHostToDevice) == hipSuccess;
+}
 
 #define CK(expr)                                                       \
     do {                                                               \
@@ -760,7 +1014,8 @@ struct EventPair {
 // ones.  `only` (host flags, one per cluster) restricts the list to some
 // clusters: every workgroup pulls items one atomic at a time, so items of
 // retired clusters would cost a serial chain of atomics per step.
-// fill: when the covered clusters give fewer than two items per compute unit
+// Clusters of a class in pair_class are pair-once items (njs = 0) at boost 1.
+// fill: when the covered clusters' pair-once units fill less than the chip and they give fewer than two items per compute unit
 // (the last clusters of a run, often with the smallest steps), raise the
 // lanes per i (up to 64) until they do, so a step's latency is not that of
 // a few long items.
@@ -772,7 +1027,15 @@ int build_items(Ensemble *E, const int *only = nullptr, bool fill = false)
         return std::min(64, E->d.njs_class[size_class(n)] * boost);
     };
     int boost = 1;
-    if (fill) {
+    long long units = 0;
+    pair_rule(E);
+    auto pair = [&](int c) {
+        return boost == 1 && !E->ws_at.empty() && E->ws_at[c] >= 0 &&
+               ((E->d.pair_class >> size_class(E->cnt[c])) & 1);
+    };
+    for (int c = 0; c < E->d.nc; c++)
+        if (!(only && !only[c]) && pair(c)) units += g6cp::Plan(E->cnt[c], E->d.pair_per).work();
+    if (fill && units < E->d.pair_fill) {
         const int target = std::max(1, E->persistent_wgs / 2);
         for (; boost < 64; boost *= 2) {
             long long count = 0;
@@ -796,6 +1059,16 @@ int build_items(Ensemble *E, const int *only = nullptr, bool fill = false)
         for (int i = 0; i < n; i++) plist.push_back(E->off[c] + i);
         const int njs = njs_of(n, boost);
         const int rows = kWG / njs;
+        if (pair(c)) {
+            const int items = (g6cp::Plan(n, E->d.pair_per).waves() + 3) / 4;
+            for (int i = 0; i < items; i++) {
+                ic.push_back(c);
+                ii0.push_back(i);
+                injs.push_back(0);
+                cost.push_back(double(kWG) * 128 * E->d.pair_per);
+            }
+            continue;
+        }
         for (int i0 = 0; i0 < n; i0 += rows) {
             ic.push_back(c);
             ii0.push_back(i0);
@@ -828,6 +1101,7 @@ int build_items(Ensemble *E, const int *only = nullptr, bool fill = false)
     if (!plist.empty())
         CK(hipMemcpy(E->d.plist, plist.data(), sizeof(int) * plist.size(), hipMemcpyHostToDevice));
     E->d.nitems = n;
+    E->d.boost = boost;
     E->d.nlist = int(plist.size());
     E->items_clusters = covered;
     if (E->graph) {
@@ -837,15 +1111,20 @@ int build_items(Ensemble *E, const int *only = nullptr, bool fill = false)
     return 0;
 }
 
-int launch_force(Ensemble *E, int prec)
+// Whether the current list holds pair-once items.
+bool has_pairs(const Ensemble *E) { return E->d.pair_class && E->d.boost == 1; }
+
+// pot: with the potential
+int launch_force(Ensemble *E, int prec, bool pot)
 {
     // no more workgroups than items: the surplus would only take the atomic
     // that tells it the queue is empty
     const int wgs = std::max(1, std::min(E->persistent_wgs, E->d.nitems));
-    if (prec == G6X_MIXED)
-        hipLaunchKernelGGL(kc_force<true>, dim3(wgs), dim3(kWG), 0, E->stream, E->d);
-    else
-        hipLaunchKernelGGL(kc_force<false>, dim3(wgs), dim3(kWG), 0, E->stream, E->d);
+    void (*k)(Dev) = prec == G6X_MIXED ? kc_force<true> : kc_force<false>;
+    if (has_pairs(E))
+        k = prec == G6X_MIXED ? (pot ? kc_force_pairs<true, 7> : kc_force_pairs<true, 6>)
+                              : (pot ? kc_force_pairs<false, 7> : kc_force_pairs<false, 6>);
+    hipLaunchKernelGGL(k, dim3(wgs), dim3(kWG), 0, E->stream, E->d);
     return hipGetLastError() == hipSuccess ? 0 : G6X_ERR_HIP;
 }
 
@@ -857,8 +1136,12 @@ int enqueue_step(Ensemble *E, int prec)
 {
     const int pb = list_blocks(E), cb = (E->d.nc + 255) / 256;
     hipLaunchKernelGGL(kc_predict, dim3(pb), dim3(256), 0, E->stream, E->d, 0);
-    if (launch_force(E, prec)) return G6X_ERR_HIP;
-    hipLaunchKernelGGL(kc_correct, dim3(pb), dim3(256), 0, E->stream, E->d);
+    if (launch_force(E, prec, false)) return G6X_ERR_HIP;
+    // (FP32 or FP64 column records; without any, one kernel)
+    void (*correct)(Dev) = !has_pairs(E)       ? kc_correct<false, false>
+                           : prec == G6X_MIXED ? kc_correct<true, true>
+                                               : kc_correct<false, true>;
+    hipLaunchKernelGGL(correct, dim3(pb, 3), dim3(256), 0, E->stream, E->d);
     hipLaunchKernelGGL(kc_update, dim3(cb), dim3(256), 0, E->stream, E->d, 0);
     return hipGetLastError() == hipSuccess ? 0 : G6X_ERR_HIP;
 }
@@ -875,6 +1158,7 @@ static void release(Ensemble *E)
     if (E->d.item_c) (void)hipFree(E->d.item_c);
     if (E->wl_base) (void)hipFree(E->wl_base);
     if (E->base) (void)hipFree(E->base);
+    if (E->pair_base) (void)hipFree(E->pair_base);
     if (E->stream) (void)hipStreamDestroy(E->stream);
     delete E;
 }
@@ -914,7 +1198,7 @@ G6C_API void *g6c_create(int nc, const int counts[], const double m[], const dou
     d.np = int(np);
     d.eps2 = eps2;
     d.dt_param = dt_param > 0.0 ? dt_param : 0.03;
-    for (int k = 0; k < kClasses; k++) E->d.njs_class[k] = k <= 1 ? 16 : (k <= 3 ? 4 : 1);
+    for (int k = 0; k < kClasses; k++) E->d.njs_class[k] = auto_njs(k);
     if (hipStreamCreateWithFlags(&E->stream, hipStreamNonBlocking) != hipSuccess) {
         E->stream = nullptr;
         release(E);
@@ -1008,6 +1292,7 @@ G6C_API void *g6c_create(int nc, const int counts[], const double m[], const dou
         const int zero8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         ok &= hipMemcpy(d.ctl, zero8, sizeof(zero8), hipMemcpyHostToDevice) == hipSuccess;
     }
+    ok = ok && pair_setup(E, cus);
     if (!ok || build_items(E)) {
         release(E);
         return nullptr;
@@ -1028,13 +1313,17 @@ G6C_API const char *g6c_last_error(void *h) { return static_cast<Ensemble *>(h)-
 
 // Forces at the current state (no prediction) in `precision`, then the
 // per-cluster energies from their FP64 potential when precision is FP64.
-static int force_now(Ensemble *E, int precision)
+// pot: with the potentials.
+static int force_now(Ensemble *E, int precision, bool pot)
 {
     // a run may have dropped the items of retired clusters
     if (E->items_clusters < E->d.nc && build_items(E)) return G6X_ERR_HIP;
     hipLaunchKernelGGL(kc_predict, dim3(list_blocks(E)), dim3(256), 0, E->stream, E->d, 1);
-    if (launch_force(E, precision)) return G6X_ERR_HIP;
-    return 0;
+    if (launch_force(E, precision, pot)) return G6X_ERR_HIP;
+    if (has_pairs(E))
+        hipLaunchKernelGGL(precision == G6X_MIXED ? kc_pair_sum<true> : kc_pair_sum<false>,
+                           dim3(list_blocks(E), pot ? 7 : 6), dim3(256), 0, E->stream, E->d);
+    return hipGetLastError() == hipSuccess ? 0 : G6X_ERR_HIP;
 }
 
 // Initial forces and first steps; every cluster becomes active at t = 0.
@@ -1046,7 +1335,7 @@ G6C_API int g6c_start(void *h, double t_end)
     // all clusters active for the initial pass
     std::vector<int> ones(E->d.nc, 1);
     CK(hipMemcpyAsync(E->d.active, ones.data(), sizeof(int) * E->d.nc, hipMemcpyHostToDevice, E->stream));
-    if (force_now(E, E->precision)) return G6X_ERR_HIP;
+    if (force_now(E, E->precision, false)) return G6X_ERR_HIP;
     const int pb = (E->d.np + 255) / 256, cb = (E->d.nc + 255) / 256;
     hipLaunchKernelGGL(kc_take_forces, dim3(pb), dim3(256), 0, E->stream, E->d);
     hipLaunchKernelGGL(kc_update, dim3(cb), dim3(256), 0, E->stream, E->d, 1);
@@ -1063,8 +1352,10 @@ static long long run_persistent(Ensemble *E, long long max_rounds)
     int dev = 0, cus = 0, per_cu = 0;
     CK(hipGetDevice(&dev));
     CK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    const void *kern = E->precision == G6X_MIXED ? reinterpret_cast<const void *>(&kc_run<true>)
-                                                 : reinterpret_cast<const void *>(&kc_run<false>);
+    void (*run)(Dev, long long, long long *) =
+        E->d.pair_class ? (E->precision == G6X_MIXED ? kc_run_pairs<true> : kc_run_pairs<false>)
+                        : (E->precision == G6X_MIXED ? kc_run<true> : kc_run<false>);
+    const void *kern = reinterpret_cast<const void *>(run);
     CK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, kWG, 0));
     if (per_cu <= 0) {
         E->err = "kc_run: no workgroup fits a compute unit";
@@ -1206,7 +1497,7 @@ G6C_API int g6c_energy(void *h, double *energy)
     CK(hipStreamSynchronize(E->stream));
     std::vector<int> ones(E->d.nc, 1);
     CK(hipMemcpyAsync(E->d.active, ones.data(), sizeof(int) * E->d.nc, hipMemcpyHostToDevice, E->stream));
-    if (force_now(E, G6X_FP64)) return G6X_ERR_HIP;
+    if (force_now(E, G6X_FP64, true)) return G6X_ERR_HIP;
     hipLaunchKernelGGL(kc_energy, dim3(E->d.nc), dim3(256), 0, E->stream, E->d);
     CK(hipMemcpyAsync(energy, E->d.energy, sizeof(double) * E->d.nc, hipMemcpyDeviceToHost, E->stream));
     CK(hipMemcpyAsync(E->d.active, saved.data(), sizeof(int) * E->d.nc, hipMemcpyHostToDevice, E->stream));
@@ -1242,7 +1533,7 @@ G6C_API int g6c_forces(void *h, int precision, double acco[][3], double jerko[][
     std::vector<int> saved(E->d.nc), ones(E->d.nc, 1);
     CK(hipMemcpy(saved.data(), E->d.active, sizeof(int) * E->d.nc, hipMemcpyDeviceToHost));
     CK(hipMemcpy(E->d.active, ones.data(), sizeof(int) * E->d.nc, hipMemcpyHostToDevice));
-    if (force_now(E, precision)) return G6X_ERR_HIP;
+    if (force_now(E, precision, true)) return G6X_ERR_HIP;
     CK(hipStreamSynchronize(E->stream));
     const size_t P = size_t(E->d.np);
     std::vector<double> buf(P);
@@ -1279,7 +1570,11 @@ G6C_API int g6c_set_jtiles(void *h, const int *tj_per_class)
         if (v < 16 || v > kTJ || (v & (v - 1))) return G6X_ERR_ARG;
     }
     std::copy(tj_per_class, tj_per_class + kClasses, E->d.tj_class);
-    return 0;
+    const int was = E->d.pair_class;
+    pair_rule(E);
+    if (E->d.pair_class == was) return 0;
+    if (invalidate_work_list(E)) return G6X_ERR_HIP;
+    return build_items(E);
 }
 
 G6C_API int g6c_get_jtiles(void *h, int *tj_per_class)
@@ -1322,7 +1617,7 @@ static int tune_classes(Ensemble *E, hipEvent_t a, hipEvent_t b)
                 E->d.njs_class[k] = njs;
                 if (build_items(E, act.data())) return G6X_ERR_HIP;
                 hipLaunchKernelGGL(kc_predict, dim3(list_blocks(E)), dim3(256), 0, E->stream, E->d, 1);
-                if (launch_force(E, E->precision)) return G6X_ERR_HIP;
+                if (launch_force(E, E->precision, false)) return G6X_ERR_HIP;
                 // the best of two timings of `reps` passes each, reps raised
                 // until a timing covers >= 1 ms (classes of small clusters
                 // take a few µs per pass, where launch jitter would decide)
@@ -1333,7 +1628,7 @@ static int tune_classes(Ensemble *E, hipEvent_t a, hipEvent_t b)
                     for (int r = 0; r < reps; r++) {
                         hipLaunchKernelGGL(kc_predict, dim3(list_blocks(E)), dim3(256), 0,
                                            E->stream, E->d, 1);
-                        if (launch_force(E, E->precision)) return G6X_ERR_HIP;
+                        if (launch_force(E, E->precision, false)) return G6X_ERR_HIP;
                     }
                     CK(hipEventRecord(b, E->stream));
                     CK(hipEventSynchronize(b));
