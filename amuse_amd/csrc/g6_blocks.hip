@@ -61,6 +61,7 @@ struct Driver {
     JStore js;
     IBlock ib;
     double *part = nullptr;
+    long long part_entries = 0;
     void *state_base = nullptr;
     StepCtl *ctl = nullptr;    // device
     StepCtl *h_ctl = nullptr;  // pinned host mirror
@@ -355,6 +356,29 @@ __global__ void __launch_bounds__(256) kb_correct(State s, JStore js, IBlock b,
     fold_min(lo, &c->tmin[par ^ 1]);
 }
 
+// Rows j0 .. j0 + rows - 1 of x and v as [rows][3] each: as last corrected, or
+// (predict) predicted to the system time as idata::predict does.
+__global__ void __launch_bounds__(256) kb_state(State s, const StepCtl *c, int j0, int rows,
+                                                int predict, double *__restrict__ x,
+                                                double *__restrict__ v)
+{
+    const double ts = c->system_time;
+    for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < rows; r += gridDim.x * blockDim.x) {
+        const int j = j0 + r;
+        double xs[3], vs[3], a[3], jk[3], xp[3], vp[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            xs[k] = s.x[k][j]; vs[k] = s.v[k][j]; a[k] = s.a[k][j]; jk[k] = s.j[k][j];
+        }
+        h4::predict_ph4(xs, vs, a, jk, predict ? ts - s.t[j] : 0.0, xp, vp);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            x[3 * size_t(r) + k] = xp[k];
+            v[3 * size_t(r) + k] = vp[k];
+        }
+    }
+}
+
 // Arms a run: end time and block budget; the pending block time moves to
 // slot 0, where the captured sequence (which starts at parity 0) reads it.
 __global__ void kb_arm(StepCtl *c, double t_end, long long budget)
@@ -471,9 +495,9 @@ int setup(Driver *D, int n, const int *ids, const double *m, const double *x, co
     DCK(hipMalloc(&ibase, g6k::iblock_bytes(jcap)));
     g6k::iblock_carve(D->ib, ibase, jcap);
     const long long max_chunks = std::max(1, nblk(n, g6k::kTJ));
-    const long long part_entries = std::min(g6k::kStepPartBudget, max_chunks * (long long)n);
+    D->part_entries = std::min(g6k::kStepPartBudget, max_chunks * (long long)n);
     DCK(hipMalloc(reinterpret_cast<void **>(&D->part),
-                  sizeof(double) * g6k::kPartFieldsD * size_t(part_entries)));
+                  sizeof(double) * g6k::kPartFieldsD * size_t(D->part_entries)));
     DCK(hipMalloc(reinterpret_cast<void **>(&D->ctl), sizeof(StepCtl)));
     DCK(hipHostMalloc(reinterpret_cast<void **>(&D->h_ctl), sizeof(StepCtl)));
     // host state in, times zero
@@ -685,61 +709,40 @@ G6D_API int g6d_energy(void *h, double *kin, double *pot)
     return 0;
 }
 
+// x and v to the host, laid out (and predicted) on the device in the partials'
+// buffer, which no step uses now: two copies instead of thirteen and no
+// arithmetic on the host (evolve and state over one interval: N = 50021 2.28 ->
+// 1.78 ms, N = 1024 1.97 -> 1.73 ms).
+static int copy_state(Driver *D, double (*x)[3], double (*v)[3], int predict)
+{
+    const long long cap = D->part_entries * g6k::kPartFieldsD / 6;
+    for (long long j0 = 0; j0 < D->st.n; j0 += cap) {
+        const int rows = int(std::min<long long>(cap, D->st.n - j0));
+        double *dx = D->part, *dv = D->part + 3 * size_t(rows);
+        hipLaunchKernelGGL(g6b::kb_state, dim3(std::min(g6b::nblk(rows, 256), g6b::kGrid)),
+                           dim3(256), 0, D->stream, D->st, D->ctl, int(j0), rows, predict, dx, dv);
+        DCK(hipGetLastError());
+        const size_t bytes = 3 * size_t(rows) * sizeof(double);
+        DCK(hipMemcpyAsync(x[j0], dx, bytes, hipMemcpyDeviceToHost, D->stream));
+        DCK(hipMemcpyAsync(v[j0], dv, bytes, hipMemcpyDeviceToHost, D->stream));
+        DCK(hipStreamSynchronize(D->stream));
+    }
+    return 0;
+}
+
 // Positions and velocities as last corrected, each at its particle's own
 // time ([n][3] each; ph4's get_state, src/amuse_ph4/interface.cc:485-502).
 G6D_API int g6d_state_raw(void *h, double (*x)[3], double (*v)[3])
 {
     if (!h || !x || !v) return G6X_ERR_ARG;
-    Driver *D = static_cast<Driver *>(h);
-    g6b::State &s = D->st;
-    const size_t nd = size_t(s.n);
-    if (g6b::read_ctl(D)) return G6X_ERR_HIP;
-    std::vector<double> col(6 * nd);
-    double *rows[6] = {s.x[0], s.x[1], s.x[2], s.v[0], s.v[1], s.v[2]};
-    for (int r = 0; r < 6; r++)
-        if (hipMemcpyAsync(col.data() + r * nd, rows[r], nd * 8, hipMemcpyDeviceToHost,
-                           D->stream) != hipSuccess)
-            return G6X_ERR_HIP;
-    if (hipStreamSynchronize(D->stream) != hipSuccess) return G6X_ERR_HIP;
-    for (size_t i = 0; i < nd; i++)
-        for (int k = 0; k < 3; k++) {
-            x[i][k] = col[k * nd + i];
-            v[i][k] = col[(3 + k) * nd + i];
-        }
-    return 0;
+    return copy_state(static_cast<Driver *>(h), x, v, 0);
 }
 
 // Positions and velocities predicted to the system time ([n][3] each).
 G6D_API int g6d_state(void *h, double (*x)[3], double (*v)[3])
 {
     if (!h || !x || !v) return G6X_ERR_ARG;
-    Driver *D = static_cast<Driver *>(h);
-    g6b::State &s = D->st;
-    const int n = s.n;
-    const size_t nd = size_t(n);
-    if (g6b::read_ctl(D)) return G6X_ERR_HIP;
-    std::vector<double> col(12 * nd), t(nd);
-    double *rows[12] = {s.x[0], s.x[1], s.x[2], s.v[0], s.v[1], s.v[2],
-                        s.a[0], s.a[1], s.a[2], s.j[0], s.j[1], s.j[2]};
-    for (int r = 0; r < 12; r++)
-        if (hipMemcpyAsync(col.data() + r * nd, rows[r], nd * 8, hipMemcpyDeviceToHost,
-                           D->stream) != hipSuccess)
-            return G6X_ERR_HIP;
-    if (hipMemcpyAsync(t.data(), s.t, nd * 8, hipMemcpyDeviceToHost, D->stream) != hipSuccess ||
-        hipStreamSynchronize(D->stream) != hipSuccess)
-        return G6X_ERR_HIP;
-    const double ts = D->h_ctl->system_time;
-    for (int i = 0; i < n; i++) {
-        double xi[3], vi[3], ai[3], ji[3];
-        for (int k = 0; k < 3; k++) {
-            xi[k] = col[k * nd + i];
-            vi[k] = col[(3 + k) * nd + i];
-            ai[k] = col[(6 + k) * nd + i];
-            ji[k] = col[(9 + k) * nd + i];
-        }
-        h4::predict_ph4(xi, vi, ai, ji, ts - t[i], x[i], v[i]);
-    }
-    return 0;
+    return copy_state(static_cast<Driver *>(h), x, v, 1);
 }
 
 // Per-particle times and steps.

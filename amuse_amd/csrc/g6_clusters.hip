@@ -627,12 +627,22 @@ __global__ void __launch_bounds__(256) kc_energy(Dev d)
     if (threadIdx.x == 0) d.energy[c] = red[0];
 }
 
-__global__ void kc_set_active_count(Dev d)
+// Every cluster active (one workgroup).
+__global__ void __launch_bounds__(kWG) kc_activate(Dev d)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        int n = 0;
-        for (int c = 0; c < d.nc; c++) n += d.active[c];
-        *d.nactive = n;
+    for (int c = threadIdx.x; c < d.nc; c += kWG) d.active[c] = 1;
+    if (threadIdx.x == 0) *d.nactive = d.nc;
+}
+
+// x and v of every particle as [np][3] each.
+__global__ void __launch_bounds__(256) kc_state(Dev d, double *__restrict__ x, double *__restrict__ v)
+{
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= d.np) return;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        x[3 * size_t(p) + k] = d.x[k][p];
+        v[3 * size_t(p) + k] = d.v[k][p];
     }
 }
 
@@ -928,6 +938,8 @@ struct Ensemble {
     int graph_prec = -1;
     int items_clusters = 0;  // clusters covered by the current work items
     int *wl_base = nullptr;  // the persistent run's work list and cluster order
+    int *h_active = nullptr;  // the active count, read back after each launch (pinned)
+    double *aos = nullptr;    // [6][np]: x and v as the caller's arrays lay them out
     void *pair_base = nullptr;  // the pair-once clusters' record offsets, then the records
     double force_ms = 0.0;
     long long launches = 0;
@@ -1159,6 +1171,7 @@ static void release(Ensemble *E)
     if (E->wl_base) (void)hipFree(E->wl_base);
     if (E->base) (void)hipFree(E->base);
     if (E->pair_base) (void)hipFree(E->pair_base);
+    if (E->h_active) (void)hipHostFree(E->h_active);
     if (E->stream) (void)hipStreamDestroy(E->stream);
     delete E;
 }
@@ -1204,11 +1217,11 @@ G6C_API void *g6c_create(int nc, const int counts[], const double m[], const dou
         release(E);
         return nullptr;
     }
-    // one allocation: per-particle doubles (x v a j px pv na nj = 24, m, npot), floats (10),
+    // one allocation: per-particle doubles (x v a j px pv na nj = 24, m, npot, aos 6), floats (10),
     // ints (pc plist), per-cluster doubles (t dt energy) + uint (cmax) + ints (off cnt active nsteps)
     const size_t P = size_t(np), Cn = size_t(nc);
     auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
-    size_t bytes = al(P * 8) * 26 + al(P * 4) * 12 + al(Cn * 8) * 4 + al(Cn * 4) * 4 + 256;
+    size_t bytes = al(P * 8) * 32 + al(P * 4) * 12 + al(Cn * 8) * 4 + al(Cn * 4) * 4 + 256;
     if (hipMalloc(&E->base, bytes) != hipSuccess) {
         E->base = nullptr;
         release(E);
@@ -1219,6 +1232,8 @@ G6C_API void *g6c_create(int nc, const int counts[], const double m[], const dou
     auto F = [&](float *&p) { p = reinterpret_cast<float *>(q); q += al(P * 4); };
     for (int k = 0; k < 3; k++) { D(d.x[k]); D(d.v[k]); D(d.a[k]); D(d.j[k]); D(d.px[k]); D(d.pv[k]); D(d.na[k]); D(d.nj[k]); }
     D(d.m); D(d.npot);
+    E->aos = reinterpret_cast<double *>(q);
+    q += 6 * al(P * 8);
     for (int k = 0; k < 3; k++) { F(d.hx[k]); F(d.lx[k]); F(d.fv[k]); }
     F(d.fm);
     d.pc = reinterpret_cast<int *>(q); q += al(P * 4);
@@ -1292,6 +1307,7 @@ G6C_API void *g6c_create(int nc, const int counts[], const double m[], const dou
         const int zero8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         ok &= hipMemcpy(d.ctl, zero8, sizeof(zero8), hipMemcpyHostToDevice) == hipSuccess;
     }
+    ok = ok && hipHostMalloc(reinterpret_cast<void **>(&E->h_active), sizeof(int)) == hipSuccess;
     ok = ok && pair_setup(E, cus);
     if (!ok || build_items(E)) {
         release(E);
@@ -1331,15 +1347,11 @@ G6C_API int g6c_start(void *h, double t_end)
 {
     Ensemble *E = static_cast<Ensemble *>(h);
     E->d.t_end = t_end;
-    hipLaunchKernelGGL(kc_set_active_count, dim3(1), dim3(1), 0, E->stream, E->d);
-    // all clusters active for the initial pass
-    std::vector<int> ones(E->d.nc, 1);
-    CK(hipMemcpyAsync(E->d.active, ones.data(), sizeof(int) * E->d.nc, hipMemcpyHostToDevice, E->stream));
+    hipLaunchKernelGGL(kc_activate, dim3(1), dim3(kWG), 0, E->stream, E->d);
     if (force_now(E, E->precision, false)) return G6X_ERR_HIP;
     const int pb = (E->d.np + 255) / 256, cb = (E->d.nc + 255) / 256;
     hipLaunchKernelGGL(kc_take_forces, dim3(pb), dim3(256), 0, E->stream, E->d);
     hipLaunchKernelGGL(kc_update, dim3(cb), dim3(256), 0, E->stream, E->d, 1);
-    hipLaunchKernelGGL(kc_set_active_count, dim3(1), dim3(1), 0, E->stream, E->d);
     CK(hipStreamSynchronize(E->stream));
     return invalidate_work_list(E);
 }
@@ -1434,16 +1446,7 @@ G6C_API long long g6c_run(void *h, int steps_per_graph, int use_graph, long long
         E->force_ms += ms;
         return r;
     }
-    // the active count, read back after each launch (pinned, freed on return)
-    struct Pinned {
-        int *p = nullptr;
-        ~Pinned()
-        {
-            if (p) (void)hipHostFree(p);
-        }
-    } pin;
-    CK(hipHostMalloc(reinterpret_cast<void **>(&pin.p), sizeof(int)));
-    int *h_active = pin.p;
+    int *h_active = E->h_active;
     std::vector<int> flags(E->d.nc);
     long long rounds = 0;
     (void)hipEventRecord(ev.a, E->stream);
@@ -1510,14 +1513,15 @@ G6C_API int g6c_state(void *h, double xo[][3], double vo[][3], double t[], int n
     double *x = &xo[0][0];
     double *v = &vo[0][0];
     Ensemble *E = static_cast<Ensemble *>(h);
+    // laid out on the device: one copy each instead of three and a pass over
+    // the host's arrays
     const size_t P = size_t(E->d.np);
-    std::vector<double> buf(P);
-    for (int k = 0; k < 3; k++) {
-        CK(hipMemcpy(buf.data(), E->d.x[k], P * 8, hipMemcpyDeviceToHost));
-        for (size_t p = 0; p < P; p++) x[3 * p + k] = buf[p];
-        CK(hipMemcpy(buf.data(), E->d.v[k], P * 8, hipMemcpyDeviceToHost));
-        for (size_t p = 0; p < P; p++) v[3 * p + k] = buf[p];
-    }
+    double *dx = E->aos, *dv = E->aos + 3 * P;
+    hipLaunchKernelGGL(kc_state, dim3((E->d.np + 255) / 256), dim3(256), 0, E->stream, E->d, dx, dv);
+    CK(hipGetLastError());
+    CK(hipMemcpyAsync(x, dx, 3 * P * 8, hipMemcpyDeviceToHost, E->stream));
+    CK(hipMemcpyAsync(v, dv, 3 * P * 8, hipMemcpyDeviceToHost, E->stream));
+    CK(hipStreamSynchronize(E->stream));
     if (t) CK(hipMemcpy(t, E->d.t, sizeof(double) * E->d.nc, hipMemcpyDeviceToHost));
     if (nsteps) CK(hipMemcpy(nsteps, E->d.nsteps, sizeof(int) * E->d.nc, hipMemcpyDeviceToHost));
     return 0;
