@@ -25,11 +25,11 @@
 // minimum over the particles not in the block), force, and correction (the
 // fold of the force partials, the corrector, the new t + dt into the next
 // minimum); the control-block protocol is described with g6k::StepCtl.
-// g6d_run captures `steps_per_graph` of them (rounded up to even: the step
-// parity is a launch argument) into a hipGraph and replays it, reading the
-// control block (done flag, counters) back after each replay.  Kernels of a
-// finished run return at once, so a replay takes no step after the end
-// condition (system time >= t_end, or the block budget spent).
+// g6d_run captures up to kChunk of them (an even number: the step parity is
+// a launch argument) into a hipGraph and replays it, two replays queued at a
+// time, reading the control block (done flag, counters) back after each.
+// Kernels of a finished run return at once, so a replay takes no step after
+// the end condition (system time >= t_end, or the block budget spent).
 #include "../../include/g6x.h"
 #include "g6_kernels.h"
 #include "g6_predict.h"
@@ -64,7 +64,8 @@ struct Driver {
     long long part_entries = 0;
     void *state_base = nullptr;
     StepCtl *ctl = nullptr;    // device
-    StepCtl *h_ctl = nullptr;  // pinned host mirror
+    StepCtl *h_ctl = nullptr;  // pinned host mirrors, one per queued replay
+    hipEvent_t copied[2] = {};  // mirror k is filled
     hipStream_t stream = nullptr;
     hipGraphExec_t graph = nullptr;
     int graph_steps = 0, graph_prec = -1;
@@ -398,6 +399,10 @@ __global__ void kb_arm(StepCtl *c, double t_end, long long budget)
 // host side
 // ---------------------------------------------------------------------------
 constexpr int kGrid = 1024;  // workgroups of the per-particle kernels
+// Steps of a captured replay: on average kChunk / 2 + kChunk empty steps follow
+// the end of a run (N = 50021, whose intervals are 8 steps: 1.78 ms with replays
+// of 64, one at a time, 1.57 with 4 or 8 and 1.62 with 16, two queued).
+constexpr int kChunk = 8;
 
 int enqueue_step(Driver *D, int par, int sync = 0)
 {
@@ -450,6 +455,8 @@ void release(Driver *D)
     if (D->part) (void)hipFree(D->part);
     if (D->ctl) (void)hipFree(D->ctl);
     if (D->h_ctl) (void)hipHostFree(D->h_ctl);
+    for (hipEvent_t e : D->copied)
+        if (e) (void)hipEventDestroy(e);
     if (D->stream) (void)hipStreamDestroy(D->stream);
     delete D;
 }
@@ -499,7 +506,8 @@ int setup(Driver *D, int n, const int *ids, const double *m, const double *x, co
     DCK(hipMalloc(reinterpret_cast<void **>(&D->part),
                   sizeof(double) * g6k::kPartFieldsD * size_t(D->part_entries)));
     DCK(hipMalloc(reinterpret_cast<void **>(&D->ctl), sizeof(StepCtl)));
-    DCK(hipHostMalloc(reinterpret_cast<void **>(&D->h_ctl), sizeof(StepCtl)));
+    DCK(hipHostMalloc(reinterpret_cast<void **>(&D->h_ctl), 2 * sizeof(StepCtl)));
+    for (hipEvent_t &e : D->copied) DCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     // host state in, times zero
     std::vector<double> zeros(nd, 0.0), tmp(nd);
     DCK(hipMemcpyAsync(s.id, ids, nd * 4, hipMemcpyHostToDevice, D->stream));
@@ -573,7 +581,10 @@ int commit(Driver *D)
 
 int capture(Driver *D, int steps)
 {
-    if (D->graph) (void)hipGraphExecDestroy(D->graph);
+    if (D->graph) {
+        (void)hipStreamSynchronize(D->stream);  // a replay of a finished run may be queued
+        (void)hipGraphExecDestroy(D->graph);
+    }
     D->graph = nullptr;
     hipGraph_t g;
     DCK(hipStreamBeginCapture(D->stream, hipStreamCaptureModeThreadLocal));
@@ -635,28 +646,37 @@ G6D_API long long g6d_run(void *h, double t_end, long long max_blocks, int steps
     // an even number of steps per graph: a replay starts at parity 0
     if (steps_per_graph < 2) steps_per_graph = 2;
     steps_per_graph += steps_per_graph & 1;
+    steps_per_graph = std::min(steps_per_graph, g6b::kChunk);
     if (!D->graph || D->graph_steps != steps_per_graph || D->graph_prec != D->prec)
         if (g6b::capture(D, steps_per_graph)) return G6X_ERR_HIP;
     if (g6b::read_ctl(D)) return G6X_ERR_HIP;
     const long long b0 = D->h_ctl->blocks;
     hipLaunchKernelGGL(g6b::kb_arm, dim3(1), dim3(1), 0, D->stream, D->ctl, t_end,
                        max_blocks > 0 ? max_blocks : -1);
-    for (long long rounds = 0;; rounds++) {
+    auto replay = [&](int k) {
         hipError_t e = hipGraphLaunch(D->graph, D->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(D->h_ctl, D->ctl, sizeof(g6k::StepCtl),
+        if (e == hipSuccess) e = hipMemcpyAsync(D->h_ctl + k, D->ctl, sizeof(g6k::StepCtl),
                                                 hipMemcpyDeviceToHost, D->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(D->stream);
-        if (e != hipSuccess) {
-            D->err = std::string("block steps: ") + hipGetErrorString(e);
-            return G6X_ERR_HIP;
-        }
-        if (D->h_ctl->done) break;
-        // a run of the graph takes at least one step unless done, so this
-        // bound is never reached; it keeps the loop finite regardless
-        if (rounds > (1ll << 40)) break;
+        if (e == hipSuccess) e = hipEventRecord(D->copied[k], D->stream);
+        return e;
+    };
+    // a replay ahead of the one waited for, so the GPU never waits for the host
+    hipError_t e = replay(0);
+    int k = 0;
+    for (long long rounds = 0; e == hipSuccess; rounds++) {
+        e = replay(k ^ 1);
+        if (e == hipSuccess) e = hipEventSynchronize(D->copied[k]);
+        // a replay takes at least one step unless done, so the bound is never
+        // reached; it keeps the loop finite regardless
+        if (e != hipSuccess || D->h_ctl[k].done || rounds > (1ll << 40)) break;
+        k ^= 1;
     }
-    if (reached) *reached = D->h_ctl->done == 1;
-    return D->h_ctl->blocks - b0;
+    if (e != hipSuccess) {
+        D->err = std::string("block steps: ") + hipGetErrorString(e);
+        return G6X_ERR_HIP;
+    }
+    if (reached) *reached = D->h_ctl[k].done == 1;
+    return D->h_ctl[k].blocks - b0;
 }
 
 // Every particle behind the system time takes one step to it (ph4's
