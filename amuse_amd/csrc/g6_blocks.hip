@@ -25,6 +25,9 @@
 // minimum over the particles not in the block), force, and correction (the
 // fold of the force partials, the corrector, the new t + dt into the next
 // minimum); the control-block protocol is described with g6k::StepCtl.
+// Systems of up to g6k::kSmallN particles take the run's steps as one kernel
+// each instead (g6k::SmallSteps), on a copy of the state that is laid out
+// when the run starts and written back when it ends.
 // g6d_run captures up to kChunk of them (an even number: the step parity is
 // a launch argument) into a hipGraph and replays it, two replays queued at a
 // time, reading the control block (done flag, counters) back after each.
@@ -62,6 +65,7 @@ struct Driver {
     IBlock ib;
     double *part = nullptr;
     long long part_entries = 0;
+    g6k::SmallSteps small;     // n = 0: the system is larger
     void *state_base = nullptr;
     StepCtl *ctl = nullptr;    // device
     StepCtl *h_ctl = nullptr;  // pinned host mirrors, one per queued replay
@@ -380,6 +384,69 @@ __global__ void __launch_bounds__(256) kb_state(State s, const StepCtl *c, int j
     }
 }
 
+// A run by small steps: the state and the control block to its buffers 0...
+__global__ void __launch_bounds__(256) kb_small_load(State s, JStore js, const StepCtl *c,
+                                                     g6k::SmallSteps sm, double t_end,
+                                                     long long budget)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j == 0) {
+        g6k::StepCtl o = *c;
+        o.t_end = t_end;
+        o.budget = budget;
+        o.done = 0;
+        o.cur = 0;
+        sm.ctl[0] = o;
+    }
+    if (j >= s.n) return;
+    const size_t n = size_t(s.n);
+    double *f = sm.state + j;
+    f[g6k::kSmT * n] = s.t[j];
+    f[g6k::kSmDt * n] = s.dt[j];
+    f[g6k::kSmPot * n] = s.pot[j];
+    bool loaded = false;  // the j-store holds acc and jerk (else zeros: load_j)
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        f[(g6k::kSmX + k) * n] = s.x[k][j];
+        f[(g6k::kSmV + k) * n] = s.v[k][j];
+        f[(g6k::kSmA + k) * n] = s.a[k][j];
+        f[(g6k::kSmJ + k) * n] = s.j[k][j];
+        loaded |= js.a2[k][j] != 0.0 || js.j6[k][j] != 0.0;
+    }
+    f[g6k::kSmLoaded * n] = loaded ? 1.0 : 0.0;
+}
+
+// ... and back, the j-store of the particles that have stepped too.
+__global__ void __launch_bounds__(256) kb_small_store(State s, JStore js, StepCtl *c,
+                                                      g6k::SmallSteps sm)
+{
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    const StepCtl &o = sm.ctl[0];
+    if (j == 0) {
+        c->done = o.done;
+        c->blocks = o.blocks;
+        c->psteps = o.psteps;
+        c->budget = o.budget;
+        c->t_end = o.t_end;
+        c->system_time = o.system_time;
+        c->tnext = o.tnext;
+    }
+    if (j >= s.n) return;
+    const size_t n = size_t(s.n);
+    const double *f = sm.state + size_t(o.cur) * g6k::kSmallFields * n + j;
+    s.t[j] = f[g6k::kSmT * n];
+    s.dt[j] = f[g6k::kSmDt * n];
+    s.pot[j] = f[g6k::kSmPot * n];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        s.x[k][j] = f[(g6k::kSmX + k) * n];
+        s.v[k][j] = f[(g6k::kSmV + k) * n];
+        s.a[k][j] = f[(g6k::kSmA + k) * n];
+        s.j[k][j] = f[(g6k::kSmJ + k) * n];
+    }
+    if (f[g6k::kSmLoaded * n] != 0.0) load_j(s, js, j, 0);
+}
+
 // Arms a run: end time and block budget; the pending block time moves to
 // slot 0, where the captured sequence (which starts at parity 0) reads it.
 __global__ void kb_arm(StepCtl *c, double t_end, long long budget)
@@ -468,7 +535,11 @@ int setup(Driver *D, int n, const int *ids, const double *m, const double *x, co
     // array starting on a 256-byte boundary (up to 255 bytes of padding
     // after each of the 18)
     const size_t nd = size_t(n);
-    const size_t bytes = nd * sizeof(double) * 16 + nd * sizeof(int) * 2 + 19 * 256;
+    // and, for small systems, the two buffers of their steps
+    const bool small = n <= g6k::kSmallN;
+    const size_t sm_bytes = small ? 2 * g6k::kSmallFields * nd * sizeof(double) : 0;
+    const size_t bytes = nd * sizeof(double) * 16 + nd * sizeof(int) * 2 + sm_bytes +
+                         2 * sizeof(StepCtl) + 21 * 256;
     DCK(hipMalloc(&D->state_base, bytes));
     char *p = static_cast<char *>(D->state_base);
     auto take = [&](size_t b) {
@@ -488,6 +559,10 @@ int setup(Driver *D, int n, const int *ids, const double *m, const double *x, co
     for (int k = 0; k < 3; k++) s.j[k] = reinterpret_cast<double *>(take(nd * 8));
     s.id = reinterpret_cast<int *>(take(nd * 4));
     s.list = reinterpret_cast<int *>(take(nd * 4));
+    if (small) {
+        D->small.state = reinterpret_cast<double *>(take(sm_bytes));
+        D->small.ctl = reinterpret_cast<StepCtl *>(take(2 * sizeof(StepCtl)));
+    }
     if (size_t(p - static_cast<char *>(D->state_base)) > bytes) {
         D->err = "state layout";
         return G6X_ERR_HIP;
@@ -501,6 +576,16 @@ int setup(Driver *D, int n, const int *ids, const double *m, const double *x, co
     DCK(g6k::launch_reset(D->js, 0, jcap, D->stream));
     DCK(hipMalloc(&ibase, g6k::iblock_bytes(jcap)));
     g6k::iblock_carve(D->ib, ibase, jcap);
+    if (small) {
+        D->small.n = n;
+        D->small.id = s.id;
+        D->small.pid = D->js.pid;
+        D->small.pm = D->js.pm;
+        D->small.fm = D->js.fm;
+        D->small.eps2 = D->eps2;
+        D->small.eta = D->eta;
+        D->small.compat = D->compat;
+    }
     const long long max_chunks = std::max(1, nblk(n, g6k::kTJ));
     D->part_entries = std::min(g6k::kStepPartBudget, max_chunks * (long long)n);
     DCK(hipMalloc(reinterpret_cast<void **>(&D->part),
@@ -589,7 +674,8 @@ int capture(Driver *D, int steps)
     hipGraph_t g;
     DCK(hipStreamBeginCapture(D->stream, hipStreamCaptureModeThreadLocal));
     for (int k = 0; k < steps; k++)
-        if (enqueue_step(D, k & 1)) {
+        if (D->small.n ? g6k::launch_small_step(D->small, D->prec, k & 1, D->stream) != hipSuccess
+                       : enqueue_step(D, k & 1)) {
             (void)hipStreamEndCapture(D->stream, &g);
             return G6X_ERR_HIP;
         }
@@ -651,12 +737,17 @@ G6D_API long long g6d_run(void *h, double t_end, long long max_blocks, int steps
         if (g6b::capture(D, steps_per_graph)) return G6X_ERR_HIP;
     if (g6b::read_ctl(D)) return G6X_ERR_HIP;
     const long long b0 = D->h_ctl->blocks;
-    hipLaunchKernelGGL(g6b::kb_arm, dim3(1), dim3(1), 0, D->stream, D->ctl, t_end,
-                       max_blocks > 0 ? max_blocks : -1);
+    const long long budget = max_blocks > 0 ? max_blocks : -1;
+    const bool small = D->small.n > 0;
+    if (small)
+        hipLaunchKernelGGL(g6b::kb_small_load, dim3(g6b::nblk(D->st.n, 256)), dim3(256), 0, D->stream,
+                           D->st, D->js, D->ctl, D->small, t_end, budget);
+    else
+        hipLaunchKernelGGL(g6b::kb_arm, dim3(1), dim3(1), 0, D->stream, D->ctl, t_end, budget);
     auto replay = [&](int k) {
         hipError_t e = hipGraphLaunch(D->graph, D->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(D->h_ctl + k, D->ctl, sizeof(g6k::StepCtl),
-                                                hipMemcpyDeviceToHost, D->stream);
+        if (e == hipSuccess) e = hipMemcpyAsync(D->h_ctl + k, small ? D->small.ctl : D->ctl,
+                                                sizeof(g6k::StepCtl), hipMemcpyDeviceToHost, D->stream);
         if (e == hipSuccess) e = hipEventRecord(D->copied[k], D->stream);
         return e;
     };
@@ -670,6 +761,11 @@ G6D_API long long g6d_run(void *h, double t_end, long long max_blocks, int steps
         // reached; it keeps the loop finite regardless
         if (e != hipSuccess || D->h_ctl[k].done || rounds > (1ll << 40)) break;
         k ^= 1;
+    }
+    if (e == hipSuccess && small) {
+        hipLaunchKernelGGL(g6b::kb_small_store, dim3(g6b::nblk(D->st.n, 256)), dim3(256), 0, D->stream,
+                           D->st, D->js, D->ctl, D->small);
+        e = hipGetLastError();
     }
     if (e != hipSuccess) {
         D->err = std::string("block steps: ") + hipGetErrorString(e);

@@ -204,6 +204,27 @@ hipError_t launch_step_force(const JStore &s, const IBlock &b, double *part, int
                              double eps2, int prec, StepCtl *c, int ni_slot, int tmin_slot,
                              bool with_reduce, hipStream_t st);
 
+// Block steps of a small system, one kernel each.  The state (kSmallFields
+// values per particle, [field][n]) and the control block are kept twice: a
+// step reads buffer ctl[par].cur and ctl[par], writes the other buffer whole
+// and ctl[par ^ 1], so no workgroup reads what another one writes and the end
+// of the kernel is the only synchronisation.  Of StepCtl the fields done,
+// blocks, psteps, budget, t_end, system_time and tnext are used, and cur.
+enum SmallField { kSmT, kSmDt, kSmX, kSmV = kSmX + 3, kSmA = kSmV + 3, kSmJ = kSmA + 3,
+                  kSmPot = kSmJ + 3, kSmLoaded, kSmallFields };
+constexpr int kSmallN = 2048;  // particles: as many predicted ones as a CU's LDS holds
+struct SmallSteps {
+    int n = 0;
+    double *state = nullptr;  // [2][kSmallFields][n]
+    StepCtl *ctl = nullptr;   // [2]
+    const int *id = nullptr, *pid = nullptr;  // ids, and those of the force (-1: empty)
+    const double *pm = nullptr;
+    const float *fm = nullptr;
+    double eps2 = 0.0, eta = 0.0;
+    int compat = 0;
+};
+hipError_t launch_small_step(const SmallSteps &s, int prec, int par, hipStream_t st);
+
 size_t jstore_bytes(int cap);
 void jstore_carve(JStore &s, void *base, int cap);
 size_t iblock_bytes(int cap);

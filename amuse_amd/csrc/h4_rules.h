@@ -32,6 +32,14 @@ namespace h4 {
 // block times advancing and commensurate (all steps are powers of two).
 constexpr double kStepFloor = 0x1p-40;
 
+// Whether the power of two `step` divides t exactly: fmod(t, step) == 0,
+// without fmod's loop (the quotient is exact).
+H4_HD inline bool divides(double step, double t)
+{
+    const double q = t / step;
+    return q == std::trunc(q);
+}
+
 H4_HD inline void predict_ph4(const double *x, const double *v, const double *a,
                               const double *j, double dt, double *xp, double *vp)
 {
@@ -74,13 +82,13 @@ H4_HD inline double correct_ph4(double tnext, double t_old, double step_old, dou
     int e;
     double old2 = step_old / (2 * std::frexp(step_old, &e));
     // bounded: tnext is a sum of powers of two no smaller than the steps
-    for (int it = 0; it < 200 && old2 > 0 && std::fmod(tnext, old2) != 0; it++) old2 /= 2;
+    for (int it = 0; it < 200 && old2 > 0 && !divides(old2, tnext); it++) old2 /= 2;
     if (!(newstep > 0)) newstep = old2;  // degenerate derivative sums
     if (newstep < old2) {
         newstep = old2 / 2;
     } else {
         const double t2 = 2 * old2;
-        if (newstep >= t2 && std::fmod(tnext, t2) == 0) newstep = t2;
+        if (newstep >= t2 && divides(t2, tnext)) newstep = t2;
         else newstep = old2;
     }
     if (newstep < kStepFloor) newstep = kStepFloor;

@@ -145,3 +145,70 @@ def test_mixed_energy_error_at_default_eta():
         d.close()
     print("device driver |dE/E| fp64", de[0], "mixed", de[1], flush=True)
     assert de[1] <= 2 * de[0] + 1e-10
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 512, 1024, 1025, 2047, 2048, 2049])
+def test_small_systems(n):
+    """Systems whose steps are one kernel each (up to 2048 particles; 2049
+    takes three), at the edges of the particles per lane, of the workgroups
+    and of the range: block structure as the host driver's, states within the
+    bounds of test_matches_host_driver, in runs cut by a block budget, with the
+    energy and new runs between them; then a synchronisation and a run on."""
+    from amuse_amd.hermite import Hermite4
+    m, x, v = ic.plummer(max(n, 2), 90 + n)
+    m, x, v = m[:n], x[:n], v[:n]
+    print_case(f"small steps N={n}")
+    h = Hermite4(precision=0)
+    h.commit(m, x, v, eps2=1e-4, eta=0.02)
+    d = driver()
+    d.commit(m, x, v, eps2=1e-4, eta=0.02)
+
+    def same():
+        ch, cd = h.counters(), d.counters()
+        assert ch["block_steps"] == cd["block_steps"]
+        assert ch["particle_steps"] == cd["particle_steps"]
+        assert h.time == cd["system_time"]
+        for a, b in zip(h.timesteps(), d.timesteps()):
+            assert np.array_equal(a, b)
+        for a, b, tol in zip(h.state(), d.state(), (1e-12, 1e-11)):
+            assert np.abs(a - b).max() < tol
+
+    for blocks in (1, 2, 5):
+        d.steps(blocks)
+        assert d.counters()["system_time"] > 0
+    h.evolve(d.counters()["system_time"])
+    same()
+    k0, u0 = d.energy()
+    for t in (1 / 256, 1 / 128):
+        h.evolve(t)
+        d.evolve(t)
+        same()
+    d.synchronize()
+    assert (d.timesteps()[0] == d.time).all()
+    d.evolve(1 / 64)
+    k1, u1 = d.energy()
+    assert abs((k1 + u1) - (k0 + u0)) <= 1e-6 * abs(k0 + u0) + 1e-300
+    h.close()
+    d.close()
+
+
+@pytest.mark.parametrize("n", [300, 1024, 2048])
+def test_small_systems_mixed(n):
+    """Mixed small steps: a run in pieces ends bit for bit where one run ends,
+    and at the default eta conserves energy as the FP64 driver does (the bound
+    of test_mixed_energy_error_at_default_eta)."""
+    m, x, v = ic.plummer(n, 40 + n)
+    runs, de = [], {}
+    for prec, pieces in ((1, (0.25,)), (1, (0.0625, 0.125, 0.25)), (0, (0.25,))):
+        print_case(f"small steps mixed N={n} prec={prec} {pieces}")
+        d = driver(prec)
+        d.commit(m, x, v, eps2=1e-4, eta=0.14)
+        e0 = sum(d.energy())
+        for t in pieces:
+            assert d.evolve(t)
+        runs.append((*d.state(), *d.timesteps()))
+        de[prec] = abs((sum(d.energy()) - e0) / e0)
+        d.close()
+    for a, b in zip(runs[0], runs[1]):
+        assert np.array_equal(a, b)
+    assert de[1] <= 2 * de[0] + 1e-7
