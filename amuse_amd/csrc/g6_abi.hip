@@ -91,6 +91,16 @@ struct Unit {
     JRecord *d_stage = nullptr;
     size_t d_stage_cap = 0;
     hipEvent_t ev_stage = nullptr;
+    // A g6x_set_j_particles call with rising addresses, waiting for the next
+    // flush (before `stage`): its arrays one after the other in pinned memory
+    // and, beyond kDirectRows records, on their way to the device.
+    int cols = 0;  // records
+    bool cols_k18 = false;
+    double *h_cols = nullptr;
+    double *d_hcols = nullptr;  // the device's address of h_cols
+    double *d_cols = nullptr;
+    size_t h_cols_cap = 0, d_cols_cap = 0;  // values
+    size_t flushed_max = 0;  // records of the largest flush that could allocate
 
     // pinned mirrors of the device i-block rows (same row pitch): [8][cap]
     // x y z vx vy vz h2 id and [8][cap] acc3 jerk3 pot nn; id and nn are
@@ -347,8 +357,48 @@ int ensure_partials(int nchunk, int ni)
 // may_allocate = false (the allocation-free entry point): pending records
 // that do not fit the staging buffers already there are an error, and
 // without the staging event the stream is synchronised instead of recorded.
-int flush_stage(bool may_allocate = true)
+bool pred_current(double t);
+
+// The columns of a g6x_set_j_particles call to the store.  predict: the caller
+// needs the store predicted to U.ti next; if the columns set every slot that
+// is done along with them (30000 slots: a 9 us kernel less).
+int flush_columns(bool may_allocate, bool predict)
 {
+    const int n = U.cols;
+    if (n == 0) return 0;
+    // (the allocation-free call takes what the staging buffers of a flush
+    // before it could hold)
+    if (!may_allocate && size_t(n) > U.flushed_max)
+        return fail(G6X_ERR_NOMEM, "pending set_j_particle records exceed the staging buffers "
+                                   "(the allocation-free call cannot grow them)");
+    const bool pv = U.pred_valid && U.pred_prec == U.prec && U.pred_compat == U.compat;
+    const bool all = predict && n == U.nj_hw && !pred_current(U.ti);
+    HIPCHK(g6k::launch_scatter_columns(U.js, n > kDirectRows ? U.d_cols : U.d_hcols, n, U.cols_k18,
+                                       U.prec, pv || all, all ? U.ti : U.pred_ti, U.compat, U.stream),
+           "scatter");
+    U.cols = 0;
+    if (all) {
+        U.pred_valid = true;
+        U.pred_ti = U.ti;
+        U.pred_prec = U.prec;
+        U.pred_compat = U.compat;
+    } else if (!pv) {
+        U.pred_valid = false;
+    }
+    if (!U.ev_stage && !may_allocate) {
+        HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
+    } else {
+        if (!U.ev_stage) HIPCHK(hipEventCreateWithFlags(&U.ev_stage, hipEventDisableTiming), "event");
+        HIPCHK(hipEventRecord(U.ev_stage, U.stream), "stage record");
+    }
+    if (may_allocate) U.flushed_max = std::max(U.flushed_max, std::max(size_t(n), size_t(4096)));
+    return 0;
+}
+
+int flush_stage(bool may_allocate = true, bool predict = false)
+{
+    const int rc = flush_columns(may_allocate, predict);
+    if (rc) return rc;
     const size_t n = U.stage.size();
     if (n == 0) return 0;
     if (!may_allocate && (n > U.h_stage_cap || (n > size_t(kDirectRows) && n > U.d_stage_cap)))
@@ -389,6 +439,7 @@ int flush_stage(bool may_allocate = true)
     }
     for (const auto &r : U.stage) U.stage_pos[r.addr] = -1;
     U.stage.clear();
+    if (may_allocate) U.flushed_max = std::max(U.flushed_max, std::max(n, size_t(4096)));
     if (!pv) U.pred_valid = false;
     return 0;
 }
@@ -635,6 +686,9 @@ int do_open(int cluster)
         if (U.ib.base) (void)hipFree(U.ib.base);
         if (U.ib.part_base) (void)hipFree(U.ib.part_base);
         if (U.d_stage) (void)hipFree(U.d_stage);
+        if (U.d_cols) (void)hipFree(U.d_cols);
+        U.d_cols = nullptr;
+        U.d_cols_cap = 0;
         if (U.sp_base) (void)hipFree(U.sp_base);
         if (U.sp_rows) (void)hipFree(U.sp_rows);
         if (U.sp_buf.base) (void)hipFree(U.sp_buf.base);
@@ -674,6 +728,7 @@ int do_open(int cluster)
     if (rc) return rc;
     HIPCHK(g6k::launch_reset(U.js, 0, U.js.cap, U.stream), "reset");
     HIPCHK(hipStreamSynchronize(U.stream), "open sync");
+    U.cols = 0;
     U.stage.clear();
     std::fill(U.stage_pos.begin(), U.stage_pos.end(), -1);
     clear_ids();
@@ -734,7 +789,7 @@ int do_firsthalf(int nj, int ni, const int *index, const double (*xi)[3], const 
     if (nj > U.nj_hw) U.nj_hw = nj;  // slots never written are empty (id -1)
     rc = grow_iblock(std::max(ni, 1));
     if (rc) return rc;
-    rc = flush_stage();
+    rc = flush_stage(true, true);
     if (rc) return rc;
     const ForceCfg cfg = choose_cfg(std::max(ni, 1), std::max(nj, 1));
     // a short j-range's force kernel predicts the j-slots as it loads them
@@ -893,6 +948,7 @@ G6_API int g6_reset_(int *)
 {
     int rc = check_open();
     if (rc) return rc;
+    U.cols = 0;
     U.stage.clear();
     std::fill(U.stage_pos.begin(), U.stage_pos.end(), -1);
     clear_ids();
@@ -1227,7 +1283,7 @@ G6_API int g6x_calc_self(int nj, int i0, int ni, double eps2, int want_nn)
     if ((long long)i0 + ni > U.js.cap) return fail(G6X_ERR_ARG, "i-range beyond j-store");
     rc = grow_iblock(std::max(ni, 1));
     if (rc) return rc;
-    rc = flush_stage();
+    rc = flush_stage(true, true);
     if (rc) return rc;
     rc = ensure_predicted(U.ti);
     if (rc) return rc;
@@ -1273,7 +1329,7 @@ G6_API int g6x_calc_self_noalloc(int nj, int i0, int ni, double eps2, double acc
     if (rc) return rc;
     double *base = scratch_ptr[U.device];
     if (nj > U.nj_hw) U.nj_hw = nj;
-    rc = flush_stage(false);
+    rc = flush_stage(false, true);
     if (rc) return rc;
     rc = ensure_predicted(U.ti, false);
     if (rc) return rc;
@@ -1364,12 +1420,98 @@ G6_API int g6x_set_tiles(int njs, int ipl, int nchunk, int smem)
     return 0;
 }
 
+// The records of a call whose addresses rise, array by array to pinned memory
+// (taken = false: left to do_set_j).  Host-bound: record by record through the
+// staging vector and from there to pinned memory the host took 30 ns each
+// (N = 262144 8.7 ms of a full pass), by columns about half, and the copy to the device
+// is under way meanwhile.
+static int set_columns(int n, const int *address, const int *index, const double *tj,
+                       const double *dtj, const double *mass, const double (*k18)[3],
+                       const double (*j6)[3], const double (*a2)[3], const double (*v)[3],
+                       const double (*x)[3], bool &taken)
+{
+    if (n < 64 || !U.open || address[0] < 0 || address[n - 1] >= kMaxSlots) return 0;
+    bool rising = true;
+    for (int q = 1; q < n; q++) rising &= address[q] > address[q - 1];
+    if (!rising) return 0;
+    int rc = flush_stage();  // records of earlier calls come before these
+    if (rc) return rc;
+    if (address[n - 1] >= U.js.cap) {
+        rc = grow_jstore(address[n - 1] + 1);
+        if (rc) return rc;
+    }
+    const size_t N = size_t(n);
+    bool any18 = false;
+    for (size_t q = 0; q < N; q++)
+        any18 |= (k18[q][0] != 0.0) | (k18[q][1] != 0.0) | (k18[q][2] != 0.0);
+    const size_t values = N * (any18 ? g6k::kColumnRowK18 : g6k::kColumnRow);
+    if (U.ev_stage) HIPCHK(hipEventSynchronize(U.ev_stage), "stage event");
+    if (values > U.h_cols_cap) {
+        HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
+        if (U.h_cols) (void)hipHostFree(U.h_cols);
+        U.h_cols = nullptr;
+        U.h_cols_cap = 0;
+        const size_t cap = std::max<size_t>(values, 4096 * g6k::kColumnRowK18);
+        hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&U.h_cols), sizeof(double) * cap);
+        if (e != hipSuccess) { U.h_cols = nullptr; return fail(G6X_ERR_NOMEM, "hipHostMalloc stage", e); }
+        U.h_cols_cap = cap;
+        HIPCHK(hipHostGetDevicePointer(reinterpret_cast<void **>(&U.d_hcols), U.h_cols, 0), "stage map");
+    }
+    if (n > kDirectRows && values > U.d_cols_cap) {
+        HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
+        if (U.d_cols) (void)hipFree(U.d_cols);
+        U.d_cols = nullptr;
+        U.d_cols_cap = 0;
+        hipError_t e = hipMalloc(reinterpret_cast<void **>(&U.d_cols), sizeof(double) * values);
+        if (e != hipSuccess) { U.d_cols = nullptr; return fail(G6X_ERR_NOMEM, "hipMalloc stage", e); }
+        U.d_cols_cap = values;
+    }
+    size_t at = 0, sent = 0;
+    auto send = [&]() {
+        const size_t from = sent;
+        sent = at;
+        return n > kDirectRows && at > from
+                   ? hipMemcpyAsync(U.d_cols + from, U.h_cols + from, sizeof(double) * (at - from),
+                                    hipMemcpyHostToDevice, U.stream)
+                   : hipSuccess;
+    };
+    auto put = [&](const void *p, size_t vals) {
+        memcpy(U.h_cols + at, p, sizeof(double) * vals);
+        at += vals;
+    };
+    put(x, 3 * N);
+    put(v, 3 * N);
+    HIPCHK(send(), "stage H2D");
+    put(a2, 3 * N);
+    put(j6, 3 * N);
+    HIPCHK(send(), "stage H2D");
+    put(tj, N);
+    put(dtj, N);
+    put(mass, N);
+    memcpy(U.h_cols + at, address, sizeof(int) * N);
+    memcpy(reinterpret_cast<int *>(U.h_cols + at) + N, index, sizeof(int) * N);
+    at += N;
+    if (any18) put(k18, 3 * N);
+    HIPCHK(send(), "stage H2D");
+    for (int q = 0; q < n; q++)
+        if (U.slot_id[address[q]] != index[q]) note_id(address[q], index[q]);
+    if (any18) U.k18_nonzero = true;
+    U.nj_hw = std::max(U.nj_hw, address[n - 1] + 1);
+    U.cols = n;
+    U.cols_k18 = any18;
+    taken = true;
+    return 0;
+}
+
 G6_API int g6x_set_j_particles(int n, const int address[], const int index[], const double tj[],
                                const double dtj[], const double mass[], const double k18[][3],
                                const double j6[][3], const double a2[][3], const double v[][3],
                                const double x[][3])
 {
     if (n < 0) return fail(G6X_ERR_ARG, "negative count");
+    bool taken = false;
+    const int rc = set_columns(n, address, index, tj, dtj, mass, k18, j6, a2, v, x, taken);
+    if (rc || taken) return rc;
     for (int q = 0; q < n; q++) {
         int rc = do_set_j(address[q], index[q], tj[q], dtj[q], mass[q], k18[q], j6[q], a2[q], v[q],
                           x[q]);

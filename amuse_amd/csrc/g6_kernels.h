@@ -236,6 +236,12 @@ hipError_t launch_copy_store(const JStore &dst, const JStore &src, int n,
 hipError_t launch_scatter(const JStore &s, const JRecord *rec, int n,
                           int prec, int pred_valid, double ti, int compat,
                           hipStream_t st);
+// n records as the caller's arrays lie one after the other at `rec`: x, v, a2,
+// j6 [n][3], tj, dtj, m [n], addresses and ids [n] (ints), k18 [n][3] when
+// has_k18 (else zeros); the addresses differ.  pred: as k_scatter's, to ti.
+constexpr int kColumnRow = 16, kColumnRowK18 = 19;  // FP64 values per record
+hipError_t launch_scatter_columns(const JStore &s, const double *rec, int n, bool has_k18,
+                                  int prec, int pred, double ti, int compat, hipStream_t st);
 hipError_t launch_predict(const JStore &s, int nj, double ti, int prec,
                           int compat, int use_k18, hipStream_t st);
 hipError_t launch_iblock_self(const JStore &s, const IBlock &b, int i0,

@@ -156,6 +156,41 @@ __global__ void __launch_bounds__(256) k_scatter(JStore s, const JRecord *__rest
     }
 }
 
+// k_scatter for records in columns (launch_scatter_columns).  Memory-bound (PCIe
+// where the columns lie in host memory); with pred it takes the predictor
+// kernel's pass along when every slot is set.
+__global__ void __launch_bounds__(256) k_scatter_columns(JStore s, const double *__restrict__ rec,
+                                                         int n, int has_k18, int prec, int pred,
+                                                         double ti, int compat)
+{
+    const int r = blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= n) return;
+    const size_t N = size_t(n);
+    const int *ids = reinterpret_cast<const int *>(rec + 15 * N);
+    const int j = ids[r], id = ids[N + r];
+    double x[3], v[3], a2[3], j6[3], k18[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        x[k] = rec[3 * size_t(r) + k];
+        v[k] = rec[3 * (N + r) + k];
+        a2[k] = rec[3 * (2 * N + r) + k];
+        j6[k] = rec[3 * (3 * N + r) + k];
+        k18[k] = has_k18 ? rec[16 * N + 3 * size_t(r) + k] : 0.0;
+    }
+    const double tj = rec[12 * N + r], m = rec[14 * N + r];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        s.x[k][j] = x[k]; s.v[k][j] = v[k]; s.a2[k][j] = a2[k];
+        s.j6[k][j] = j6[k]; s.k18[k][j] = k18[k];
+    }
+    s.tj[j] = tj; s.dtj[j] = rec[13 * N + r]; s.m[j] = m; s.id[j] = id;
+    const double mp = id == -1 ? 0.0 : m;
+    s.pm[j] = mp;
+    s.fm[j] = float(mp);
+    s.pid[j] = id;
+    if (pred) write_pred(s, j, prec, id, predict_slot(ti, tj, x, v, a2, j6, k18, compat, has_k18 != 0));
+}
+
 // Full predictor pass over slots [0, nj): streams 13 doubles + 1 int in
 // and 6 doubles (plain) or 9 floats (mixed) out per slot; HBM-bound.
 __global__ void __launch_bounds__(256) k_predict(JStore s, int nj, double ti, int prec, int compat,
@@ -1784,6 +1819,15 @@ hipError_t launch_scatter(const JStore &s, const JRecord *rec, int n, int prec, 
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_scatter, dim3(nblocks(n, 256)), dim3(256), 0, st, s, rec, n, prec,
                        pred_valid, ti, compat);
+    return hipGetLastError();
+}
+
+hipError_t launch_scatter_columns(const JStore &s, const double *rec, int n, bool has_k18, int prec,
+                                  int pred, double ti, int compat, hipStream_t st)
+{
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_scatter_columns, dim3(nblocks(n, 256)), dim3(256), 0, st, s, rec, n,
+                       int(has_k18), prec, pred, ti, compat);
     return hipGetLastError();
 }
 

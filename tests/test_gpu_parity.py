@@ -689,3 +689,60 @@ def test_pair_once_full_pass_edges(g6, prec, n):
     finally:
         g6.set_tiles(0, 0)
         g6.set_precision(0)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("n", [63, 64, 65, 2049, 4096, 4097])
+def test_set_j_particles_by_columns(g6, n, prec):
+    """g6x_set_j_particles with rising addresses (array by array, from 64
+    records on; read in place up to 4096) leaves what one g6_set_j_particle
+    per record leaves, bit for bit: a whole store, predicted along with it;
+    a store with gaps; updates of part of it at the same time; snap terms;
+    records before and after it by other calls; a call that does not rise."""
+    rng = np.random.Generator(np.random.PCG64(n))
+    x, v, a2, j6, k18 = (rng.normal(0, 1, (n, 3)) for _ in range(5))
+    m, tj = rng.uniform(0.1, 1, n), 1.0 - rng.integers(0, 5, n) / 256.0
+    zero = np.zeros((n, 3))
+    up = np.arange(n)
+
+    def one_by_one(addr, ids, k, xx):
+        for q in range(n):
+            g6.set_j_particle(addr[q], ids[q], tj[q], 0.0, m[q], k[q], j6[q], a2[q], v[q], xx[q])
+
+    def together(addr, ids, k, xx):
+        g6.set_j_particles(addr, ids, tj, 0.0, m, k, j6, a2, v, xx)
+
+    def forces(nj):
+        g6.calc_self(nj, 0, nj, 1e-4)
+        return g6.fetch(nj)
+
+    def run(put):
+        out = []
+        g6.reset()
+        g6.set_precision(prec)
+        put(up, up + 1, zero, x)                      # every slot
+        g6.set_ti(1.0)
+        out += forces(n)
+        sel = np.sort(rng2.choice(n, n // 2, replace=False))
+        for q in sel[:3]:                             # singles before it ...
+            g6.set_j_particle(q, q + 1, tj[q], 0.0, m[q], zero[q], j6[q], a2[q], v[q], x[q] + 1)
+        put(up, up + 1, zero, x + 0.25)               # ... superseded
+        g6.set_j_particle(5, 6, tj[5], 0.0, m[5], zero[5], j6[5], a2[5], v[5], x[5] - 1)
+        out += forces(n)
+        put(2 * up, up + 1, k18, x)                   # gaps (old records), snap
+        out += forces(2 * n - 1)
+        g6.set_ti(1.0 + 1 / 1024)
+        out += forces(2 * n - 1)
+        put(up[::-1], up + 1, zero, x)                # falling
+        out += forces(2 * n - 1)
+        return out
+
+    print_case(f"set_j_particles by columns n={n} prec={prec}")
+    res = []
+    for put in (one_by_one, together):
+        rng2 = np.random.Generator(np.random.PCG64(7))
+        res.append(run(put))
+    g6.reset()
+    g6.set_precision(0)
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
