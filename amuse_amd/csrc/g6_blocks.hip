@@ -42,6 +42,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #define G6D_API extern "C" __attribute__((visibility("default")))
@@ -95,15 +96,22 @@ inline int nblk(int n, int b) { return (n + b - 1) / b; }
 // ---------------------------------------------------------------------------
 constexpr unsigned long long kInfBits = 0x7ff0000000000000ull;  // +inf
 
-// Folds a lane's candidate next block time into *slot: wave shuffles, then
-// one 64-bit atomicMin per wave on the order-preserving bits of the
-// (positive) times.
+// Folds the workgroup's candidates for the next block time into *slot: one
+// 64-bit atomicMin on the order-preserving bits of the (positive) times, and
+// only where it would lower the value.  Every thread takes part.
 __device__ __forceinline__ void fold_min(double lo, unsigned long long *slot)
 {
+    __shared__ double w[4];
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) lo = fmin(lo, __shfl_xor(lo, off));
-    if ((threadIdx.x & 63) == 0 && lo < __builtin_inf())
-        atomicMin(slot, static_cast<unsigned long long>(__double_as_longlong(lo)));
+    if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = lo;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    lo = fmin(fmin(w[0], w[1]), fmin(w[2], w[3]));
+    const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(lo));
+    if (lo < __builtin_inf() &&
+        bits < __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMin(slot, bits);
 }
 
 // Control block for a fresh run of steps: no block time yet, counts zero.
@@ -170,11 +178,16 @@ __global__ void __launch_bounds__(256) kb_select(State s, JStore js, IBlock b, S
             g6k::write_pred(js, j, prec, js.id[j], pr);
         }
         const double tj = s.t[j] + s.dt[j];
-        if (sync ? !(s.t[j] < tnext) : tj != tnext) {
-            lo = fmin(lo, tj);
-            continue;
-        }
-        const int q = atomicAdd(&c->ni[par], 1);
+        const bool in = sync ? s.t[j] < tnext : tj == tnext;
+        // one addition to the count per wave
+        const unsigned long long members = __ballot(in);
+        if (!in) lo = fmin(lo, tj);
+        if (!members) continue;
+        const int lane = threadIdx.x & 63, leader = __ffsll((long long)members) - 1;
+        int q = 0;
+        if (lane == leader) q = atomicAdd(&c->ni[par], __popcll(members));
+        q = __shfl(q, leader) + __popcll(members & ((1ull << lane) - 1));
+        if (!in) continue;
         s.list[q] = j;
         double x[3], v[3], a[3], jk[3], xp[3], vp[3];
 #pragma unroll
@@ -261,66 +274,102 @@ __global__ void __launch_bounds__(256) kb_take_all(State s, IBlock b)
     }
 }
 
-// Corrects particle list[q] with the forces f (acc3 jerk3 pot), reloads it
-// into the j-store and returns its new t + dt.
-__device__ __forceinline__ double correct_one(const State &s, const JStore &js, const IBlock &b,
-                                              int q, double tnext, double eta, const double *f)
+// A block row's particle: the old derivatives, the predicted state, its step.
+struct Row {
+    int j;
+    double oa[3], oj[3], ip[3], iv[3], t, dt;
+};
+
+__device__ __forceinline__ void load_row(const State &s, const IBlock &b, int q, Row &r)
 {
-    const int j = s.list[q];
-    double oa[3], oj[3], ia[3], ij[3], ip[3], iv[3];
+    r.j = s.list[q];
 #pragma unroll
     for (int k = 0; k < 3; k++) {
-        oa[k] = s.a[k][j];
-        oj[k] = s.j[k][j];
-        ia[k] = f[k];
-        ij[k] = f[3 + k];
-        ip[k] = b.x[k][q];
-        iv[k] = b.v[k][q];
+        r.ip[k] = b.x[k][q];
+        r.iv[k] = b.v[k][q];
+        r.oa[k] = s.a[k][r.j];
+        r.oj[k] = s.j[k][r.j];
     }
-    const double newstep = h4::correct_ph4(tnext, s.t[j], s.dt[j], eta, oa, oj, ia, ij, ip, iv);
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        s.x[k][j] = ip[k];
-        s.v[k][j] = iv[k];
-        s.a[k][j] = ia[k];
-        s.j[k][j] = ij[k];
-    }
-    s.pot[j] = f[6];
-    s.t[j] = tnext;
-    s.dt[j] = newstep;
-    load_j(s, js, j, 0);
-    return s.t[j] + s.dt[j];
+    r.t = s.t[r.j];
+    r.dt = s.dt[r.j];
 }
 
-// Forces of block row q folded from the j-chunk partials (the order and
-// arithmetic of the library's reduce kernel: lane form, or lane `lane` of the
-// wave form followed by the butterfly; the result is valid in lane 0).
-template <bool MX>
-__device__ __forceinline__ void fold_forces(const double *part, int nchunk, int ni, int q,
-                                            bool wave, double *f)
+// Corrects it with the forces f (acc3 jerk3 pot), writes it to the state and
+// the j-store (whose mass, ids and k18 stay) and returns its new t + dt.
+__device__ __forceinline__ double correct_row(const State &s, const JStore &js, Row &r,
+                                              double tnext, double eta, const double *f)
 {
-    const int lane = threadIdx.x & 63;
-    const int first = wave ? lane : 0, step = wave ? 64 : 1;
-    int addr;
-    if constexpr (MX) {
-        float h[7], l[7], best;
-        g6k::reduce_i_mx(part, nchunk, ni, q, first, step, h, l, best, addr, 0);
-        if (wave) g6k::butterfly_mx(h, l, best, addr);
+    const int j = r.j;
+    const double step = h4::correct_ph4(tnext, r.t, r.dt, eta, r.oa, r.oj, f, f + 3, r.ip, r.iv);
 #pragma unroll
-        for (int k = 0; k < 7; k++) f[k] = double(h[k]) + double(l[k]);
-    } else {
-        double h[7], l[7], best;
-        g6k::reduce_i_f64(part, nchunk, ni, q, first, step, h, l, best, addr, 0);
-        if (wave) g6k::butterfly_f64(h, l, best, addr);
-#pragma unroll
-        for (int k = 0; k < 7; k++) f[k] = h[k] + l[k];
+    for (int k = 0; k < 3; k++) {
+        s.x[k][j] = js.x[k][j] = r.ip[k];
+        s.v[k][j] = js.v[k][j] = r.iv[k];
+        s.a[k][j] = f[k];
+        s.j[k][j] = f[3 + k];
+        js.a2[k][j] = f[k] / 2;
+        js.j6[k][j] = f[3 + k] / 6;
     }
+    s.pot[j] = f[6];
+    s.t[j] = js.tj[j] = tnext;
+    s.dt[j] = js.dtj[j] = step;
+    return tnext + step;
+}
+
+// Rows whose forces lie in nchunk partial records each: RPW rows per wave, 64 /
+// RPW lanes each (neighbouring rows in neighbouring lanes, whose loads share
+// lines) fold every 64 / RPW-th chunk and meet in a fixed butterfly; the
+// rows' own loads are under way meanwhile.
+template <bool MX, int RPW>
+__device__ __forceinline__ double fold_and_correct(const State &s, const JStore &js,
+                                                   const IBlock &b, const double *part, int nchunk,
+                                                   int ni, double tnext, double eta)
+{
+    using T = std::conditional_t<MX, float, double>;
+    constexpr int G = 64 / RPW;
+    const int lane = threadIdx.x & 63, g = lane / RPW;
+    double lo = __builtin_inf();
+    // the loop bound is wave-uniform
+    for (int q0 = (blockIdx.x * 4 + int(threadIdx.x >> 6)) * RPW; q0 < ni; q0 += gridDim.x * 4 * RPW) {
+        const int q = min(q0 + lane % RPW, ni - 1);
+        Row r;
+        load_row(s, b, q, r);
+        T h[7], l[7], best;
+        int addr;
+        if constexpr (MX)
+            g6k::reduce_i_mx(part, nchunk, ni, q, g, G, h, l, best, addr, 0);
+        else
+            g6k::reduce_i_f64(part, nchunk, ni, q, g, G, h, l, best, addr, 0);
+#pragma unroll
+        for (int off = 32; off >= RPW; off >>= 1) {
+#pragma unroll
+            for (int k = 0; k < 7; k++) {
+                const T oh = __shfl_xor(h[k], off), ol = __shfl_xor(l[k], off);
+                if constexpr (MX)
+                    g6k::two_sum_add(h[k], l[k], oh);
+                else
+                    g6k::two_sum_add_d(h[k], l[k], oh);
+                l[k] += ol;
+            }
+        }
+        if (g == 0 && q0 + lane < ni) {
+            double f[7];
+#pragma unroll
+            for (int k = 0; k < 7; k++) f[k] = double(h[k]) + double(l[k]);
+            lo = fmin(lo, correct_row(s, js, r, tnext, eta, f));
+        }
+    }
+    return lo;
 }
 
 // Step k, parity par: the block's forces (from b.out, or folded here from
 // the partials when the plan split j over workgroups), ph4's corrector, the
 // new t + dt into tmin[par ^ 1]; the first thread advances the counters and
-// clears ni[par ^ 1] for the next step's selection.
+// clears ni[par ^ 1] for the next step's selection.  Latency-bound: enough
+// waves for the chip decide the rows per wave.  us at N = 16384 FP64, the rows
+// loaded after the fold, an atomic per row and a wave per row up to 8192 rows,
+// a lane per row beyond -> now: 10 -> 7.5 for a few rows, 17 -> 14 for hundreds,
+// 40 -> 26 and 85 -> 33 for thousands.
 template <bool MX>
 __global__ void __launch_bounds__(256) kb_correct(State s, JStore js, IBlock b,
                                                   const double *__restrict__ part, StepCtl *c,
@@ -340,23 +389,21 @@ __global__ void __launch_bounds__(256) kb_correct(State s, JStore js, IBlock b,
     }
     const g6k::StepPlan sp = g6k::plan_step(ni, s.n);
     double lo = __builtin_inf();
-    double f[7];
-    if (sp.nchunk > 1 && sp.nchunk >= g6k::kReduceWaveMin && ni <= g6k::kReduceWaveMaxNi) {
-        // one wave per row; the loop bound is wave-uniform
-        for (int q = blockIdx.x * 4 + int(threadIdx.x >> 6); q < ni; q += gridDim.x * 4) {
-            fold_forces<MX>(part, sp.nchunk, ni, q, true, f);
-            if ((threadIdx.x & 63) == 0) lo = fmin(lo, correct_one(s, js, b, q, tnext, eta, f));
-        }
-    } else {
+    if (sp.nchunk <= 1) {
         for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < ni; q += gridDim.x * blockDim.x) {
-            if (sp.nchunk > 1) {
-                fold_forces<MX>(part, sp.nchunk, ni, q, false, f);
-            } else {
+            Row r;
+            load_row(s, b, q, r);
+            double f[7];
 #pragma unroll
-                for (int k = 0; k < 7; k++) f[k] = b.out[k * S + q];
-            }
-            lo = fmin(lo, correct_one(s, js, b, q, tnext, eta, f));
+            for (int k = 0; k < 7; k++) f[k] = b.out[k * S + q];
+            lo = fmin(lo, correct_row(s, js, r, tnext, eta, f));
         }
+    } else if (ni <= 1024) {
+        lo = fold_and_correct<MX, 1>(s, js, b, part, sp.nchunk, ni, tnext, eta);
+    } else if (ni <= 8192) {
+        lo = fold_and_correct<MX, 4>(s, js, b, part, sp.nchunk, ni, tnext, eta);
+    } else {
+        lo = fold_and_correct<MX, 16>(s, js, b, part, sp.nchunk, ni, tnext, eta);
     }
     fold_min(lo, &c->tmin[par ^ 1]);
 }
