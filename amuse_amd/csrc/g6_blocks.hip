@@ -28,9 +28,11 @@
 // Systems of up to g6k::kSmallN particles take the run's steps as one kernel
 // each instead (g6k::SmallSteps), on a copy of the state that is laid out
 // when the run starts and written back when it ends.
-// g6d_run captures up to kChunk of them (an even number: the step parity is
-// a launch argument) into a hipGraph and replays it, two replays queued at a
-// time, reading the control block (done flag, counters) back after each.
+// g6d_run captures up to kChunk steps (an even number: the step parity is a
+// launch argument) into a hipGraph and replays it, two replays queued at a
+// time; a replay's last kernel leaves the control block (done flag, counters)
+// in pinned memory (as a copy between the replays it cost 18 us, more than a
+// step of a small system: N = 1024 interval and state 1.32 -> 0.94 ms).
 // Kernels of a finished run return at once, so a replay takes no step after
 // the end condition (system time >= t_end, or the block budget spent).
 #include "../../include/g6x.h"
@@ -70,7 +72,9 @@ struct Driver {
     void *state_base = nullptr;
     StepCtl *ctl = nullptr;    // device
     StepCtl *h_ctl = nullptr;  // pinned host mirrors, one per queued replay
-    hipEvent_t copied[2] = {};  // mirror k is filled
+    StepCtl *d_hctl = nullptr;  // the device's address of them
+    hipEvent_t filled[2] = {};  // mirror k is filled
+    long long blocks = 0;       // block steps so far (< 0: not known)
     hipStream_t stream = nullptr;
     hipGraphExec_t graph = nullptr;
     int graph_steps = 0, graph_prec = -1;
@@ -365,17 +369,21 @@ __device__ __forceinline__ double fold_and_correct(const State &s, const JStore 
 // Step k, parity par: the block's forces (from b.out, or folded here from
 // the partials when the plan split j over workgroups), ph4's corrector, the
 // new t + dt into tmin[par ^ 1]; the first thread advances the counters and
-// clears ni[par ^ 1] for the next step's selection.  Latency-bound: enough
+// clears ni[par ^ 1] for the next step's selection.  mirror: as of
+// g6k::launch_small_step.  Latency-bound: enough
 // waves for the chip decide the rows per wave.  us at N = 16384 FP64, the rows
 // loaded after the fold, an atomic per row and a wave per row up to 8192 rows,
 // a lane per row beyond -> now: 10 -> 7.5 for a few rows, 17 -> 14 for hundreds,
-// 40 -> 26 and 85 -> 33 for thousands.
+// 40 -> 26 and 85 -> 31 for thousands.
 template <bool MX>
 __global__ void __launch_bounds__(256) kb_correct(State s, JStore js, IBlock b,
                                                   const double *__restrict__ part, StepCtl *c,
-                                                  double eta, int par)
+                                                  double eta, int par, StepCtl *mirror)
 {
-    if (c->done) return;
+    if (c->done) {
+        if (mirror && blockIdx.x == 0 && threadIdx.x == 0) g6k::mirror_ctl(mirror, *c, c);
+        return;
+    }
     const double tnext = c->tnext;
     const int ni = c->ni[par];
     const int S = b.cap;
@@ -386,6 +394,7 @@ __global__ void __launch_bounds__(256) kb_correct(State s, JStore js, IBlock b,
         if (c->budget > 0) c->budget -= 1;
         c->ni[par ^ 1] = 0;
         c->cur = par ^ 1;
+        if (mirror) g6k::mirror_ctl(mirror, *c, c);
     }
     const g6k::StepPlan sp = g6k::plan_step(ni, s.n);
     double lo = __builtin_inf();
@@ -443,6 +452,7 @@ __global__ void __launch_bounds__(256) kb_small_load(State s, JStore js, const S
         o.budget = budget;
         o.done = 0;
         o.cur = 0;
+        o.replays = 0;
         sm.ctl[0] = o;
     }
     if (j >= s.n) return;
@@ -501,6 +511,7 @@ __global__ void kb_arm(StepCtl *c, double t_end, long long budget)
     c->t_end = t_end;
     c->budget = budget;
     c->done = 0;
+    c->replays = 0;
     if (c->cur == 1) {
         c->tmin[0] = c->tmin[1];
         c->tmin[1] = kInfBits;
@@ -518,7 +529,7 @@ constexpr int kGrid = 1024;  // workgroups of the per-particle kernels
 // of 64, one at a time, 1.57 with 4 or 8 and 1.62 with 16, two queued).
 constexpr int kChunk = 8;
 
-int enqueue_step(Driver *D, int par, int sync = 0)
+int enqueue_step(Driver *D, int par, int sync = 0, StepCtl *mirror = nullptr)
 {
     const int n = D->st.n;
     const int g = std::min(nblk(n, 256), kGrid);
@@ -531,10 +542,10 @@ int enqueue_step(Driver *D, int par, int sync = 0)
     const int gc = std::min(g6k::kStepGrid, std::max(g, nblk(n, 4)));
     if (D->prec == G6X_MIXED)
         hipLaunchKernelGGL(kb_correct<true>, dim3(gc), dim3(256), 0, D->stream, D->st, D->js,
-                           D->ib, D->part, D->ctl, D->eta, par);
+                           D->ib, D->part, D->ctl, D->eta, par, mirror);
     else
         hipLaunchKernelGGL(kb_correct<false>, dim3(gc), dim3(256), 0, D->stream, D->st, D->js,
-                           D->ib, D->part, D->ctl, D->eta, par);
+                           D->ib, D->part, D->ctl, D->eta, par, mirror);
     DCK(hipGetLastError());
     return 0;
 }
@@ -569,7 +580,7 @@ void release(Driver *D)
     if (D->part) (void)hipFree(D->part);
     if (D->ctl) (void)hipFree(D->ctl);
     if (D->h_ctl) (void)hipHostFree(D->h_ctl);
-    for (hipEvent_t e : D->copied)
+    for (hipEvent_t e : D->filled)
         if (e) (void)hipEventDestroy(e);
     if (D->stream) (void)hipStreamDestroy(D->stream);
     delete D;
@@ -639,7 +650,8 @@ int setup(Driver *D, int n, const int *ids, const double *m, const double *x, co
                   sizeof(double) * g6k::kPartFieldsD * size_t(D->part_entries)));
     DCK(hipMalloc(reinterpret_cast<void **>(&D->ctl), sizeof(StepCtl)));
     DCK(hipHostMalloc(reinterpret_cast<void **>(&D->h_ctl), 2 * sizeof(StepCtl)));
-    for (hipEvent_t &e : D->copied) DCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    DCK(hipHostGetDevicePointer(reinterpret_cast<void **>(&D->d_hctl), D->h_ctl, 0));
+    for (hipEvent_t &e : D->filled) DCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     // host state in, times zero
     std::vector<double> zeros(nd, 0.0), tmp(nd);
     DCK(hipMemcpyAsync(s.id, ids, nd * 4, hipMemcpyHostToDevice, D->stream));
@@ -720,12 +732,14 @@ int capture(Driver *D, int steps)
     D->graph = nullptr;
     hipGraph_t g;
     DCK(hipStreamBeginCapture(D->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < steps; k++)
-        if (D->small.n ? g6k::launch_small_step(D->small, D->prec, k & 1, D->stream) != hipSuccess
-                       : enqueue_step(D, k & 1)) {
+    for (int k = 0; k < steps; k++) {
+        StepCtl *mirror = k == steps - 1 ? D->d_hctl : nullptr;
+        if (D->small.n ? g6k::launch_small_step(D->small, D->prec, k & 1, mirror, D->stream) != hipSuccess
+                       : enqueue_step(D, k & 1, 0, mirror)) {
             (void)hipStreamEndCapture(D->stream, &g);
             return G6X_ERR_HIP;
         }
+    }
     DCK(hipStreamEndCapture(D->stream, &g));
     DCK(hipGraphInstantiate(&D->graph, g, nullptr, nullptr, 0));
     (void)hipGraphDestroy(g);
@@ -782,8 +796,12 @@ G6D_API long long g6d_run(void *h, double t_end, long long max_blocks, int steps
     steps_per_graph = std::min(steps_per_graph, g6b::kChunk);
     if (!D->graph || D->graph_steps != steps_per_graph || D->graph_prec != D->prec)
         if (g6b::capture(D, steps_per_graph)) return G6X_ERR_HIP;
-    if (g6b::read_ctl(D)) return G6X_ERR_HIP;
-    const long long b0 = D->h_ctl->blocks;
+    if (D->blocks < 0) {
+        if (g6b::read_ctl(D)) return G6X_ERR_HIP;
+        D->blocks = D->h_ctl->blocks;
+    }
+    const long long b0 = D->blocks;
+    D->blocks = -1;
     const long long budget = max_blocks > 0 ? max_blocks : -1;
     const bool small = D->small.n > 0;
     if (small)
@@ -793,9 +811,7 @@ G6D_API long long g6d_run(void *h, double t_end, long long max_blocks, int steps
         hipLaunchKernelGGL(g6b::kb_arm, dim3(1), dim3(1), 0, D->stream, D->ctl, t_end, budget);
     auto replay = [&](int k) {
         hipError_t e = hipGraphLaunch(D->graph, D->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(D->h_ctl + k, small ? D->small.ctl : D->ctl,
-                                                sizeof(g6k::StepCtl), hipMemcpyDeviceToHost, D->stream);
-        if (e == hipSuccess) e = hipEventRecord(D->copied[k], D->stream);
+        if (e == hipSuccess) e = hipEventRecord(D->filled[k], D->stream);
         return e;
     };
     // a replay ahead of the one waited for, so the GPU never waits for the host
@@ -803,7 +819,7 @@ G6D_API long long g6d_run(void *h, double t_end, long long max_blocks, int steps
     int k = 0;
     for (long long rounds = 0; e == hipSuccess; rounds++) {
         e = replay(k ^ 1);
-        if (e == hipSuccess) e = hipEventSynchronize(D->copied[k]);
+        if (e == hipSuccess) e = hipEventSynchronize(D->filled[k]);
         // a replay takes at least one step unless done, so the bound is never
         // reached; it keeps the loop finite regardless
         if (e != hipSuccess || D->h_ctl[k].done || rounds > (1ll << 40)) break;
@@ -819,7 +835,8 @@ G6D_API long long g6d_run(void *h, double t_end, long long max_blocks, int steps
         return G6X_ERR_HIP;
     }
     if (reached) *reached = D->h_ctl[k].done == 1;
-    return D->h_ctl[k].blocks - b0;
+    D->blocks = D->h_ctl[k].blocks;
+    return D->blocks - b0;
 }
 
 // Every particle behind the system time takes one step to it (ph4's
@@ -834,6 +851,7 @@ G6D_API int g6d_synchronize(void *h)
     // the pending block time to slot 0 (parity 0 below), no end time
     hipLaunchKernelGGL(g6b::kb_arm, dim3(1), dim3(1), 0, D->stream, D->ctl,
                        __builtin_inf(), -1ll);
+    D->blocks = -1;
     if (g6b::enqueue_step(D, 0, 1)) return G6X_ERR_HIP;
     if (g6b::read_ctl(D)) return G6X_ERR_HIP;
     return 0;

@@ -110,7 +110,18 @@ struct StepCtl {
     double t_end;
     double system_time;
     double tnext;               // block time of the current step
+    int replays;                // captured replays since the run was armed
 };
+
+// One thread, at the end of a replay's last step: c to the host's mirror of
+// this replay (c0 holds the count).
+__device__ __forceinline__ void mirror_ctl(StepCtl *mirror, const StepCtl &c, StepCtl *c0)
+{
+    const int r = c.replays;
+    c0->replays = r + 1;
+    mirror[r & 1] = c;
+    __threadfence_system();
+}
 
 struct StepPlan {
     int shape;    // 0..3: (lanes per i, i per lane) = (1,2) (4,1) (16,1) (64,1)
@@ -223,7 +234,10 @@ struct SmallSteps {
     double eps2 = 0.0, eta = 0.0;
     int compat = 0;
 };
-hipError_t launch_small_step(const SmallSteps &s, int prec, int par, hipStream_t st);
+// mirror (the last step of a replay; else null): two control blocks in pinned
+// memory, of which the step fills the one of its replay's parity.
+hipError_t launch_small_step(const SmallSteps &s, int prec, int par, StepCtl *mirror,
+                             hipStream_t st);
 
 size_t jstore_bytes(int cap);
 void jstore_carve(JStore &s, void *base, int cap);

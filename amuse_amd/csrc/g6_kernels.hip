@@ -1532,7 +1532,7 @@ struct SmallTile<true> {
 
 // K: particles per lane (n <= 256 K).
 template <bool MX, int K>
-__global__ void __launch_bounds__(kWG) kd_small_step(SmallSteps s, int par)
+__global__ void __launch_bounds__(kWG) kd_small_step(SmallSteps s, int par, StepCtl *mirror)
 {
     extern __shared__ double2 lds[];
     __shared__ double wmin[kWG / 64];
@@ -1546,6 +1546,7 @@ __global__ void __launch_bounds__(kWG) kd_small_step(SmallSteps s, int par)
             // 1: t_end reached, 2: block budget spent
             if (!o.done) o.done = !(c.system_time < c.t_end) ? 1 : 2;
             s.ctl[par ^ 1] = o;
+            if (mirror) mirror_ctl(mirror, o, &s.ctl[par ^ 1]);
         }
         return;
     }
@@ -1607,6 +1608,7 @@ __global__ void __launch_bounds__(kWG) kd_small_step(SmallSteps s, int par)
         if (o.budget > 0) o.budget -= 1;
         o.cur ^= 1;
         s.ctl[par ^ 1] = o;
+        if (mirror) mirror_ctl(mirror, o, &s.ctl[par ^ 1]);
     }
     if (int(blockIdx.x) >= ni) return;
 
@@ -2047,7 +2049,7 @@ hipError_t launch_step_predict(const JStore &s, int nj, const StepCtl *c, int at
 }
 
 template <bool MX, int K>
-hipError_t small_step(const SmallSteps &s, int par, hipStream_t st)
+hipError_t small_step(const SmallSteps &s, int par, StepCtl *mirror, hipStream_t st)
 {
     const size_t lds = SmallTile<MX>::kBytes * K * kWG;
     if (lds > 65536) {
@@ -2059,19 +2061,20 @@ hipError_t small_step(const SmallSteps &s, int par, hipStream_t st)
     // of a block of up to 512)
     const int grid = std::min(128, nblocks(s.n, 4));
     static_assert(128 * kWG >= kSmallFields * kSmallN && 4 * kSmallFields <= kWG, "a value per thread");
-    hipLaunchKernelGGL((kd_small_step<MX, K>), dim3(grid), dim3(kWG), lds, st, s, par);
+    hipLaunchKernelGGL((kd_small_step<MX, K>), dim3(grid), dim3(kWG), lds, st, s, par, mirror);
     return hipGetLastError();
 }
 
-hipError_t launch_small_step(const SmallSteps &s, int prec, int par, hipStream_t st)
+hipError_t launch_small_step(const SmallSteps &s, int prec, int par, StepCtl *mirror,
+                             hipStream_t st)
 {
     if (s.n < 1 || s.n > kSmallN) return hipErrorInvalidValue;
     const int k = nblocks(s.n, kWG);
     if (prec == kMixed)
-        return k <= 1 ? small_step<true, 1>(s, par, st) : k <= 2 ? small_step<true, 2>(s, par, st)
-             : k <= 4 ? small_step<true, 4>(s, par, st) : small_step<true, 8>(s, par, st);
-    return k <= 1 ? small_step<false, 1>(s, par, st) : k <= 2 ? small_step<false, 2>(s, par, st)
-         : k <= 4 ? small_step<false, 4>(s, par, st) : small_step<false, 8>(s, par, st);
+        return k <= 1 ? small_step<true, 1>(s, par, mirror, st) : k <= 2 ? small_step<true, 2>(s, par, mirror, st)
+             : k <= 4 ? small_step<true, 4>(s, par, mirror, st) : small_step<true, 8>(s, par, mirror, st);
+    return k <= 1 ? small_step<false, 1>(s, par, mirror, st) : k <= 2 ? small_step<false, 2>(s, par, mirror, st)
+         : k <= 4 ? small_step<false, 4>(s, par, mirror, st) : small_step<false, 8>(s, par, mirror, st);
 }
 
 hipError_t launch_step_force(const JStore &s, const IBlock &b, double *part, int nj,
