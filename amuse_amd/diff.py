@@ -76,41 +76,65 @@ def _check(t: torch.Tensor, name: str) -> torch.Tensor:
     return t.contiguous()
 
 
-def _suffix(dtype):
-    if dtype == torch.float32:
-        return "f32"
-    if dtype == torch.float64:
-        return "f64"
-    raise TypeError(f"unsupported dtype {dtype}")
+_NAMES = {torch.float32: "f32", torch.float64: "f64"}
 
 
-@functools.lru_cache(maxsize=256)
-def _workspace_size(query, dtype, n):
-    return getattr(_kernels(), query + _suffix(dtype))(n)
+class _Bound:
+    """The kernels' entry points of one dtype."""
+
+    def __init__(self, dtype):
+        L, name = _kernels(), _NAMES[dtype]
+        for fn in ("forces_ws", "adjoint_ws", "step_predict", "step_correct", "step_correct_t",
+                   "step_predict_t"):
+            setattr(self, fn, getattr(L, f"g6a_{fn}_{name}"))
+        size = torch.empty(0, dtype=dtype).element_size()
+        self.size = size
+        # values of the workspace of n particles
+        self.forces_values, self.adjoint_values = (
+            functools.lru_cache(maxsize=256)(
+                lambda n, q=getattr(L, f"g6a_{what}_workspace_{name}"): -(-q(n) // size))
+            for what in ("forces", "adjoint"))
 
 
-def _workspace(query, dtype, n, device):
-    """Device memory for one launch, from torch's allocator on the current
-    stream (which orders its reuse), and its size; (None, 0) where none is
-    used."""
-    size = _workspace_size(query, dtype, n)
-    ws = torch.empty(size, dtype=torch.uint8, device=device) if size > 0 else None
-    return ws, size
+_bound = {}
 
 
-def _forces(x, v, m, eps2, acc, jerk, stream):
+def _entries(dtype):
+    k = _bound.get(dtype)
+    if k is None:
+        if dtype not in _NAMES:
+            raise TypeError(f"unsupported dtype {dtype}")
+        k = _bound[dtype] = _Bound(dtype)
+    return k
+
+
+def _stream(t):
+    """The current stream of t's device, as the entry points take it."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+def _ok(rc, what):
+    if rc != 0:
+        raise RuntimeError(f"g6a_{what} failed ({rc})")
+
+
+def _forces(k, x, v, m, eps2, acc, jerk, stream):
     n = x.shape[0]
-    ws, size = _workspace("g6a_forces_workspace_", x.dtype, n, x.device)
-    _call("g6a_forces_ws_", x.dtype, n, x.data_ptr(), v.data_ptr(), m.data_ptr(), float(eps2),
-          acc.data_ptr(), jerk.data_ptr(), _ptr(ws), size, stream)
+    # device memory for one launch, from torch's allocator on the current
+    # stream (which orders its reuse)
+    values = k.forces_values(n)
+    ws = x.new_empty(values) if values else None
+    _ok(k.forces_ws(n, x.data_ptr(), v.data_ptr(), m.data_ptr(), eps2, acc.data_ptr(),
+                    jerk.data_ptr(), _ptr(ws), values * k.size, stream), "forces")
 
 
 def _adjoint(x, v, m, ga, gj, eps2, gx, gv, gm, stream):
-    n = x.shape[0]
-    ws, size = _workspace("g6a_adjoint_workspace_", x.dtype, n, x.device)
-    _call("g6a_adjoint_ws_", x.dtype, n, x.data_ptr(), v.data_ptr(), m.data_ptr(), ga.data_ptr(),
-          gj.data_ptr(), float(eps2), gx.data_ptr(), gv.data_ptr(), gm.data_ptr(), _ptr(ws), size,
-          stream)
+    k, n = _entries(x.dtype), x.shape[0]
+    values = k.adjoint_values(n)
+    ws = x.new_empty(values) if values else None
+    _ok(k.adjoint_ws(n, x.data_ptr(), v.data_ptr(), m.data_ptr(), ga.data_ptr(), gj.data_ptr(),
+                     eps2, gx.data_ptr(), gv.data_ptr(), gm.data_ptr(), _ptr(ws),
+                     values * k.size, stream), "adjoint")
 
 
 class PairForce(torch.autograd.Function):
@@ -121,7 +145,7 @@ class PairForce(torch.autograd.Function):
         x, v, m = _check(x, "x"), _check(v, "v"), _check(m, "m")
         acc = torch.empty_like(x)
         jerk = torch.empty_like(x)
-        _forces(x, v, m, eps2, acc, jerk, torch.cuda.current_stream(x.device).cuda_stream)
+        _forces(_entries(x.dtype), x, v, m, float(eps2), acc, jerk, _stream(x))
         ctx.save_for_backward(x, v, m)
         ctx.eps2 = float(eps2)
         return acc, jerk
@@ -134,8 +158,7 @@ class PairForce(torch.autograd.Function):
         gx = torch.empty_like(x)
         gv = torch.empty_like(v)
         gm = torch.empty_like(m)
-        _adjoint(x, v, m, ga, gj, ctx.eps2, gx, gv, gm,
-                 torch.cuda.current_stream(x.device).cuda_stream)
+        _adjoint(x, v, m, ga, gj, ctx.eps2, gx, gv, gm, _stream(x))
         return gx, gv, gm, None
 
 
@@ -145,12 +168,6 @@ def pair_force(x, v, m, eps2):
 
 def _ptr(t):
     return None if t is None else t.data_ptr()
-
-
-def _call(name, dtype, *args):
-    rc = getattr(_kernels(), name + _suffix(dtype))(*args)
-    if rc != 0:
-        raise RuntimeError(f"{name}{_suffix(dtype)} failed ({rc})")
 
 
 class HermiteStep(torch.autograd.Function):
@@ -163,39 +180,45 @@ class HermiteStep(torch.autograd.Function):
     def forward(ctx, x, v, a, j, m, dt: float, eps2: float):
         x, v, a, j, m = (_check(t, n) for t, n in ((x, "x"), (v, "v"), (a, "a"), (j, "j"),
                                                     (m, "m")))
-        n = x.shape[0]
-        stream = torch.cuda.current_stream(x.device).cuda_stream
+        n, k, stream = x.shape[0], _entries(x.dtype), _stream(x)
+        dt, eps2 = float(dt), float(eps2)
         xp, vp = torch.empty_like(x), torch.empty_like(v)
-        _call("g6a_step_predict_", x.dtype, n, x.data_ptr(), v.data_ptr(), a.data_ptr(),
-              j.data_ptr(), float(dt), xp.data_ptr(), vp.data_ptr(), stream)
+        _ok(k.step_predict(n, x.data_ptr(), v.data_ptr(), a.data_ptr(), j.data_ptr(), dt,
+                           xp.data_ptr(), vp.data_ptr(), stream), "step_predict")
         a1, j1 = torch.empty_like(x), torch.empty_like(x)
-        _forces(xp, vp, m, eps2, a1, j1, stream)
+        _forces(k, xp, vp, m, eps2, a1, j1, stream)
         x1, v1 = torch.empty_like(x), torch.empty_like(v)
-        _call("g6a_step_correct_", x.dtype, n, x.data_ptr(), v.data_ptr(), a.data_ptr(),
-              j.data_ptr(), a1.data_ptr(), j1.data_ptr(), float(dt), x1.data_ptr(),
-              v1.data_ptr(), stream)
+        _ok(k.step_correct(n, x.data_ptr(), v.data_ptr(), a.data_ptr(), j.data_ptr(),
+                           a1.data_ptr(), j1.data_ptr(), dt, x1.data_ptr(), v1.data_ptr(),
+                           stream), "step_correct")
         ctx.save_for_backward(xp, vp, m)
-        ctx.dt, ctx.eps2 = float(dt), float(eps2)
+        ctx.dt, ctx.eps2 = dt, eps2
         return x1, v1, a1, j1
 
     @staticmethod
     def backward(ctx, gx1, gv1, ga1, gj1):
         xp, vp, m = ctx.saved_tensors
-        n = xp.shape[0]
-        stream = torch.cuda.current_stream(xp.device).cuda_stream
+        n, k, stream = xp.shape[0], _entries(xp.dtype), _stream(xp)
         gx1 = torch.zeros_like(xp) if gx1 is None else gx1.contiguous()
         gv1 = torch.zeros_like(xp) if gv1 is None else gv1.contiguous()
         ga1 = None if ga1 is None else ga1.contiguous()
         gj1 = None if gj1 is None else gj1.contiguous()
         gx, gv, ga, gj = (torch.empty_like(xp) for _ in range(4))
-        ga1t, gj1t = torch.empty_like(xp), torch.empty_like(xp)
-        _call("g6a_step_correct_t_", xp.dtype, n, gx1.data_ptr(), gv1.data_ptr(), _ptr(ga1),
-              _ptr(gj1), ctx.dt, gx.data_ptr(), gv.data_ptr(), ga.data_ptr(), gj.data_ptr(),
-              ga1t.data_ptr(), gj1t.data_ptr(), stream)
-        gxp, gvp, gm = torch.empty_like(xp), torch.empty_like(vp), torch.empty_like(m)
-        _adjoint(xp, vp, m, ga1t, gj1t, ctx.eps2, gxp, gvp, gm, stream)
-        _call("g6a_step_predict_t_", xp.dtype, n, gxp.data_ptr(), gvp.data_ptr(), ctx.dt,
-              gx.data_ptr(), gv.data_ptr(), ga.data_ptr(), gj.data_ptr(), stream)
+        gm = torch.empty_like(m)
+        # the adjoints on the way (of a1 and j1, of xp and vp: [n][3] each, on
+        # 64-value boundaries) and the pair sum's workspace, in one allocation
+        pitch = (3 * n + 63) // 64 * 64
+        values = k.adjoint_values(n)
+        tmp = xp.new_empty(4 * pitch + values)
+        ga1t, gj1t, gxp, gvp, ws = (tmp.data_ptr() + q * pitch * k.size for q in range(5))
+        _ok(k.step_correct_t(n, gx1.data_ptr(), gv1.data_ptr(), _ptr(ga1), _ptr(gj1), ctx.dt,
+                             gx.data_ptr(), gv.data_ptr(), ga.data_ptr(), gj.data_ptr(), ga1t,
+                             gj1t, stream), "step_correct_t")
+        _ok(k.adjoint_ws(n, xp.data_ptr(), vp.data_ptr(), m.data_ptr(), ga1t, gj1t, ctx.eps2, gxp,
+                         gvp, gm.data_ptr(), ws if values else None, values * k.size, stream),
+            "adjoint")
+        _ok(k.step_predict_t(n, gxp, gvp, ctx.dt, gx.data_ptr(), gv.data_ptr(), ga.data_ptr(),
+                             gj.data_ptr(), stream), "step_predict_t")
         return gx, gv, ga, gj, gm, None, None
 
 
