@@ -564,7 +564,7 @@ long long sym_bytes(int n)
 {
     if (n < kSymMin<T, Op>) return 0;
     const g6s::Plan p = sym_plan<T, Op>(n);
-    const long long bytes = 8 * (p.row_values(Op::NC) + p.col_values(Op::NC));
+    const long long bytes = 8 * p.row_values(Op::NC) + (long long)sizeof(T) * p.col_values(Op::NC);
     return bytes <= kSymMaxBytes ? bytes : 0;
 }
 
@@ -572,7 +572,8 @@ template <class T, class Op>
 int launch_sym(int n, const Op &op, T *o0, T *o1, T *o2, void *ws, hipStream_t st)
 {
     const g6s::Plan p = sym_plan<T, Op>(n);
-    double *rowpart = static_cast<double *>(ws), *colpart = rowpart + p.row_values(Op::NC);
+    double *rowpart = static_cast<double *>(ws);
+    T *colpart = reinterpret_cast<T *>(rowpart + p.row_values(Op::NC));
     const dim3 grid(p.items()), wg(g6s::kWG);
     switch (p.rows / 64) {
     case 1: hipLaunchKernelGGL((g6s::k_sym<T, Op, 1>), grid, wg, 0, st, p, op, rowpart, colpart); break;

@@ -44,7 +44,8 @@ struct Plan {
     __host__ __device__ int items() const { return nb * parts; }
     // Whether row block b takes the block d places on (1 <= d <= nb / 2).
     __host__ __device__ bool takes(int b, int d) const { return 2 * d < nb || b < nb / 2; }
-    // values of the partial records, `nc` sums per particle
+    // values of the partial records, `nc` sums per particle (the rows' in FP64,
+    // the columns', plain sums over one tile, in the pass's own type)
     long long row_values(int nc) const { return (long long)items() * nc * rows; }
     long long col_values(int nc) const { return (long long)(nb / 2) * nc * n; }
     // row record of workgroup `it`, sum c, row i of the block
@@ -178,7 +179,7 @@ __device__ __forceinline__ void sym_steps(const Op &op, const typename Word<T>::
 // against 154), ds_add_f64 cost the same as the rotation.
 template <class T, class Op, int IPL>
 __global__ void __launch_bounds__(kWG) k_sym(Plan p, Op op, double *__restrict__ rowpart,
-                                             double *__restrict__ colpart)
+                                             T *__restrict__ colpart)
 {
     using V = typename Word<T>::type;
     constexpr int W = kWords<T, Op>, NC = Op::NC, R = kCol * IPL, N = Word<T>::n;
@@ -231,7 +232,7 @@ __global__ void __launch_bounds__(kWG) k_sym(Plan p, Op op, double *__restrict__
             if (col0 + lane < p.n) {
 #pragma unroll
                 for (int k = 0; k < NC; k++)
-                    colpart[p.col_at(u / IPL, NC, k, col0 + lane)] = double(c[k]);
+                    colpart[p.col_at(u / IPL, NC, k, col0 + lane)] = c[k];
             }
         } else {
             sym_steps<T, Op, IPL, false>(op, tile, col0, row0, r, s, c);
@@ -260,7 +261,7 @@ __global__ void __launch_bounds__(kWG) k_sym(Plan p, Op op, double *__restrict__
 // row block, then those of its own block's workgroups.  HBM-bound.
 template <class T, int NC>
 __global__ void __launch_bounds__(256) k_sym_sum(Plan p, const double *__restrict__ rowpart,
-                                                 const double *__restrict__ colpart,
+                                                 const T *__restrict__ colpart,
                                                  T *__restrict__ o0, T *__restrict__ o1,
                                                  T *__restrict__ o2)
 {
@@ -271,7 +272,7 @@ __global__ void __launch_bounds__(256) k_sym_sum(Plan p, const double *__restric
     const int nd = p.nb / 2 - (p.nb % 2 == 0 && b < p.nb / 2 ? 1 : 0);
     Long<double> z;
 #pragma unroll 8
-    for (int d = 1; d <= nd; d++) z.add(colpart[p.col_at(d, NC, c, i)]);
+    for (int d = 1; d <= nd; d++) z.add(double(colpart[p.col_at(d, NC, c, i)]));
 #pragma unroll 8
     for (int k = 0; k < p.parts; k++)
         z.add(rowpart[p.row_at(b * p.parts + k, NC, c, i - b * p.rows)]);
