@@ -43,6 +43,11 @@ constexpr long long kPartBudget = 1ll << 24;  // nchunk * ni limit for partials 
 // copy launches: at the block sizes of a block-step integrator the copies'
 // latency, not their bytes, is the cost); larger ones are copied.
 constexpr int kDirectRows = 4096;
+// The same for the columns of a g6x_set_j_particles call, which the scatter
+// kernel reads once, in order.  us of load and forces on 250 rows, copied /
+// in place: 122 / 109 at 4500 records, 126 / 114 at 5500, 136 / 128 at 8000,
+// 152 / 149 at 12000, 171 / 173 at 16000, 352 / 443 at 60000.
+constexpr int kDirectCols = 12000;
 
 struct TuneEntry {
     int ni_lo, ni_hi;  // bucket [lo, hi]
@@ -93,7 +98,7 @@ struct Unit {
     hipEvent_t ev_stage = nullptr;
     // A g6x_set_j_particles call with rising addresses, waiting for the next
     // flush (before `stage`): its arrays one after the other in pinned memory
-    // and, beyond kDirectRows records, on their way to the device.
+    // and, beyond kDirectCols records, on their way to the device.
     int cols = 0;  // records
     bool cols_k18 = false;
     double *h_cols = nullptr;
@@ -373,7 +378,7 @@ int flush_columns(bool may_allocate, bool predict)
                                    "(the allocation-free call cannot grow them)");
     const bool pv = U.pred_valid && U.pred_prec == U.prec && U.pred_compat == U.compat;
     const bool all = predict && n == U.nj_hw && !pred_current(U.ti);
-    HIPCHK(g6k::launch_scatter_columns(U.js, n > kDirectRows ? U.d_cols : U.d_hcols, n, U.cols_k18,
+    HIPCHK(g6k::launch_scatter_columns(U.js, n > kDirectCols ? U.d_cols : U.d_hcols, n, U.cols_k18,
                                        U.prec, pv || all, all ? U.ti : U.pred_ti, U.compat, U.stream),
            "scatter");
     U.cols = 0;
@@ -1457,7 +1462,7 @@ static int set_columns(int n, const int *address, const int *index, const double
         U.h_cols_cap = cap;
         HIPCHK(hipHostGetDevicePointer(reinterpret_cast<void **>(&U.d_hcols), U.h_cols, 0), "stage map");
     }
-    if (n > kDirectRows && values > U.d_cols_cap) {
+    if (n > kDirectCols && values > U.d_cols_cap) {
         HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
         if (U.d_cols) (void)hipFree(U.d_cols);
         U.d_cols = nullptr;
@@ -1470,7 +1475,7 @@ static int set_columns(int n, const int *address, const int *index, const double
     auto send = [&]() {
         const size_t from = sent;
         sent = at;
-        return n > kDirectRows && at > from
+        return n > kDirectCols && at > from
                    ? hipMemcpyAsync(U.d_cols + from, U.h_cols + from, sizeof(double) * (at - from),
                                     hipMemcpyHostToDevice, U.stream)
                    : hipSuccess;

@@ -692,10 +692,10 @@ def test_pair_once_full_pass_edges(g6, prec, n):
 
 
 @pytest.mark.parametrize("prec", [0, 1])
-@pytest.mark.parametrize("n", [63, 64, 65, 2049, 4096, 4097])
+@pytest.mark.parametrize("n", [63, 64, 65, 2049, 4097, 12000, 12001])
 def test_set_j_particles_by_columns(g6, n, prec):
     """g6x_set_j_particles with rising addresses (array by array, from 64
-    records on; read in place up to 4096) leaves what one g6_set_j_particle
+    records on; read in place up to 12000) leaves what one g6_set_j_particle
     per record leaves, bit for bit: a whole store, predicted along with it;
     a store with gaps; updates of part of it at the same time; snap terms;
     records before and after it by other calls; a call that does not rise."""
