@@ -985,7 +985,10 @@ void pair_rule(Ensemble *E)
 }
 
 // The records of the clusters that can be taken pair-once and the units of a
-// wave: as many as leave four waves for each of the chip's SIMDs, at most 4.
+// wave: as many as leave sixteen waves for each of the chip's SIMDs, at most 4
+// (1 against the 3 that four waves allow: a round of 512 clusters mixed 221 ->
+// 208 us, of 350 in FP64 245 -> 234; 2 and 3 are the slower ones everywhere
+// below).
 // With a cluster above kPairMaxN, or without room for the records every cluster keeps the other kernels.
 bool pair_setup(Ensemble *E, int cus)
 {
@@ -996,7 +999,7 @@ bool pair_setup(Ensemble *E, int cus)
         if (size_class(n) >= kPairClass) units += g6cp::Plan(n, 1).work();
     }
     if (units == 0) return true;
-    d.pair_per = int(std::min(4ll, std::max(1ll, units / (16 * cus))));
+    d.pair_per = int(std::min(4ll, std::max(1ll, units / (64 * cus))));
     d.pair_fill = 4 * cus;
     E->ws_at.assign(d.nc, -1);
     long long at = 0;
