@@ -152,7 +152,9 @@ int g6c_state(void *ens, double x[][3], double v[][3], double t[],
 int g6c_forces(void *ens, int precision, double acc[][3], double jerk[][3],
                double pot[]);
 /* lanes per i-particle (1..64, a power of two) for each of 8 size classes
- * (<=16, <=32, ..., <=2048, more) */
+ * (<=16, <=32, ..., <=2048, more).  While a class above 128 particles has the
+ * shape it starts with (one lane, 256 j), its clusters are taken pair by
+ * unordered pair, in ensembles without a cluster above 8192. */
 int g6c_set_tiles(void *ens, const int njs_per_class[8]);
 int g6c_get_tiles(void *ens, int njs_per_class[8]);
 /* j per LDS tile (16..256, a power of two) for each size class */
@@ -247,7 +249,8 @@ int g6a_step_predict_t_f64(int n, const double *gxp, const double *gvp, double d
  * evolve_model loop, src/amuse_ph4/interface.cc:673-674: the system time
  * ends >= t_end, past it when t_end is not commensurate with the steps), or
  * for max_blocks (> 0) block steps, replaying `steps_per_graph` captured
- * steps at a time; returns the block steps taken or a negative code, and
+ * steps (at most 8) at a time; returns the block steps taken or a negative
+ * code, and
  * sets *reached (if not NULL) to 1 when it stopped at t_end, 0 when the
  * block budget ran out first.
  * g6d_energy: kinetic and potential energy at the system time (FP64 pass).
