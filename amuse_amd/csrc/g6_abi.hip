@@ -97,15 +97,11 @@ struct Unit {
     size_t d_stage_cap = 0;
     hipEvent_t ev_stage = nullptr;
     // A g6x_set_j_particles call with rising addresses, waiting for the next
-    // flush (before `stage`): its arrays one after the other in pinned memory
-    // and, beyond kDirectCols records, on their way to the device.
+    // flush (before `stage`): its arrays one after the other at the start of
+    // h_stage (no more bytes than as many JRecords) and, beyond kDirectCols
+    // records, on their way to d_stage.
     int cols = 0;  // records
     bool cols_k18 = false;
-    double *h_cols = nullptr;
-    double *d_hcols = nullptr;  // the device's address of h_cols
-    double *d_cols = nullptr;
-    size_t h_cols_cap = 0, d_cols_cap = 0;  // values
-    size_t flushed_max = 0;  // records of the largest flush that could allocate
 
     // pinned mirrors of the device i-block rows (same row pitch): [8][cap]
     // x y z vx vy vz h2 id and [8][cap] acc3 jerk3 pot nn; id and nn are
@@ -364,6 +360,18 @@ int ensure_partials(int nchunk, int ni)
 // without the staging event the stream is synchronised instead of recorded.
 bool pred_current(double t);
 
+// Marks the staging buffers as read once the work queued so far is done.
+int stage_read(bool may_allocate)
+{
+    if (!U.ev_stage && !may_allocate) {
+        HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
+        return 0;
+    }
+    if (!U.ev_stage) HIPCHK(hipEventCreateWithFlags(&U.ev_stage, hipEventDisableTiming), "event");
+    HIPCHK(hipEventRecord(U.ev_stage, U.stream), "stage record");
+    return 0;
+}
+
 // The columns of a g6x_set_j_particles call to the store.  predict: the caller
 // needs the store predicted to U.ti next; if the columns set every slot that
 // is done along with them (30000 slots: a 9 us kernel less).
@@ -371,14 +379,10 @@ int flush_columns(bool may_allocate, bool predict)
 {
     const int n = U.cols;
     if (n == 0) return 0;
-    // (the allocation-free call takes what the staging buffers of a flush
-    // before it could hold)
-    if (!may_allocate && size_t(n) > U.flushed_max)
-        return fail(G6X_ERR_NOMEM, "pending set_j_particle records exceed the staging buffers "
-                                   "(the allocation-free call cannot grow them)");
     const bool pv = U.pred_valid && U.pred_prec == U.prec && U.pred_compat == U.compat;
     const bool all = predict && n == U.nj_hw && !pred_current(U.ti);
-    HIPCHK(g6k::launch_scatter_columns(U.js, n > kDirectCols ? U.d_cols : U.d_hcols, n, U.cols_k18,
+    const JRecord *rec = n > kDirectCols ? U.d_stage : U.d_hstage;
+    HIPCHK(g6k::launch_scatter_columns(U.js, reinterpret_cast<const double *>(rec), n, U.cols_k18,
                                        U.prec, pv || all, all ? U.ti : U.pred_ti, U.compat, U.stream),
            "scatter");
     U.cols = 0;
@@ -390,26 +394,12 @@ int flush_columns(bool may_allocate, bool predict)
     } else if (!pv) {
         U.pred_valid = false;
     }
-    if (!U.ev_stage && !may_allocate) {
-        HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
-    } else {
-        if (!U.ev_stage) HIPCHK(hipEventCreateWithFlags(&U.ev_stage, hipEventDisableTiming), "event");
-        HIPCHK(hipEventRecord(U.ev_stage, U.stream), "stage record");
-    }
-    if (may_allocate) U.flushed_max = std::max(U.flushed_max, std::max(size_t(n), size_t(4096)));
-    return 0;
+    return stage_read(may_allocate);
 }
 
-int flush_stage(bool may_allocate = true, bool predict = false)
+// h_stage and d_stage for n records.
+int grow_stage(size_t n)
 {
-    const int rc = flush_columns(may_allocate, predict);
-    if (rc) return rc;
-    const size_t n = U.stage.size();
-    if (n == 0) return 0;
-    if (!may_allocate && (n > U.h_stage_cap || (n > size_t(kDirectRows) && n > U.d_stage_cap)))
-        return fail(G6X_ERR_NOMEM, "pending set_j_particle records exceed the staging buffers "
-                                   "(the allocation-free call cannot grow them)");
-    if (U.ev_stage) HIPCHK(hipEventSynchronize(U.ev_stage), "stage event");
     if (n > U.h_stage_cap) {
         if (U.h_stage) (void)hipHostFree(U.h_stage);
         size_t cap = std::max<size_t>(n, 4096);
@@ -426,25 +416,46 @@ int flush_stage(bool may_allocate = true, bool predict = false)
         if (e != hipSuccess) { U.d_stage = nullptr; U.d_stage_cap = 0; return fail(G6X_ERR_NOMEM, "hipMalloc stage", e); }
         U.d_stage_cap = cap;
     }
-    memcpy(U.h_stage, U.stage.data(), sizeof(JRecord) * n);
+    return 0;
+}
+
+// Whether the staging buffers hold n records as they are.
+bool stage_holds(size_t n)
+{
+    return n <= U.h_stage_cap && (n <= size_t(kDirectRows) || n <= U.d_stage_cap);
+}
+
+int flush_stage(bool may_allocate = true, bool predict = false)
+{
+    const size_t n = U.stage.size();
+    if (!may_allocate && !stage_holds(n))
+        return fail(G6X_ERR_NOMEM, "pending set_j_particle records exceed the staging buffers "
+                                   "(the allocation-free call cannot grow them)");
+    // the records go behind pending columns, or where there is no room for
+    // them (or no columns) to the start, once what lies there has been read
+    size_t at = size_t(U.cols);
+    int rc = flush_columns(may_allocate, predict);
+    if (rc || n == 0) return rc;
+    if (at + n > U.h_stage_cap || !stage_holds(n)) at = 0;
+    if (at == 0) {
+        if (U.ev_stage) HIPCHK(hipEventSynchronize(U.ev_stage), "stage event");
+        rc = grow_stage(n);
+        if (rc) return rc;
+    }
+    memcpy(U.h_stage + at, U.stage.data(), sizeof(JRecord) * n);
     // small stages are read by the scatter kernel where they lie (pinned
     // host memory); large ones are copied to the device first
-    const JRecord *rec = U.d_hstage;
+    const JRecord *rec = U.d_hstage + at;
     if (n > size_t(kDirectRows)) {
-        HIPCHK(hipMemcpyAsync(U.d_stage, U.h_stage, sizeof(JRecord) * n, hipMemcpyHostToDevice, U.stream), "stage H2D");
+        HIPCHK(hipMemcpyAsync(U.d_stage, U.h_stage + at, sizeof(JRecord) * n, hipMemcpyHostToDevice, U.stream), "stage H2D");
         rec = U.d_stage;
     }
     const bool pv = U.pred_valid && U.pred_prec == U.prec && U.pred_compat == U.compat;
     HIPCHK(g6k::launch_scatter(U.js, rec, int(n), U.prec, pv ? 1 : 0, U.pred_ti, U.compat, U.stream), "scatter");
-    if (!U.ev_stage && !may_allocate) {
-        HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
-    } else {
-        if (!U.ev_stage) HIPCHK(hipEventCreateWithFlags(&U.ev_stage, hipEventDisableTiming), "event");
-        HIPCHK(hipEventRecord(U.ev_stage, U.stream), "stage record");
-    }
+    rc = stage_read(may_allocate);
+    if (rc) return rc;
     for (const auto &r : U.stage) U.stage_pos[r.addr] = -1;
     U.stage.clear();
-    if (may_allocate) U.flushed_max = std::max(U.flushed_max, std::max(n, size_t(4096)));
     if (!pv) U.pred_valid = false;
     return 0;
 }
@@ -691,9 +702,6 @@ int do_open(int cluster)
         if (U.ib.base) (void)hipFree(U.ib.base);
         if (U.ib.part_base) (void)hipFree(U.ib.part_base);
         if (U.d_stage) (void)hipFree(U.d_stage);
-        if (U.d_cols) (void)hipFree(U.d_cols);
-        U.d_cols = nullptr;
-        U.d_cols_cap = 0;
         if (U.sp_base) (void)hipFree(U.sp_base);
         if (U.sp_rows) (void)hipFree(U.sp_rows);
         if (U.sp_buf.base) (void)hipFree(U.sp_buf.base);
@@ -1430,58 +1438,49 @@ G6_API int g6x_set_tiles(int njs, int ipl, int nchunk, int smem)
 // staging vector and from there to pinned memory the host took 30 ns each
 // (N = 262144 8.7 ms of a full pass), by columns about half, and the copy to the device
 // is under way meanwhile.
+// Only while nothing else is pending (a flush here would change the store
+// under a latched calc), with staging buffers that no queued work still reads
+// and that hold the records as they are; they grow here only in a call that
+// grows the j-store as well, else in a flush.
 static int set_columns(int n, const int *address, const int *index, const double *tj,
                        const double *dtj, const double *mass, const double (*k18)[3],
-                       const double (*j6)[3], const double (*a2)[3], const double (*v)[3],
-                       const double (*x)[3], bool &taken)
+                const double (*j6)[3], const double (*a2)[3], const double (*v)[3],
+                const double (*x)[3], bool &taken)
 {
-    if (n < 64 || !U.open || address[0] < 0 || address[n - 1] >= kMaxSlots) return 0;
+    if (n < 64 || !U.open || U.cols > 0 || !U.stage.empty()) return 0;
+    if (address[0] < 0 || address[n - 1] >= kMaxSlots) return 0;
     bool rising = true;
     for (int q = 1; q < n; q++) rising &= address[q] > address[q - 1];
     if (!rising) return 0;
-    int rc = flush_stage();  // records of earlier calls come before these
-    if (rc) return rc;
-    if (address[n - 1] >= U.js.cap) {
-        rc = grow_jstore(address[n - 1] + 1);
-        if (rc) return rc;
-    }
     const size_t N = size_t(n);
+    const bool grow = address[n - 1] >= U.js.cap;
+    if (!grow && !stage_holds(N)) return 0;
+    if (grow) {
+        int rc = grow_jstore(address[n - 1] + 1);
+        if (rc) return rc;
+        if (U.ev_stage) HIPCHK(hipEventSynchronize(U.ev_stage), "stage event");
+        if (grow_stage(N)) return 0;  // (and an error again in the flush)
+    } else if (U.ev_stage && hipEventQuery(U.ev_stage) != hipSuccess) {
+        (void)hipGetLastError();  // not ready
+        return 0;
+    }
     bool any18 = false;
     for (size_t q = 0; q < N; q++)
         any18 |= (k18[q][0] != 0.0) | (k18[q][1] != 0.0) | (k18[q][2] != 0.0);
-    const size_t values = N * (any18 ? g6k::kColumnRowK18 : g6k::kColumnRow);
-    if (U.ev_stage) HIPCHK(hipEventSynchronize(U.ev_stage), "stage event");
-    if (values > U.h_cols_cap) {
-        HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
-        if (U.h_cols) (void)hipHostFree(U.h_cols);
-        U.h_cols = nullptr;
-        U.h_cols_cap = 0;
-        const size_t cap = std::max<size_t>(values, 4096 * g6k::kColumnRowK18);
-        hipError_t e = hipHostMalloc(reinterpret_cast<void **>(&U.h_cols), sizeof(double) * cap);
-        if (e != hipSuccess) { U.h_cols = nullptr; return fail(G6X_ERR_NOMEM, "hipHostMalloc stage", e); }
-        U.h_cols_cap = cap;
-        HIPCHK(hipHostGetDevicePointer(reinterpret_cast<void **>(&U.d_hcols), U.h_cols, 0), "stage map");
-    }
-    if (n > kDirectCols && values > U.d_cols_cap) {
-        HIPCHK(hipStreamSynchronize(U.stream), "stage sync");
-        if (U.d_cols) (void)hipFree(U.d_cols);
-        U.d_cols = nullptr;
-        U.d_cols_cap = 0;
-        hipError_t e = hipMalloc(reinterpret_cast<void **>(&U.d_cols), sizeof(double) * values);
-        if (e != hipSuccess) { U.d_cols = nullptr; return fail(G6X_ERR_NOMEM, "hipMalloc stage", e); }
-        U.d_cols_cap = values;
-    }
+    static_assert(sizeof(JRecord) >= sizeof(double) * g6k::kColumnRowK18, "columns fit h_stage");
+    double *const h = reinterpret_cast<double *>(U.h_stage);
+    double *const d = reinterpret_cast<double *>(U.d_stage);
     size_t at = 0, sent = 0;
     auto send = [&]() {
         const size_t from = sent;
         sent = at;
         return n > kDirectCols && at > from
-                   ? hipMemcpyAsync(U.d_cols + from, U.h_cols + from, sizeof(double) * (at - from),
+                   ? hipMemcpyAsync(d + from, h + from, sizeof(double) * (at - from),
                                     hipMemcpyHostToDevice, U.stream)
                    : hipSuccess;
     };
     auto put = [&](const void *p, size_t vals) {
-        memcpy(U.h_cols + at, p, sizeof(double) * vals);
+        memcpy(h + at, p, sizeof(double) * vals);
         at += vals;
     };
     put(x, 3 * N);
@@ -1493,8 +1492,8 @@ static int set_columns(int n, const int *address, const int *index, const double
     put(tj, N);
     put(dtj, N);
     put(mass, N);
-    memcpy(U.h_cols + at, address, sizeof(int) * N);
-    memcpy(reinterpret_cast<int *>(U.h_cols + at) + N, index, sizeof(int) * N);
+    memcpy(h + at, address, sizeof(int) * N);
+    memcpy(reinterpret_cast<int *>(h + at) + N, index, sizeof(int) * N);
     at += N;
     if (any18) put(k18, 3 * N);
     HIPCHK(send(), "stage H2D");
