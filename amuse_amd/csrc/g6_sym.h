@@ -116,8 +116,11 @@ struct Long<double> {
 // BOTH, to the column's z (FIRST: sets them); self: r and c are one particle
 // (only met without BOTH).
 
-// Particle j's values, or for j >= n those of one that contributes nothing
-// (zero mass and adjoints, far away).
+// Particle j's values, or for j >= n those of one that contributes nothing:
+// zero mass and adjoints, away from every particle (so that y is finite with
+// eps2 = 0) but no further than its products with real particles' values stay
+// finite, as 0 times an infinity would reach their sums: in FP32 velocities and
+// adjoints up to 1e28 (at 1e18, adjoints of 1e21 made every gradient NaN).
 template <class T, class Op>
 __device__ __forceinline__ void load_values(const Op &op, int j, int n, T (&f)[Op::NV])
 {
@@ -125,7 +128,8 @@ __device__ __forceinline__ void load_values(const Op &op, int j, int n, T (&f)[O
         op.load(j, f);
     } else {
 #pragma unroll
-        for (int k = 0; k < Op::NV; k++) f[k] = k < 3 ? T(sizeof(T) == 4 ? 1e18 : 1e150) : T(0);
+        for (int k = 0; k < Op::NV; k++)
+            f[k] = k < 3 ? T(sizeof(T) == 4 ? 1.03e10 - 0.07e10 * k : 1e150) : T(0);
     }
 }
 

@@ -296,3 +296,21 @@ def test_adjoint_pair_once_edges(n):
             assert L.g6a_adjoint_ws_f64(n, *ptrs(*ins), 1e-4, *ptrs(*same), None, 0, st) == 0
             for o, r in zip(same, ref):
                 assert torch.equal(o, r)
+
+
+@pytest.mark.parametrize("n", [5003, 10003])
+def test_large_adjoint_inputs(n):
+    """FP32 gradients of a loss scaled by 2^70 are 2^70 times those of the loss
+    (every product with a pair's geometry stays far inside FP32's range), also
+    where the last blocks and tiles are filled up with padding."""
+    from amuse_amd import diff
+    x, v, m = (t.to(torch.float32).requires_grad_() for t in tensors(n, 9))
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    w = [torch.randn(n, 3, device="cuda", generator=gen) for _ in range(2)]
+    out = diff.pair_force(x, v, m, 1e-2)
+    plain = torch.autograd.grad(out, (x, v, m), grad_outputs=w, retain_graph=True)
+    scaled = torch.autograd.grad(out, (x, v, m), grad_outputs=[q * 2.0 ** 70 for q in w])
+    for p, s in zip(plain, scaled):
+        assert torch.isfinite(s).all()
+        # a power of two: the same roundings
+        assert (s * 2.0 ** -70 - p).abs().max() <= 1e-6 * p.abs().max()
