@@ -118,20 +118,29 @@ def _ok(rc, what):
         raise RuntimeError(f"g6a_{what} failed ({rc})")
 
 
+def _room(x, head, values):
+    """New memory like x's for one launch: `head` values and a workspace of
+    `values` (from torch's allocator on the current stream, which orders its
+    reuse), and the workspace's values.  Without room for the workspace it has
+    none: the entry points then take the kernels that need none."""
+    if values:
+        try:
+            return x.new_empty(head + values), values
+        except torch.OutOfMemoryError:
+            pass
+    return (x.new_empty(head) if head else None), 0
+
+
 def _forces(k, x, v, m, eps2, acc, jerk, stream):
     n = x.shape[0]
-    # device memory for one launch, from torch's allocator on the current
-    # stream (which orders its reuse)
-    values = k.forces_values(n)
-    ws = x.new_empty(values) if values else None
+    ws, values = _room(x, 0, k.forces_values(n))
     _ok(k.forces_ws(n, x.data_ptr(), v.data_ptr(), m.data_ptr(), eps2, acc.data_ptr(),
                     jerk.data_ptr(), _ptr(ws), values * k.size, stream), "forces")
 
 
 def _adjoint(x, v, m, ga, gj, eps2, gx, gv, gm, stream):
     k, n = _entries(x.dtype), x.shape[0]
-    values = k.adjoint_values(n)
-    ws = x.new_empty(values) if values else None
+    ws, values = _room(x, 0, k.adjoint_values(n))
     _ok(k.adjoint_ws(n, x.data_ptr(), v.data_ptr(), m.data_ptr(), ga.data_ptr(), gj.data_ptr(),
                      eps2, gx.data_ptr(), gv.data_ptr(), gm.data_ptr(), _ptr(ws),
                      values * k.size, stream), "adjoint")
@@ -208,9 +217,8 @@ class HermiteStep(torch.autograd.Function):
         # the adjoints on the way (of a1 and j1, of xp and vp: [n][3] each, on
         # 64-value boundaries) and the pair sum's workspace, in one allocation
         pitch = (3 * n + 63) // 64 * 64
-        values = k.adjoint_values(n)
-        tmp = xp.new_empty(4 * pitch + values)
-        ga1t, gj1t, gxp, gvp, ws = (tmp.data_ptr() + q * pitch * k.size for q in range(5))
+        tmp, values = _room(xp, 4 * pitch, k.adjoint_values(n))
+        ga1t, gj1t, gxp, gvp, ws = ((_ptr(tmp) or 0) + q * pitch * k.size for q in range(5))
         _ok(k.step_correct_t(n, gx1.data_ptr(), gv1.data_ptr(), _ptr(ga1), _ptr(gj1), ctx.dt,
                              gx.data_ptr(), gv.data_ptr(), ga.data_ptr(), gj.data_ptr(), ga1t,
                              gj1t, stream), "step_correct_t")
