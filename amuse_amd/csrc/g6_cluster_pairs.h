@@ -62,7 +62,8 @@ struct WaveLds {
 
 // Steps k0 <= k < k1 of a tile: lane l pairs its rows with column
 // (l + k) mod 64.  BOTH: the columns' sums u travel with their columns and
-// come out with lane l holding those of column (l + k1 - 1) mod 64.
+// come out with lane l holding those of column (l + k1 - 1) mod 64 (for
+// g6s::settle).
 template <class Op, int IPL, int NC, bool BOTH, int W>
 __device__ __forceinline__ void steps(const typename g6s::Word<typename Op::T>::type (&tile)[W][2 * kCol],
                                       int k0, int k1, const Op &op,
@@ -154,7 +155,8 @@ __device__ __forceinline__ float bits_max(float a, float b)
 // the second).
 struct Mixed {
     using T = float;
-    static constexpr int NV = 10, W = 3, kHalf = kCol;
+    static constexpr int NV = 10, W = 3;
+    static constexpr int kRowSteps = kCol;  // steps of a row's plain sum
     struct Near {
         float a = 0.0f, b = 0.0f;
         __device__ __forceinline__ float value() const { return bits_max(a * a, b); }
@@ -189,11 +191,13 @@ struct Mixed {
     }
 };
 
-// FP64.  Values: x y z m vx vy vz.  A plain sum runs over half a tile
-// (kHalf steps).
+// FP64.  Values: x y z m vx vy vz.
 struct Plain {
     using T = double;
-    static constexpr int NV = 7, W = 4, kHalf = kCol / 2;
+    static constexpr int NV = 7, W = 4;
+    // (of 32 terms; 32 steps would leave the rows' records, rounded once each,
+    // above the pair by pair kernels' error by 3-8 % below 1000 particles)
+    static constexpr int kRowSteps = kCol / 4;
     struct Near {
         float b = 0.0f;
         __device__ __forceinline__ float value() const { return b; }
@@ -252,24 +256,6 @@ __device__ __forceinline__ void stage(const Op &op, WaveLds<typename Op::T, Op::
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// Puts the columns' sums down, lane l those of column (l + shift) mod 64, and
-// picks them up in the columns' own lanes.
-template <class Op, int NC>
-__device__ __forceinline__ void put(WaveLds<typename Op::T, Op::W> &lds, int shift,
-                                    const typename Op::T (&u)[kNC])
-{
-    const int e = ((threadIdx.x & 63) + shift) & 63;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-#pragma unroll
-    for (int q = 0; q < NC; q++) lds.put[q][e] = u[q];
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-}
-template <class Op>
-__device__ __forceinline__ typename Op::T pick(const WaveLds<typename Op::T, Op::W> &lds, int q)
-{
-    return lds.put[q][threadIdx.x & 63];
-}
-
 template <class T, int NC, int IPL>
 __device__ __forceinline__ void fold(g6s::Long<T> (*tot)[kNC], T (*s)[kNC])
 {
@@ -293,17 +279,18 @@ __device__ __forceinline__ void diagonal(const Op &op, WaveLds<typename Op::T, O
 {
     using T = typename Op::T;
     T u[kNC];
+    g6s::put_zero<NC>(lds.put);
     steps<Op, 1, NC, true>(lds.tile, 1, kCol / 2, op, r, s, u, near);
-    put<Op, NC>(lds, kCol / 2 - 1, u);
+    g6s::settle<NC>(lds.put, kCol / 2 - 1, u);
     fold<T, NC, 1>(tot, s);
 #pragma unroll
-    for (int q = 0; q < NC; q++) tot[0][q].add(pick<Op>(lds, q));
+    for (int q = 0; q < NC; q++) tot[0][q].add(lds.put[q][threadIdx.x & 63]);
     steps<Op, 1, NC, false>(lds.tile, kCol / 2, kCol / 2 + 1, op, r, s, u, near);
     fold<T, NC, 1>(tot, s);
 }
 
 // All 64 steps of a staged tile for IPL rows per lane; sink(q, sum) takes the
-// columns' sums, of either half of the steps where plain sums are that short.
+// columns' sums, in their own lanes.
 template <class Op, int NC, int IPL, class Sink>
 __device__ __forceinline__ void whole(const Op &op, WaveLds<typename Op::T, Op::W> &lds,
                                       const typename Op::T (*r)[Op::NV],
@@ -312,17 +299,20 @@ __device__ __forceinline__ void whole(const Op &op, WaveLds<typename Op::T, Op::
                                       Sink &&sink)
 {
     using T = typename Op::T;
+    constexpr int kSeg = g6s::kSeg;
     T u[kNC];
-    // one loop body for both halves: the first half's sums wait in LDS
+    g6s::put_zero<NC>(lds.put);
 #pragma unroll 1
-    for (int k = 0; k < kCol; k += Op::kHalf) {
-        steps<Op, IPL, NC, true>(lds.tile, k, k + Op::kHalf, op, r, s, u, near);
+    for (int h = 0; h < kCol; h += Op::kRowSteps) {
+#pragma unroll 1
+        for (int k = h; k < h + Op::kRowSteps; k += kSeg) {
+            steps<Op, IPL, NC, true>(lds.tile, k, k + kSeg, op, r, s, u, near);
+            g6s::settle<NC>(lds.put, k + kSeg - 1, u);
+        }
         fold<T, NC, IPL>(tot, s);
-        if (k + Op::kHalf < kCol) put<Op, NC>(lds, k + Op::kHalf - 1, u);
     }
 #pragma unroll
-    for (int q = 0; q < NC; q++)
-        sink(q, g6s::from_next_lane(u[q]), Op::kHalf < kCol ? pick<Op>(lds, q) : T(0));
+    for (int q = 0; q < NC; q++) sink(q, lds.put[q][threadIdx.x & 63]);
 }
 
 // Wave `wi` of a cluster whose particles are off .. off + n - 1: its rows'
@@ -358,10 +348,8 @@ __device__ __forceinline__ float wave_item(const Op &op, const Plan &p, int off,
             if (row0 + kCol < end) {
                 stage(op, lds, row0 + kCol, end);
                 // (the columns are the second rows)
-                whole<Op, NC, 1>(op, lds, &r[0], &tot[0], &s[0], near, [&](int q, T x, T y) {
-                    tot[1][q].add(x);
-                    if (Op::kHalf < kCol) tot[1][q].add(y);
-                });
+                whole<Op, NC, 1>(op, lds, &r[0], &tot[0], &s[0], near,
+                                  [&](int q, T x) { tot[1][q].add(x); });
                 diagonal<Op, NC>(op, lds, &r[1], &tot[1], &s[1], near);
             }
             continue;
@@ -371,8 +359,8 @@ __device__ __forceinline__ float wave_item(const Op &op, const Plan &p, int off,
         if (c0 >= p.n) continue;
         stage(op, lds, off + c0, end);
         T *w = colrec + (size_t(d - 1) * kNC) * p.n + c0;
-        whole<Op, NC, kIPL>(op, lds, &r[0], &tot[0], &s[0], near, [&](int q, T x, T y) {
-            if (c0 + lane < p.n) w[size_t(q) * p.n + lane] = x + y;
+        whole<Op, NC, kIPL>(op, lds, &r[0], &tot[0], &s[0], near, [&](int q, T x) {
+            if (c0 + lane < p.n) w[size_t(q) * p.n + lane] = x;
         });
     }
     double *w = rowrec + size_t(wi) * kNC * kRows + lane;

@@ -120,10 +120,15 @@ struct PassF64 {
     using T = double;
     using V = double2;
     static constexpr int W = 4;  // LDS words of a column: (x y), (z m), (vx vy), (vz -)
-    // tiles a lane's plain sums run over before they are folded (256 pairs)
-    static constexpr int kFold = 4;
+    // tiles a lane's plain sums run over before they are folded: 64 pairs below
+    // 50000 particles, 256 above, where the many partial sums' roundings average
+    // out (the pair by pair kernels: 128 and 256).  Root mean square error over
+    // theirs, acc / jerk / pot: 0.87 / 0.82 / 0.76 at N = 20000 (256 pairs and
+    // columns' sums of a whole tile: 1.11 / 1.07 / 1.21), 0.90 / 0.83 / 0.87 at 65536.
+    template <int IPL>
+    static constexpr int kFold = IPL == 2 ? 1 : 4;
     static constexpr int kSum = 2, kRow = 16;  // values of a row's sum, of its record
-    // the columns' sums continue on from lane to lane (plain sums of 64 IPL
+    // the columns' sums continue on from lane to lane (plain sums of kSeg IPL
     // terms): a rotation moves 64-bit values and does not fuse with an add
     static constexpr bool kChain = true;
 
@@ -190,6 +195,7 @@ struct PassMx {
     using T = float;
     using V = float4;
     static constexpr int W = 3;  // (hx hy hz m), (lx ly lz vx), (vy vz - -)
+    template <int IPL>
     static constexpr int kFold = 1;
     static constexpr int kSum = 1, kRow = 9;
     static constexpr bool kChain = false;
@@ -264,6 +270,7 @@ struct PassMx {
     }
 };
 
+// The 64 steps of a tile; acc: its columns' sums (g6s::settle) and smallest r^2.
 template <class Op, int IPL, bool BOTH, class Row, int TW>
 __device__ __forceinline__ void pass_steps(const typename Op::V (&tile)[TW][2 * kCol],
                                            typename Op::T (&acc)[8][kCol], typename Op::T eps2,
@@ -271,38 +278,41 @@ __device__ __forceinline__ void pass_steps(const typename Op::V (&tile)[TW][2 * 
                                            typename Op::T (&s)[IPL][7], typename Op::T (&rm)[IPL])
 {
     using T = typename Op::T;
+    constexpr int kStep = BOTH ? g6s::kSeg : kCol;
     const int lane = threadIdx.x & 63;
     T u[8];
-#pragma unroll
-    for (int q = 0; q < 7; q++) u[q] = T(0);
     u[7] = T(__builtin_inf());
+    if (BOTH) g6s::put_zero<7>(acc);
 #pragma unroll 1
-    for (int k = 0; k < kCol; k++) {
-        typename Op::V c[Op::W];
+    for (int k0 = 0; k0 < kCol; k0 += kStep) {
 #pragma unroll
-        for (int w = 0; w < Op::W; w++) c[w] = tile[w][lane + k];
-        const int j = col0 + ((lane + k) & 63);
-        T z[8];
-        if (BOTH && Op::kChain) {
+        for (int q = 0; q < 7; q++) u[q] = T(0);
+#pragma unroll 1
+        for (int k = k0; k < k0 + kStep; k++) {
+            typename Op::V c[Op::W];
 #pragma unroll
-            for (int q = 0; q < 8; q++) z[q] = g6s::from_next_lane(u[q]);
+            for (int w = 0; w < Op::W; w++) c[w] = tile[w][lane + k];
+            const int j = col0 + ((lane + k) & 63);
+            T z[8];
+            if (BOTH && Op::kChain) {
+#pragma unroll
+                for (int q = 0; q < 8; q++) z[q] = g6s::from_next_lane(u[q]);
+            }
+            Op::template pair<BOTH, !Op::kChain>(r[0], c, eps2, j == row0 + lane, s[0], rm[0], z, z[7]);
+#pragma unroll
+            for (int q = 1; q < IPL; q++)
+                Op::template pair<BOTH, false>(r[q], c, eps2, j == row0 + lane + kCol * q, s[q],
+                                               rm[q], z, z[7]);
+            if (BOTH) {
+#pragma unroll
+                for (int q = 0; q < 7; q++)
+                    u[q] = Op::kChain ? z[q] : z[q] + g6s::from_next_lane(u[q]);
+                u[7] = Op::kChain ? z[7] : vmin(z[7], g6s::from_next_lane(u[7]));
+            }
         }
-        Op::template pair<BOTH, !Op::kChain>(r[0], c, eps2, j == row0 + lane, s[0], rm[0], z, z[7]);
-#pragma unroll
-        for (int q = 1; q < IPL; q++)
-            Op::template pair<BOTH, false>(r[q], c, eps2, j == row0 + lane + kCol * q, s[q],
-                                           rm[q], z, z[7]);
-        if (BOTH) {
-#pragma unroll
-            for (int q = 0; q < 7; q++)
-                u[q] = Op::kChain ? z[q] : z[q] + g6s::from_next_lane(u[q]);
-            u[7] = Op::kChain ? z[7] : vmin(z[7], g6s::from_next_lane(u[7]));
-        }
+        if (BOTH) g6s::settle<7>(acc, k0 + kStep - 1, u);
     }
-    if (BOTH) {
-#pragma unroll
-        for (int q = 0; q < 8; q++) acc[q][lane] = g6s::from_next_lane(u[q]);
-    }
+    if (BOTH) acc[7][lane] = g6s::from_next_lane(u[7]);
 }
 
 template <class Op, int IPL>
@@ -416,7 +426,7 @@ __global__ void __launch_bounds__(kWG, (sizeof(typename Op::T) == 8 ? 2 : IPL ==
                 if (col0 + e < p.n) cr[size_t(f) * p.n + col0 + e] = v;
             }
         }
-        if (++tiles == Op::kFold) {
+        if (++tiles == Op::template kFold<IPL>) {
             tiles = 0;
             fold();
         }

@@ -137,41 +137,75 @@ __device__ __forceinline__ void load_values(const Op &op, int j, int n, T (&f)[O
 template <class T, class Op>
 constexpr int kWords = (Op::NV + Word<T>::n - 1) / Word<T>::n;
 
+// Steps between two settlements of the columns' travelling sums, each of IPL
+// terms: plain sums of 16 to 64 terms and three additions more per tile, where
+// the pair by pair kernels fold plain sums of 64 (FP32 and the FP64
+// differentiable sums) or 32 (FP64 clusters) terms.  Settled once a tile, their
+// error was up to 1.2 times that of those kernels (pot of clusters and full
+// passes); now it is no larger (tests/test_gpu_rounding.py).  1-3 % of a pass:
+// FP32 forward n = 16384 125.7 -> 127.7 us, FP64 adjoint 542 -> 553 us.
+constexpr int kSeg = 16;
+
+// Settles the columns' sums u after step k of a tile, lane l holding those of
+// column (l + k) mod 64: added to put[sum][column] (put_zero before a tile's
+// first; all read before the first is written, so one LDS round trip).  put is
+// the wave's own LDS and its LDS operations are in order: the fences only keep
+// the compiler from moving them across each other.
+template <int NC, class T>
+__device__ __forceinline__ void put_zero(T (*put)[kCol])
+{
+#pragma unroll
+    for (int q = 0; q < NC; q++) put[q][threadIdx.x & 63] = T(0);
+}
+template <int NC, class T>
+__device__ __forceinline__ void settle(T (*put)[kCol], int k, const T *u)
+{
+    const int e = ((threadIdx.x & 63) + k) & 63;
+    T had[NC];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int q = 0; q < NC; q++) had[q] = put[q][e];
+#pragma unroll
+    for (int q = 0; q < NC; q++) put[q][e] = had[q] + u[q];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
 // The 64 steps of a tile whose column c is stored at entries c and c + 64, so
-// that column (l + k) mod 64 is entry l + k.  The columns' sums u travel from
-// lane to lane and are back in their columns' own lanes at the end.
+// that column (l + k) mod 64 is entry l + k.  The columns' sums travel from
+// lane to lane and are settled in `put`.
 template <class T, class Op, int IPL, bool BOTH, int W>
 __device__ __forceinline__ void sym_steps(const Op &op, const typename Word<T>::type (&tile)[W][2 * kCol],
-                                          int col0, int row0, const T (&r)[IPL][Op::NV],
-                                          T (&s)[IPL][Op::NC], T (&u)[Op::NC])
+                                          T (*put)[kCol], int col0, int row0,
+                                          const T (&r)[IPL][Op::NV], T (&s)[IPL][Op::NC])
 {
-    constexpr int N = Word<T>::n;
+    constexpr int N = Word<T>::n, kStep = BOTH ? kSeg : kCol;
     const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int q = 0; q < Op::NC; q++) u[q] = T(0);
+    T u[Op::NC];
 #pragma unroll 1
-    for (int k = 0; k < kCol; k++) {
-        T c[W * N], z[Op::NC];
+    for (int k0 = 0; k0 < kCol; k0 += kStep) {
 #pragma unroll
-        for (int w = 0; w < W; w++) {
-            const auto e = tile[w][lane + k];
-            const T *f = reinterpret_cast<const T *>(&e);
+        for (int q = 0; q < Op::NC; q++) u[q] = T(0);
+#pragma unroll 1
+        for (int k = k0; k < k0 + kStep; k++) {
+            T c[W * N], z[Op::NC];
 #pragma unroll
-            for (int q = 0; q < N; q++) c[w * N + q] = f[q];
+            for (int w = 0; w < W; w++) {
+                const auto e = tile[w][lane + k];
+                const T *f = reinterpret_cast<const T *>(&e);
+#pragma unroll
+                for (int q = 0; q < N; q++) c[w * N + q] = f[q];
+            }
+            const int j = col0 + ((lane + k) & 63);
+            op.template pair<BOTH, true>(r[0], c, j == row0 + lane, s[0], z);
+#pragma unroll
+            for (int q = 1; q < IPL; q++)
+                op.template pair<BOTH, false>(r[q], c, j == row0 + lane + 64 * q, s[q], z);
+            if (BOTH) {
+#pragma unroll
+                for (int q = 0; q < Op::NC; q++) u[q] = z[q] + from_next_lane(u[q]);
+            }
         }
-        const int j = col0 + ((lane + k) & 63);
-        op.template pair<BOTH, true>(r[0], c, j == row0 + lane, s[0], z);
-#pragma unroll
-        for (int q = 1; q < IPL; q++)
-            op.template pair<BOTH, false>(r[q], c, j == row0 + lane + 64 * q, s[q], z);
-        if (BOTH) {
-#pragma unroll
-            for (int q = 0; q < Op::NC; q++) u[q] = z[q] + from_next_lane(u[q]);
-        }
-    }
-    if (BOTH) {
-#pragma unroll
-        for (int q = 0; q < Op::NC; q++) u[q] = from_next_lane(u[q]);
+        if (BOTH) settle<Op::NC>(put, k0 + kStep - 1, u);
     }
 }
 
@@ -188,8 +222,14 @@ __global__ void __launch_bounds__(kWG) k_sym(Plan p, Op op, double *__restrict__
     using V = typename Word<T>::type;
     constexpr int W = kWords<T, Op>, NC = Op::NC, R = kCol * IPL, N = Word<T>::n;
     __shared__ union {
-        V tile[kWaves][W][2 * kCol];  // each wave's own tile
-        double sum[kWaves][NC][R];    // then the waves' row sums
+        // each wave's own tile and its columns' sums, on 2 KB boundaries (with
+        // an address register more the compiler takes the FP32 forward's two
+        // rows one after the other: n = 8192 56.3 us, not 49.7)
+        struct alignas(2048) {
+            V tile[W][2 * kCol];
+            T put[NC][kCol];
+        } wave[kWaves];
+        double sum[kWaves][NC][R];  // then the waves' row sums
     } sh;
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int b = blockIdx.x / p.parts, u0 = (blockIdx.x - b * p.parts) * p.per;
@@ -204,7 +244,8 @@ __global__ void __launch_bounds__(kWG) k_sym(Plan p, Op op, double *__restrict__
     Long<T> tot[IPL][NC];
 #pragma unroll
     for (int i = 0; i < IPL; i++) load_values<T, Op>(op, row0 + lane + kCol * i, p.n, r[i]);
-    auto &tile = sh.tile[wave];
+    auto &tile = sh.wave[wave].tile;
+    auto &put = sh.wave[wave].put;
     load_values<T, Op>(op, column(u0 + wave) + lane, p.n, pre);
     for (int u = u0 + wave; u < u1; u += kWaves) {
         const int col0 = column(u);
@@ -224,27 +265,26 @@ __global__ void __launch_bounds__(kWG) k_sym(Plan p, Op op, double *__restrict__
             tile[w][lane] = e;
             tile[w][lane + kCol] = e;
         }
+        put_zero<NC>(put);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         load_values<T, Op>(op, column(u + kWaves) + lane, p.n, pre);
 #pragma unroll
         for (int i = 0; i < IPL; i++)
 #pragma unroll
             for (int k = 0; k < NC; k++) s[i][k] = T(0);
-        T c[NC];
-        if (u >= IPL) {
-            sym_steps<T, Op, IPL, true>(op, tile, col0, row0, r, s, c);
-            if (col0 + lane < p.n) {
-#pragma unroll
-                for (int k = 0; k < NC; k++)
-                    colpart[p.col_at(u / IPL, NC, k, col0 + lane)] = c[k];
-            }
-        } else {
-            sym_steps<T, Op, IPL, false>(op, tile, col0, row0, r, s, c);
-        }
+        if (u >= IPL)
+            sym_steps<T, Op, IPL, true>(op, tile, put, col0, row0, r, s);
+        else
+            sym_steps<T, Op, IPL, false>(op, tile, put, col0, row0, r, s);
 #pragma unroll
         for (int i = 0; i < IPL; i++)
 #pragma unroll
             for (int k = 0; k < NC; k++) tot[i][k].add(s[i][k]);
+        if (u >= IPL && col0 + lane < p.n) {
+#pragma unroll
+            for (int k = 0; k < NC; k++)
+                colpart[p.col_at(u / IPL, NC, k, col0 + lane)] = put[k][lane];
+        }
     }
     // the waves' row sums, added in wave order
     __syncthreads();
