@@ -87,8 +87,8 @@ struct Dev {
     unsigned int *bar = nullptr;  // grid barrier of kc_run (g6bar::kWords, zero at each launch)
     int fill_target = 512;  // items a rebuilt list aims at (see build_items)
     // Pair-once clusters (g6_cluster_pairs.h): those of the classes in
-    // pair_class whose records start at ws[ws_at[c]] (ws_at < 0: too large for
-    // it), while the list's boost is 1.  boost: of the current host-built list.
+    // pair_class whose records start at ws[ws_at[c]] (ws_at < 0: not taken so),
+    // while the list's boost is 1.  boost: of the current host-built list.
     double *ws = nullptr;
     long long *ws_at = nullptr;
     int pair_per = 1;  // units per wave
@@ -106,9 +106,16 @@ __host__ __device__ inline int size_class_d(int n)
 }
 
 // Whether cluster c of n particles is taken pair-once in a list of this boost.
+// One value for its callers' branches (the empty asm keeps it so): with a
+// branch for each part, the compiler (hipcc 7.2) left the axis that
+// correct_axis indexes the state by unset on the last part's edge, where the
+// class is taken pair-once and the cluster is not, and kc_run_pairs read the
+// state's addresses from behind its arguments.
 __device__ __forceinline__ bool pair_once(const Dev &d, int c, int n, int boost)
 {
-    return boost == 1 && ((d.pair_class >> size_class_d(n)) & 1) && d.ws_at[c] >= 0;
+    int once = boost == 1 && ((d.pair_class >> size_class_d(n)) & 1) && d.ws_at[c] >= 0;
+    asm volatile("" : "+v"(once));
+    return once != 0;
 }
 
 // Work items of a pair-once cluster: four waves each, and never fewer than
@@ -972,10 +979,11 @@ int auto_njs(int k) { return k <= 1 ? 16 : (k <= 3 ? 4 : 1); }
 // Classes taken pair-once: from kPairClass on, while their shape is the
 // automatic one (a shape that was set or tuned is taken as asked).  Up to 128
 // particles a cluster is one block with one busy wave.  Records grow as n^2
-// (8192 particles: 130 MB), and a larger cluster has rows enough for the
-// other kernels.
+// (8192 particles: 45 MB), and a larger cluster has rows enough to go pair by
+// pair beside the others.
 constexpr int kPairClass = 4;      // clusters of more than 128
 constexpr int kPairMaxN = 8192;
+bool pair_size(int n) { return size_class(n) >= kPairClass && n <= kPairMaxN; }
 void pair_rule(Ensemble *E)
 {
     E->d.pair_class = 0;
@@ -989,15 +997,13 @@ void pair_rule(Ensemble *E)
 // (1 against the 3 that four waves allow: a round of 512 clusters mixed 221 ->
 // 208 us, of 350 in FP64 245 -> 234; 2 and 3 are the slower ones everywhere
 // below).
-// With a cluster above kPairMaxN, or without room for the records every cluster keeps the other kernels.
+// Without room for the records every cluster keeps the other kernels.
 bool pair_setup(Ensemble *E, int cus)
 {
     Dev &d = E->d;
     long long units = 0;
-    for (int n : E->cnt) {
-        if (n > kPairMaxN) return true;
-        if (size_class(n) >= kPairClass) units += g6cp::Plan(n, 1).work();
-    }
+    for (int n : E->cnt)
+        if (pair_size(n)) units += g6cp::Plan(n, 1).work();
     if (units == 0) return true;
     d.pair_per = int(std::min(4ll, std::max(1ll, units / (64 * cus))));
     d.pair_fill = 4 * cus;
@@ -1005,7 +1011,7 @@ bool pair_setup(Ensemble *E, int cus)
     long long at = 0;
     for (int c = 0; c < d.nc; c++) {
         const int n = E->cnt[c];
-        if (size_class(n) < kPairClass) continue;
+        if (!pair_size(n)) continue;
         E->ws_at[c] = at;
         at += (g6cp::Plan(n, d.pair_per).values() + 31) / 32 * 32;
     }

@@ -357,3 +357,43 @@ def test_pair_once_clusters(prec, sizes):
     for other in states[1:]:
         for q, r in zip(states[0], other):
             assert np.array_equal(q, r)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("sizes", [(8193, 40, 200), (2049, 8193, 1025)])
+def test_clusters_beyond_pair_once(prec, sizes):
+    """A cluster too large to be taken pair by unordered pair in a class whose
+    other clusters are, beside one of those: sampled forces against the 80-bit
+    oracle within the bounds of test_ensemble_forces, and the step rounds of
+    the three run modes bit for bit."""
+    from amuse_amd import ic
+    rng = np.random.Generator(np.random.PCG64(sum(sizes)))
+    counts = np.array(sizes, dtype=np.int32)
+    total = int(counts.sum())
+    _, x, v = ic.plummer_raw(total, rng)
+    x, v = ic.to_nbody_units(x, v)
+    m = rng.uniform(0.5, 1.5, total)
+    states = []
+    for mode in ("eager", "graph", "persistent"):
+        print_case(f"beyond pair-once {sizes} prec={prec} {mode}")
+        ens = Ensemble(counts, m, x, v, eps2=EPS2, dt_param=DTP, precision=prec)
+        if mode == "eager":
+            a, j, p = ens.forces(prec)
+            for n, sl in zip(counts, per_cluster(counts)):
+                ids = np.arange(n, dtype=np.int32)
+                row = np.unique(np.r_[0:3, 63:66, 127:130, n // 2, n - 3:n] % n)
+                ea, ej, ep, sa, sj, sp = oracle.force_ld(ids[row], x[sl][row], v[sl][row], EPS2, ids,
+                                                         m[sl], x[sl], v[sl])
+                for val, ex, s, tol in ((a[sl][row], ea, sa, (1e-15, 2e-6)),
+                                        (j[sl][row], ej, sj, (4e-15, 1e-5)),
+                                        (p[sl][row], ep, sp, (1e-15, 2e-6))):
+                    d = np.abs(val - ex).reshape(len(s), -1).max(1)
+                    assert (d <= tol[prec] * s).all(), (n, (d / s).max())
+        ens.start(1.0)
+        ens.run(steps_per_graph=2, use_graph=mode == "graph", max_rounds=4,
+                persistent=mode == "persistent")
+        states.append(ens.state())
+        ens.close()
+    for other in states[1:]:
+        for q, r in zip(states[0], other):
+            assert np.array_equal(q, r)
