@@ -17,8 +17,9 @@
 //             (double-single dx, FP32 r^-3, compensated sums) or FP64; the
 //             inverse quartic collision time max(v^4/s^2, m_ij^2 r^2/s^4) is
 //             reduced per cluster with an atomic maximum; clusters of more
-//             than 128 particles are taken pair by unordered pair
-//             (g6_cluster_pairs.h) while there is work for the whole chip
+//             than 192 particles are taken pair by unordered pair
+//             (g6_cluster_pairs.h) where they weigh enough (pair_pays) and
+//             while there is work for the whole chip
 //   update    t += dt, next step from the collision time, retire clusters
 //             that reached t_end
 //   advance   the time-symmetric corrector (FP64) and the next step's
@@ -81,14 +82,14 @@ struct Dev {
     // work list of the persistent run (kc_run), built on the device: items
     // (cluster, first row, lanes per row) of the active clusters, clusters
     // taken in the order corder (largest first); ctl = {items, clusters
-    // covered, boost, built}
+    // covered, built}
     int *wl_c = nullptr, *wl_i0 = nullptr, *wl_njs = nullptr, *corder = nullptr, *ctl = nullptr;
     int wl_cap = 0;
     unsigned int *bar = nullptr;  // grid barrier of kc_run (g6bar::kWords, zero at each launch)
     int fill_target = 512;  // items a rebuilt list aims at (see build_items)
-    // Pair-once clusters (g6_cluster_pairs.h): those of the classes in
-    // pair_class whose records start at ws[ws_at[c]] (ws_at < 0: not taken so),
-    // while the list's boost is 1.  boost: of the current host-built list.
+    // Pair-once clusters (g6_cluster_pairs.h): those of pair_size in the
+    // classes of pair_class, while the list's boost is 1; their records start
+    // at ws[ws_at[c]].  boost: of the current host-built list.
     double *ws = nullptr;
     long long *ws_at = nullptr;
     int pair_per = 1;  // units per wave
@@ -105,17 +106,18 @@ __host__ __device__ inline int size_class_d(int n)
     return k;
 }
 
-// Whether cluster c of n particles is taken pair-once in a list of this boost.
-// One value for its callers' branches (the empty asm keeps it so): with a
-// branch for each part, the compiler (hipcc 7.2) left the axis that
-// correct_axis indexes the state by unset on the last part's edge, where the
-// class is taken pair-once and the cluster is not, and kc_run_pairs read the
-// state's addresses from behind its arguments.
-__device__ __forceinline__ bool pair_once(const Dev &d, int c, int n, int boost)
+// Clusters that can be taken pair-once.  Below, a second block of 128 is
+// mostly padding: us a round, pair by pair / pair-once, of 1000 clusters in FP64
+// 93 / 124 at 130 particles, 104 / 125 at 150, 126 / 131 at 190, 158 / 136 at 256, mixed
+// 70 / 82, 77 / 83, 91 / 89 and 110 / 105.  Records grow as n^2 (8192 particles: 45 MB),
+// and a larger cluster has rows enough to go pair by pair beside the others.
+constexpr int kPairMinN = 193, kPairMaxN = 8192;
+__host__ __device__ inline bool pair_size(int n) { return n >= kPairMinN && n <= kPairMaxN; }
+
+// Whether a cluster of n particles is taken pair-once in a list of this boost.
+__device__ __forceinline__ bool pair_once(const Dev &d, int n, int boost)
 {
-    int once = boost == 1 && ((d.pair_class >> size_class_d(n)) & 1) && d.ws_at[c] >= 0;
-    asm volatile("" : "+v"(once));
-    return once != 0;
+    return boost == 1 && pair_size(n) && ((d.pair_class >> size_class_d(n)) & 1);
 }
 
 // Work items of a pair-once cluster: four waves each, and never fewer than
@@ -511,7 +513,7 @@ __global__ void __launch_bounds__(256) kc_pair_sum(Dev d)
     if (q >= d.nlist) return;
     const int pt = d.plist[q];
     const int c = d.pc[pt], n = d.cnt[c];
-    if (!d.active[c] || !pair_once(d, c, n, d.boost)) return;
+    if (!d.active[c] || !pair_once(d, n, d.boost)) return;
     const g6cp::Plan p(n, d.pair_per);
     const PairRecords<MIXED> rec(d, c, p);
     const double z = g6cp::record_sum(p, rec.col, rec.row, pt - d.off[c], k);
@@ -522,16 +524,18 @@ __global__ void __launch_bounds__(256) kc_pair_sum(Dev d)
 // time-symmetric corrector (FP64), src/amuse_hermite/interface.cc:536-556
 // ---------------------------------------------------------------------------
 // One axis of a particle of cluster c, its new force from the result rows or,
-// for a pair-once cluster, from its records.
+// for a pair-once cluster (once), from its records.  once is one value that
+// the callers have: worked out here, in a branch for each part, hipcc 7.2 left k
+// unset on the last part's edge in kc_run_pairs' loop over k, and the state's
+// addresses were read from behind the kernel's arguments.
 // next: the particle's next step, to which the axis is predicted then (0: not).
 template <bool MIXED, bool PAIRS>
-__device__ __forceinline__ void correct_axis(const Dev &d, int p, int c, double dt, int boost, int k,
+__device__ __forceinline__ void correct_axis(const Dev &d, int p, int c, double dt, bool once, int k,
                                              double next)
 {
-    const int n = d.cnt[c];
     double na, nj;
-    if (PAIRS && pair_once(d, c, n, boost)) {
-        const g6cp::Plan pl(n, d.pair_per);
+    if (PAIRS && once) {
+        const g6cp::Plan pl(d.cnt[c], d.pair_per);
         const PairRecords<MIXED> rec(d, c, pl);
         na = g6cp::record_sum(pl, rec.col, rec.row, p - d.off[c], k);
         nj = g6cp::record_sum(pl, rec.col, rec.row, p - d.off[c], 3 + k);
@@ -565,7 +569,8 @@ __global__ void __launch_bounds__(256) kc_advance(Dev d)
     const int c = d.pc[p];
     const double dt = d.taken[c];
     if (dt == 0.0) return;
-    correct_axis<MIXED, PAIRS>(d, p, c, dt, d.boost, blockIdx.y, d.active[c] ? d.dt[c] : 0.0);
+    correct_axis<MIXED, PAIRS>(d, p, c, dt, PAIRS && pair_once(d, d.cnt[c], d.boost), blockIdx.y,
+                               d.active[c] ? d.dt[c] : 0.0);
 }
 
 // first forces of each cluster become its current acc and jerk
@@ -764,7 +769,7 @@ __device__ void build_work_list(const Dev &d, int fill, int *red)
         int units = 0;
         for (int k = c0; k < c1; k++) {
             const int c = d.corder[k], n = d.cnt[c];
-            if (d.active[c] && pair_once(d, c, n, 1)) units += int(g6cp::Plan(n, d.pair_per).work());
+            if (d.active[c] && pair_once(d, n, 1)) units += int(g6cp::Plan(n, d.pair_per).work());
         }
         if (wg_sum(units, red) >= d.pair_fill) fill = 0;
     }
@@ -791,7 +796,7 @@ __device__ void build_work_list(const Dev &d, int fill, int *red)
         const int c = d.corder[k];
         if (!d.active[c]) continue;
         const int n = d.cnt[c], rows = kWG / lanes_of(d, n, boost);
-        mine += PAIRS && pair_once(d, c, n, boost) ? pair_items(n, d.pair_per) : (n + rows - 1) / rows;
+        mine += PAIRS && pair_once(d, n, boost) ? pair_items(n, d.pair_per) : (n + rows - 1) / rows;
     }
     int incl = mine;
     const int lane = t & 63;
@@ -811,7 +816,7 @@ __device__ void build_work_list(const Dev &d, int fill, int *red)
         const int c = d.corder[k];
         if (!d.active[c]) continue;
         const int n = d.cnt[c], njs = lanes_of(d, n, boost), rows = kWG / njs;
-        if (PAIRS && pair_once(d, c, n, boost)) {
+        if (PAIRS && pair_once(d, n, boost)) {
             const int items = pair_items(n, d.pair_per);
             for (int i = 0; i < items && at < d.wl_cap; i++, at++) {
                 d.wl_c[at] = c;
@@ -829,21 +834,21 @@ __device__ void build_work_list(const Dev &d, int fill, int *red)
     if (t == 0) {
         d.ctl[0] = min(total, d.wl_cap);
         d.ctl[1] = covered;
-        d.ctl[2] = boost;
-        d.ctl[3] = 1;
+        d.ctl[2] = 1;
     }
     __syncthreads();
 }
 
 // Rows of work item `it`: the particles of (cluster, i0 .. i0 + kWG/njs - 1),
-// or the k-th kWG particles of a pair-once cluster.
+// or the k-th kWG particles of a pair-once cluster (once).
 template <bool PAIRS>
-__device__ __forceinline__ int item_particle(const Dev &d, int it, int t, int &c)
+__device__ __forceinline__ int item_particle(const Dev &d, int it, int t, int &c, bool &once)
 {
     c = d.wl_c[it];
     const int njs = d.wl_njs[it];
-    const int i = d.wl_i0[it] * (PAIRS && !njs ? kWG : 1) + t;
-    if (t >= (PAIRS && !njs ? kWG : kWG / njs) || i >= d.cnt[c]) return -1;
+    once = PAIRS && !njs;
+    const int i = d.wl_i0[it] * (once ? kWG : 1) + t;
+    if (t >= (once ? kWG : kWG / njs) || i >= d.cnt[c]) return -1;
     return d.off[c] + i;
 }
 
@@ -860,7 +865,7 @@ __device__ __forceinline__ void run_rounds(const Dev &d, long long max_rounds,
     // The list state as every workgroup keeps it in registers: read by all
     // before the barrier, written (by workgroup 0, in a rebuild) only after
     // it, and read again after each rebuild's own barrier.
-    int built = load_shared_int(&d.ctl[3]);
+    int built = load_shared_int(&d.ctl[2]);
     int covered = load_shared_int(&d.ctl[1]);
     bool ok = grid_barrier(d.bar, gen++);
     while (ok) {
@@ -873,12 +878,13 @@ __device__ __forceinline__ void run_rounds(const Dev &d, long long max_rounds,
             built = 1;
             covered = load_shared_int(&d.ctl[1]);
         }
-        const int nwork = load_shared_int(&d.ctl[0]), boost = load_shared_int(&d.ctl[2]);
+        const int nwork = load_shared_int(&d.ctl[0]);
         // predict (and reset the force queue)
         if (blockIdx.x == 0 && t == 0) *d.queue = 0;
         for (int it = blockIdx.x; it < nwork; it += gridDim.x) {
             int c;
-            const int p = item_particle<PAIRS>(d, it, t, c);
+            bool once;
+            const int p = item_particle<PAIRS>(d, it, t, c, once);
             if (p >= 0 && d.active[c]) predict_particle(d, p, d.dt[c]);
         }
         if (!grid_barrier(d.bar, gen++)) break;
@@ -897,15 +903,16 @@ __device__ __forceinline__ void run_rounds(const Dev &d, long long max_rounds,
         // correct
         for (int it = blockIdx.x; it < nwork; it += gridDim.x) {
             int c;
-            const int p = item_particle<PAIRS>(d, it, t, c);
+            bool once;
+            const int p = item_particle<PAIRS>(d, it, t, c, once);
             if (p >= 0 && d.active[c]) {
                 const double dt = d.dt[c];
                 if constexpr (PAIRS) {
 #pragma unroll 1
-                    for (int k = 0; k < 3; k++) correct_axis<MIXED, PAIRS>(d, p, c, dt, boost, k, 0.0);
+                    for (int k = 0; k < 3; k++) correct_axis<MIXED, PAIRS>(d, p, c, dt, once, k, 0.0);
                 } else {
 #pragma unroll
-                    for (int k = 0; k < 3; k++) correct_axis<MIXED, PAIRS>(d, p, c, dt, boost, k, 0.0);
+                    for (int k = 0; k < 3; k++) correct_axis<MIXED, PAIRS>(d, p, c, dt, false, k, 0.0);
                 }
             }
         }
@@ -929,7 +936,8 @@ __global__ void __launch_bounds__(kWG, MIXED ? 5 : 4) kc_run(Dev d, long long ma
     });
 }
 
-// For ensembles with pair-once clusters (bounds: no spills to scratch).
+// For ensembles with pair-once clusters (bounds: no spills to scratch, which
+// leaves FP64 one wave a SIMD: kOthersMax).
 template <bool MIXED>
 __global__ void __launch_bounds__(kWG, MIXED ? 3 : 1)
 kc_run_pairs(Dev d, long long max_rounds, long long *rounds_out)
@@ -955,7 +963,6 @@ struct Ensemble {
     void *base = nullptr;
     int precision = 1;
     std::vector<int> cnt, off;
-    std::vector<long long> ws_at;  // as Dev::ws_at
     int ib_rows = 0;
     int persistent_wgs = 0;
     hipGraphExec_t graph = nullptr;
@@ -966,6 +973,7 @@ struct Ensemble {
     int *h_active = nullptr;  // the active count, read back after each launch (pinned)
     double *aos = nullptr;    // [6][np]: x and v as the caller's arrays lay them out
     void *pair_base = nullptr;  // the pair-once clusters' record offsets, then the records
+    double pairs = 0.0, others = 0.0;  // as pair_pays counts them
     double force_ms = 0.0;
     long long launches = 0;
     std::string err;
@@ -977,17 +985,48 @@ int size_class(int n) { return size_class_d(n); }
 int auto_njs(int k) { return k <= 1 ? 16 : (k <= 3 ? 4 : 1); }
 
 // Classes taken pair-once: from kPairClass on, while their shape is the
-// automatic one (a shape that was set or tuned is taken as asked).  Up to 128
-// particles a cluster is one block with one busy wave.  Records grow as n^2
-// (8192 particles: 45 MB), and a larger cluster has rows enough to go pair by
-// pair beside the others.
-constexpr int kPairClass = 4;      // clusters of more than 128
-constexpr int kPairMaxN = 8192;
-bool pair_size(int n) { return size_class(n) >= kPairClass && n <= kPairMaxN; }
+// automatic one (a shape that was set or tuned is taken as asked).
+constexpr int kPairClass = 4;
+
+// Whether an ensemble's pair-once clusters are taken so.  The kernels that
+// hold both kinds of items have half the waves of the others, which costs the
+// clusters that are not taken pair-once up to 8 %, so those that are have to
+// weigh something (ordered pairs an eighth of the others'), or the largest to
+// be the longest item of a round, a row's serial chain.  us a round in FP64,
+// pair by pair / pair-once, beside 4096 clusters of 16..128: one of 200 127 / 138, 32 of
+// 200 132 / 141, one of 500 131 / 138, 16 of 500 212 / 146, one of 1000 238 / 143;
+// beside 16384 of them: one of 1000 419 / 457, 8 of 1000 482 / 466, one of 2048 581 / 462;
+// beside 1000: one of 200 60 / 54.
+bool pair_pays(const std::vector<int> &cnt, double &pairs, double &others)
+{
+    int most = 0;
+    pairs = others = 0.0;
+    for (int n : cnt) {
+        (pair_size(n) ? pairs : others) += double(n) * n;
+        if (pair_size(n)) most = std::max(most, n);
+    }
+    return 8.0 * pairs > others || most > 80 + others / 34000.0;
+}
+
+// In FP64 the persistent kernel for both kinds has a quarter of kc_run's waves,
+// so from kOthersMax ordered pairs of the others on the pair-once ones have to
+// be two thirds as many, or every cluster is taken pair by pair: in each run
+// mode, since these give the same bits.  Persistent, pair by pair / pair-once:
+// 8 of 1000 beside 4096 of 16..128 (16 million) 494 / 371, beside 16384 (64
+// million) 738 / 1293, 8 of 2048 beside these 1009 / 1363; beside 12000 (46
+// million) 8 of 2048 929 / 993, 40 of 2048 1185 / 1260, where the steps one by
+// one or in graphs (both kernels at half their waves) take 744 / 383, 959 / 557.
+constexpr double kOthersMax = 2.4e7;
+bool pair_pays_fp64(double pairs, double others)
+{
+    return others < kOthersMax || 3.0 * pairs > 2.0 * others;
+}
+
 void pair_rule(Ensemble *E)
 {
     E->d.pair_class = 0;
-    if (!E->pair_base) return;
+    if (!E->pair_base || (E->precision == G6X_FP64 && !pair_pays_fp64(E->pairs, E->others)))
+        return;
     for (int k = kPairClass; k < kClasses; k++)
         if (E->d.njs_class[k] == auto_njs(k) && E->d.tj_class[k] == kTJ) E->d.pair_class |= 1 << k;
 }
@@ -1004,27 +1043,26 @@ bool pair_setup(Ensemble *E, int cus)
     long long units = 0;
     for (int n : E->cnt)
         if (pair_size(n)) units += g6cp::Plan(n, 1).work();
-    if (units == 0) return true;
+    if (units == 0 || !pair_pays(E->cnt, E->pairs, E->others)) return true;
     d.pair_per = int(std::min(4ll, std::max(1ll, units / (64 * cus))));
     d.pair_fill = 4 * cus;
-    E->ws_at.assign(d.nc, -1);
+    std::vector<long long> ws_at(d.nc, -1);
     long long at = 0;
     for (int c = 0; c < d.nc; c++) {
         const int n = E->cnt[c];
         if (!pair_size(n)) continue;
-        E->ws_at[c] = at;
+        ws_at[c] = at;
         at += (g6cp::Plan(n, d.pair_per).values() + 31) / 32 * 32;
     }
     const size_t head = (size_t(d.nc) * sizeof(long long) + 255) / 256 * 256;
     if (hipMalloc(&E->pair_base, head + size_t(at) * sizeof(double)) != hipSuccess) {
         (void)hipGetLastError();
         E->pair_base = nullptr;
-        E->ws_at.clear();
         return true;
     }
     d.ws_at = static_cast<long long *>(E->pair_base);
     d.ws = reinterpret_cast<double *>(static_cast<char *>(E->pair_base) + head);
-    return hipMemcpy(d.ws_at, E->ws_at.data(), size_t(d.nc) * sizeof(long long),
+    return hipMemcpy(d.ws_at, ws_at.data(), size_t(d.nc) * sizeof(long long),
                      hipMemcpyHostToDevice) == hipSuccess;
 }
 
@@ -1069,7 +1107,7 @@ int build_items(Ensemble *E, const int *only = nullptr, bool fill = false)
     long long units = 0;
     pair_rule(E);
     auto pair = [&](int c) {
-        return boost == 1 && !E->ws_at.empty() && E->ws_at[c] >= 0 &&
+        return boost == 1 && pair_size(E->cnt[c]) &&
                ((E->d.pair_class >> size_class(E->cnt[c])) & 1);
     };
     for (int c = 0; c < E->d.nc; c++)
@@ -1348,7 +1386,7 @@ G6C_API void *g6c_create(int nc, const int counts[], const double m[], const dou
 static int invalidate_work_list(Ensemble *E)
 {
     const int zero = 0;
-    CK(hipMemcpyAsync(E->d.ctl + 3, &zero, sizeof(int), hipMemcpyHostToDevice, E->stream));
+    CK(hipMemcpyAsync(E->d.ctl + 2, &zero, sizeof(int), hipMemcpyHostToDevice, E->stream));
     CK(hipStreamSynchronize(E->stream));
     return 0;
 }
@@ -1721,7 +1759,11 @@ G6C_API int g6c_set_precision(void *h, int precision)
     Ensemble *E = static_cast<Ensemble *>(h);
     if (precision != G6X_FP64 && precision != G6X_MIXED) return G6X_ERR_ARG;
     E->precision = precision;
-    return 0;
+    const int was = E->d.pair_class;
+    pair_rule(E);
+    if (E->d.pair_class == was) return 0;
+    if (invalidate_work_list(E)) return G6X_ERR_HIP;
+    return build_items(E);
 }
 
 G6C_API double g6c_elapsed_ms(void *h) { return static_cast<Ensemble *>(h)->force_ms; }

@@ -360,7 +360,7 @@ def test_pair_once_clusters(prec, sizes):
 
 
 @pytest.mark.parametrize("prec", [0, 1])
-@pytest.mark.parametrize("sizes", [(8193, 40, 200), (2049, 8193, 1025)])
+@pytest.mark.parametrize("sizes", [(8193, 40, 200), (2049, 8193, 1025), (8193, 4000, 200)])
 def test_clusters_beyond_pair_once(prec, sizes):
     """A cluster too large to be taken pair by unordered pair in a class whose
     other clusters are, beside one of those: sampled forces against the 80-bit
@@ -397,3 +397,36 @@ def test_clusters_beyond_pair_once(prec, sizes):
     for other in states[1:]:
         for q, r in zip(states[0], other):
             assert np.array_equal(q, r)
+
+
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("name,sizes,once", [
+    ("130 to 192 particles", (130, 150, 170, 192) * 8, False),
+    ("many small ones and one of 200", (40,) * 4096 + (200,), False),
+    ("many small ones and 8 of 1000", (40,) * 4096 + (1000,) * 8, True),
+    ("193 particles", (193, 193, 40), True),
+    ("one above 8192 and one of 4000", (8193, 4000), "mixed")])
+def test_where_pairs_are_taken_once(prec, name, sizes, once):
+    """Clusters are taken pair by unordered pair only where that is the faster
+    way: elsewhere the automatic shapes give the bits of the pair by pair
+    kernels (asked for by a j-tile of another size, which leaves their order
+    of additions alone), whose registers let twice the waves run."""
+    from amuse_amd import ic
+    rng = np.random.Generator(np.random.PCG64(len(sizes)))
+    counts = np.array(sizes, dtype=np.int32)
+    total = int(counts.sum())
+    _, x, v = ic.plummer_raw(total, rng)
+    x, v = ic.to_nbody_units(x, v)
+    m = rng.uniform(0.5, 1.5, total)
+    print_case(f"pair-once or not: {name} prec={prec}")
+    res = []
+    for asked, made in ((False, prec), (True, prec), (False, 1 - prec)):
+        ens = Ensemble(counts, m, x, v, eps2=EPS2, dt_param=DTP, precision=made)
+        if asked:
+            ens.set_jtiles([128] * 8)
+        ens.set_precision(prec)
+        res.append(ens.forces(prec))
+        ens.close()
+    same = all(np.array_equal(a, b) for a, b in zip(*res[:2]))
+    assert same == (not once or (once == "mixed" and prec == 0))
+    assert all(np.array_equal(a, b) for a, b in zip(*res[::2]))
