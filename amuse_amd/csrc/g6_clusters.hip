@@ -94,6 +94,7 @@ struct Dev {
     long long *ws_at = nullptr;
     int pair_per = 1;  // units per wave
     int pair_class = 0;  // bit k: size class k
+    int pair_max = 0;    // the largest cluster with room for its records
     int boost = 1;
     int pair_fill = 1024;  // units from which a rebuilt list keeps them
 };
@@ -112,12 +113,15 @@ __host__ __device__ inline int size_class_d(int n)
 // 70 / 82, 77 / 83, 91 / 89 and 110 / 105.  Records grow as n^2 (8192 particles: 45 MB),
 // and a larger cluster has rows enough to go pair by pair beside the others.
 constexpr int kPairMinN = 193, kPairMaxN = 8192;
-__host__ __device__ inline bool pair_size(int n) { return n >= kPairMinN && n <= kPairMaxN; }
+__host__ __device__ inline bool pair_size(const Dev &d, int n)
+{
+    return n >= kPairMinN && n <= d.pair_max;
+}
 
 // Whether a cluster of n particles is taken pair-once in a list of this boost.
 __device__ __forceinline__ bool pair_once(const Dev &d, int n, int boost)
 {
-    return boost == 1 && pair_size(n) && ((d.pair_class >> size_class_d(n)) & 1);
+    return boost == 1 && pair_size(d, n) && ((d.pair_class >> size_class_d(n)) & 1);
 }
 
 // Work items of a pair-once cluster: four waves each, and never fewer than
@@ -997,13 +1001,14 @@ constexpr int kPairClass = 4;
 // 200 132 / 141, one of 500 131 / 138, 16 of 500 212 / 146, one of 1000 238 / 143;
 // beside 16384 of them: one of 1000 419 / 457, 8 of 1000 482 / 466, one of 2048 581 / 462;
 // beside 1000: one of 200 60 / 54.
-bool pair_pays(const std::vector<int> &cnt, double &pairs, double &others)
+bool pair_pays(Ensemble *E)
 {
     int most = 0;
+    double &pairs = E->pairs, &others = E->others;
     pairs = others = 0.0;
-    for (int n : cnt) {
-        (pair_size(n) ? pairs : others) += double(n) * n;
-        if (pair_size(n)) most = std::max(most, n);
+    for (int n : E->cnt) {
+        (pair_size(E->d, n) ? pairs : others) += double(n) * n;
+        if (pair_size(E->d, n)) most = std::max(most, n);
     }
     return 8.0 * pairs > others || most > 80 + others / 34000.0;
 }
@@ -1035,24 +1040,40 @@ void pair_rule(Ensemble *E)
 // wave: as many as leave sixteen waves for each of the chip's SIMDs, at most 4
 // (1 against the 3 that four waves allow: a round of 512 clusters mixed 221 ->
 // 208 us, of 350 in FP64 245 -> 234; 2 and 3 are the slower ones everywhere
-// below).
-// Without room for the records every cluster keeps the other kernels.
+// below).  The records take at most kPairMaxBytes (382 clusters of 8192, 5700 of
+// 2048): in an ensemble with more the largest clusters keep the other kernels,
+// whose rows fill the chip then, and without room for them every cluster does.
+constexpr long long kPairMaxBytes = 8ll << 30;
+long long record_values(const Dev &d, int n)
+{
+    return (g6cp::Plan(n, d.pair_per).values() + 31) / 32 * 32;
+}
 bool pair_setup(Ensemble *E, int cus)
 {
     Dev &d = E->d;
     long long units = 0;
+    d.pair_max = kPairMaxN;
     for (int n : E->cnt)
-        if (pair_size(n)) units += g6cp::Plan(n, 1).work();
-    if (units == 0 || !pair_pays(E->cnt, E->pairs, E->others)) return true;
+        if (pair_size(d, n)) units += g6cp::Plan(n, 1).work();
+    if (units == 0) return true;
     d.pair_per = int(std::min(4ll, std::max(1ll, units / (64 * cus))));
     d.pair_fill = 4 * cus;
+    std::vector<int> sizes(E->cnt);
+    std::sort(sizes.begin(), sizes.end());
+    long long left = kPairMaxBytes / (long long)sizeof(double);
+    for (int n : sizes) {
+        if (!pair_size(d, n)) continue;
+        left -= record_values(d, n);
+        if (left < 0) d.pair_max = n - 1;
+    }
+    if (!pair_pays(E)) return true;
     std::vector<long long> ws_at(d.nc, -1);
     long long at = 0;
     for (int c = 0; c < d.nc; c++) {
         const int n = E->cnt[c];
-        if (!pair_size(n)) continue;
+        if (!pair_size(d, n)) continue;
         ws_at[c] = at;
-        at += (g6cp::Plan(n, d.pair_per).values() + 31) / 32 * 32;
+        at += record_values(d, n);
     }
     const size_t head = (size_t(d.nc) * sizeof(long long) + 255) / 256 * 256;
     if (hipMalloc(&E->pair_base, head + size_t(at) * sizeof(double)) != hipSuccess) {
@@ -1107,7 +1128,7 @@ int build_items(Ensemble *E, const int *only = nullptr, bool fill = false)
     long long units = 0;
     pair_rule(E);
     auto pair = [&](int c) {
-        return boost == 1 && pair_size(E->cnt[c]) &&
+        return boost == 1 && pair_size(E->d, E->cnt[c]) &&
                ((E->d.pair_class >> size_class(E->cnt[c])) & 1);
     };
     for (int c = 0; c < E->d.nc; c++)

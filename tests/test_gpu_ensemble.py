@@ -430,3 +430,22 @@ def test_where_pairs_are_taken_once(prec, name, sizes, once):
     same = all(np.array_equal(a, b) for a, b in zip(*res[:2]))
     assert same == (not once or (once == "mixed" and prec == 0))
     assert all(np.array_equal(a, b) for a, b in zip(*res[::2]))
+
+
+def test_pair_once_memory_is_bounded():
+    """The partial sums of the clusters taken pair by unordered pair take at
+    most 8 GiB: 500 clusters of 8192 (11.2 GB of them, beside some 1.5 GB of
+    state), whose largest are then taken as before, and so are the forces."""
+    import torch
+    counts = np.array([8192] * 500 + [300] * 4, dtype=np.int32)
+    total = int(counts.sum())
+    rng = np.random.Generator(np.random.PCG64(8192))
+    x, v = rng.standard_normal((2, total, 3))
+    m = rng.uniform(0.5, 1.5, total)
+    torch.cuda.empty_cache()
+    free = torch.cuda.mem_get_info()[0]
+    print_case("memory of 500 clusters of 8192")
+    ens = Ensemble(counts, m, x, v, eps2=EPS2, dt_param=DTP, precision=1)
+    used = free - torch.cuda.mem_get_info()[0]
+    ens.close()
+    assert used < (8 << 30) + 512 * total
