@@ -94,7 +94,7 @@ struct Dev {
     long long *ws_at = nullptr;
     int pair_per = 1;  // units per wave
     int pair_class = 0;  // bit k: size class k
-    int pair_max = 0;    // the largest cluster with room for its records
+    int pair_min = 0, pair_max = 0;  // sizes that are taken so
     int boost = 1;
     int pair_fill = 1024;  // units from which a rebuilt list keeps them
 };
@@ -107,15 +107,17 @@ __host__ __device__ inline int size_class_d(int n)
     return k;
 }
 
-// Clusters that can be taken pair-once.  Below, a second block of 128 is
-// mostly padding: us a round, pair by pair / pair-once, of 1000 clusters in FP64
+// Clusters that can be taken pair-once.  Below kPairMinN a second block of 128
+// is mostly padding: us a round, pair by pair / pair-once, of 1000 clusters in FP64
 // 93 / 124 at 130 particles, 104 / 125 at 150, 126 / 131 at 190, 158 / 136 at 256, mixed
-// 70 / 82, 77 / 83, 91 / 89 and 110 / 105.  Records grow as n^2 (8192 particles: 45 MB),
-// and a larger cluster has rows enough to go pair by pair beside the others.
-constexpr int kPairMinN = 193, kPairMaxN = 8192;
+// 70 / 82, 77 / 83, 91 / 89 and 110 / 105.  Where larger ones weigh more than they, those
+// from kPairLowN on are taken so too (100 of 16..2048 in FP64 110 -> 105).
+// Records grow as n^2 (8192 particles: 45 MB), and a larger cluster has rows
+// enough to go pair by pair beside the others.
+constexpr int kPairLowN = 129, kPairMinN = 193, kPairMaxN = 8192;
 __host__ __device__ inline bool pair_size(const Dev &d, int n)
 {
-    return n >= kPairMinN && n <= d.pair_max;
+    return n >= d.pair_min && n <= d.pair_max;
 }
 
 // Whether a cluster of n particles is taken pair-once in a list of this boost.
@@ -1052,6 +1054,10 @@ bool pair_setup(Ensemble *E, int cus)
 {
     Dev &d = E->d;
     long long units = 0;
+    double low = 0.0;
+    for (int n : E->cnt)
+        if (n >= kPairLowN && n <= kPairMaxN) low += (n < kPairMinN ? 1.0 : -1.0) * n * n;
+    d.pair_min = low < 0.0 ? kPairLowN : kPairMinN;
     d.pair_max = kPairMaxN;
     for (int n : E->cnt)
         if (pair_size(d, n)) units += g6cp::Plan(n, 1).work();

@@ -153,11 +153,12 @@ int g6c_forces(void *ens, int precision, double acc[][3], double jerk[][3],
                double pot[]);
 /* lanes per i-particle (1..64, a power of two) for each of 8 size classes
  * (<=16, <=32, ..., <=2048, more).  While a class above 128 particles has the
- * shape it starts with (one lane, 256 j), its clusters of 193 to 8192 are taken
- * pair by unordered pair where they are a large enough part of the ensemble's
- * work.  That takes device memory for partial sums, growing as the square of a
- * cluster's particles (2048: 1.5 to 2.9 MB, 8192: 22 to 45) and at most 8 GiB in
- * all: beyond, the largest clusters keep the other kernels. */
+ * shape it starts with (one lane, 256 j), its clusters of 193 to 8192 (beside
+ * more work in such ones, of 129) are taken pair by unordered pair where they
+ * are a large enough part of the ensemble's work.  That takes device memory for
+ * partial sums, growing as the square of a cluster's particles (2048: 1.5 to
+ * 2.9 MB, 8192: 22 to 45) and at most 8 GiB in all: beyond, the largest clusters
+ * keep the other kernels. */
 int g6c_set_tiles(void *ens, const int njs_per_class[8]);
 int g6c_get_tiles(void *ens, int njs_per_class[8]);
 /* j per LDS tile (16..256, a power of two) for each size class */
