@@ -120,13 +120,13 @@ struct PassF64 {
     using T = double;
     using V = double2;
     static constexpr int W = 4;  // LDS words of a column: (x y), (z m), (vx vy), (vz -)
-    // tiles a lane's plain sums run over before they are folded: 64 pairs below
-    // 50000 particles, 256 above, where the many partial sums' roundings average
-    // out (the pair by pair kernels: 128 and 256).  Root mean square error over
-    // theirs, acc / jerk / pot: 0.87 / 0.82 / 0.76 at N = 20000 (256 pairs and
-    // columns' sums of a whole tile: 1.11 / 1.07 / 1.21), 0.90 / 0.83 / 0.87 at 65536.
+    // tiles a lane's plain sums run over before they are folded: 128 pairs below
+    // 50000 particles, 256 above, as the pair by pair kernels.  Root mean square
+    // error over theirs, acc / jerk / pot: 0.91 / 0.90 / 0.90 at N = 20000 (256 pairs
+    // and columns' sums of a whole tile: 1.11 / 1.07 / 1.21), 0.90 / 0.83 / 0.87 at
+    // 65536.  Folds at 64 pairs: 0.87 / 0.82 / 0.76, and N = 45000 2010 -> 2150 us.
     template <int IPL>
-    static constexpr int kFold = IPL == 2 ? 1 : 4;
+    static constexpr int kFold = IPL == 2 ? 2 : 4;
     static constexpr int kSum = 2, kRow = 16;  // values of a row's sum, of its record
     // the columns' sums continue on from lane to lane (plain sums of kSeg IPL
     // terms): a rotation moves 64-bit values and does not fuse with an add
