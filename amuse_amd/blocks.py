@@ -43,7 +43,11 @@ def _bind(lib):
 
 
 class DeviceHermite4:
-    """ph4-style block-step integration with the whole step on the GPU."""
+    """ph4-style block-step integration with the whole step on the GPU.
+
+    steps_per_graph: block steps of one replay of the captured step, at most 8
+    (a larger number is taken as 8: after an interval's end a replay's steps
+    that are left run empty)."""
 
     def __init__(self, precision: int = 0, steps_per_graph: int = 64, device: int = 0,
                  ph4_initial_load: bool = True):

@@ -23,8 +23,10 @@
 // double.  Each workgroup covers 256/NJS i-particles, NJS lanes share one
 // i and split the j-range (NJS from a workgroup target per kernel); j-tiles go
 // through LDS as rows of four values.  Each lane's plain partial sums are
-// folded into compensated (TwoSum) sums every ~64 pairs.  No allocation:
-// the caller passes every buffer and its stream.
+// folded into compensated (TwoSum) sums every ~64 pairs.  With a workspace
+// and enough particles every unordered pair is taken once (g6_sym.h: rows'
+// sums folded every 64 pairs, the columns' every 16 steps of 1, 2 or 4 pairs).  No
+// allocation: the caller passes every buffer and its stream.
 #include "g6_sym.h"
 
 #include <hip/hip_runtime.h>
@@ -524,7 +526,9 @@ struct AdjointOp {
 // 130 / 127, 32768 - / 472 / 435; FP64 forward 4000 28.4 / 36.0, 6500 56.1 /
 // 53.3, 32768 1060 / 900; FP32 adjoint 4000 34.0 / 46.0, 5003 49.4 / 47.0,
 // 16384 298 / 277; FP64 adjoint 4500 57.7 / 68.2, 5003 73.7 / 69.0, 32768 2156
-// / 2050.  4 a lane in FP64 or the adjoint would leave one wave per SIMD.
+// / 2050.  The FP64 adjoint runs one wave a SIMD with 2 (256 VGPRs and some
+// AGPRs): 4 a lane would spill it, and leave the FP64 forward and the FP32
+// adjoint one wave.
 constexpr int kSymNarrow = 4800, kSymWide = 10000;
 template <class T, class Op>
 inline int sym_ipl(int n)
@@ -547,8 +551,9 @@ constexpr int kSymWgs = 4000;
 template <class T, class Op>
 constexpr int kSymMin = Op::NC == 6 ? (sizeof(T) == 4 ? 4300 : 3300)
                                     : (sizeof(T) == 4 ? 3600 : 2300);
-// The largest workspace asked for (from about n = 100,000): beyond, the pair
-// by ordered pair form, which needs none.
+// The largest workspace asked for (FP64 from about n = 100,000, FP32 from 140,000
+// in the adjoint and 210,000 in the forward): beyond, the pair by ordered pair
+// form, which needs none.
 constexpr long long kSymMaxBytes = 2ll << 30;
 
 template <class T, class Op>

@@ -45,7 +45,7 @@ struct Plan {
     // Whether row block b takes the block d places on (1 <= d <= nb / 2).
     __host__ __device__ bool takes(int b, int d) const { return 2 * d < nb || b < nb / 2; }
     // values of the partial records, `nc` sums per particle (the rows' in FP64,
-    // the columns', plain sums over one tile, in the pass's own type)
+    // the columns', one per tile, in the pass's own type)
     long long row_values(int nc) const { return (long long)items() * nc * rows; }
     long long col_values(int nc) const { return (long long)(nb / 2) * nc * n; }
     // row record of workgroup `it`, sum c, row i of the block

@@ -93,7 +93,8 @@ int g6x_sync(void);
  * the i-block's centre (same error bound as the double-single difference).
  * 0: slot order always.  The automatic choice of shapes takes full passes in
  * slot order, every unordered pair once (partial sums in a workspace of the
- * library, at most about 1.6 GB). */
+ * library, at most about 1.6 GB); the shapes of a tuned or loaded table are
+ * taken as they stand, pair by ordered pair. */
 int g6x_set_spatial(int on);
 
 /* Kernel timing with HIP events recorded on the unit's own stream around
