@@ -1182,11 +1182,12 @@ int ensure_spatial(int nj)
 
 // Full passes at least this long evaluate every unordered pair once
 // (g6k::launch_pass).  us of a whole pass, pair by ordered pair against
-// pair-once: FP64 160 / 143 at N = 8192, 461 / 360 at 16384, 1557 / 1207 at 32768,
-// 5700 / 4250 at 65536, 22000 / 15900 at 131072; mixed 105 / 115 at 8192, 198 / 180
-// at 12000, 287 / 268 at 16384, 950 / 803 at 32768, 3310 / 2630 at 65536, 12330 /
-// 9090 at 131072.
-constexpr int kPassMinF64 = 8192, kPassMinMixed = 12000;
+// pair-once: FP64 154 / 145 at N = 8192, 462 / 365 at 16384, 1515 / 1205 at 32768,
+// 5640 / 4170 at 65536, 21500 / 15800 at 131072; mixed 165 / 178 at 12000, 173 /
+// 181 at 12500, 184 / 182 at 13000, 200 / 186 at 13500, 212 / 220 at 14000, 243 / 225
+// at 15000, 274 / 262 at 16384, 945 / 800 at 32768, 3230 / 2450 at 65536, 12530 /
+// 8980 at 131072.
+constexpr int kPassMinF64 = 8192, kPassMinMixed = 13000;
 
 // Whether a full pass over nj slots holding distinct ids takes the pair-once
 // kernels: under the automatic choice of shapes (a shape that was set or

@@ -691,6 +691,32 @@ def test_pair_once_full_pass_edges(g6, prec, n):
         g6.set_precision(0)
 
 
+@pytest.mark.parametrize("n", [13000, 13312, 13313, 13823, 13824])
+def test_pair_once_mixed_smallest(g6, n):
+    """The same at the smallest sizes of mixed passes (below 13000 slots the
+    pair by ordered pair kernels are the faster ones), and the line itself:
+    one slot fewer gives the bits that the other kernels give a block of
+    12999 i-particles over the same slots."""
+    test_pair_once_full_pass_edges(g6, 1, n)
+    if n > 13000:
+        return
+    st = plummer_state(n, n, dt_nonzero=False)
+    k = slice(0, n - 1)
+    g6.set_precision(1)
+    try:
+        g6.reset()
+        upload(g6, st["x"][k], st["v"][k], st["a2"][k], st["j6"][k], st["k18"][k], st["m"][k],
+               st["tj"][k], st["ids"][k])
+        g6.set_ti(st["ti"])
+        rows = []
+        for ni in (n - 1, n - 2):
+            g6.calc_self(n - 1, 0, ni, 1e-4, nn=True)
+            rows.append(g6.fetch(ni)[0])
+        assert np.array_equal(rows[0][:n - 2], rows[1])
+    finally:
+        g6.set_precision(0)
+
+
 @pytest.mark.parametrize("prec", [0, 1])
 @pytest.mark.parametrize("n", [63, 64, 65, 2049, 4097, 12000, 12001])
 def test_set_j_particles_by_columns(g6, n, prec):
